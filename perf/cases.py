@@ -170,8 +170,21 @@ def _inputs(case, seed):
     return xyz, q, pts
 
 
+_STREAM = []
+
+
+def _stream():
+    """The one stream of the program: its tensors and the library's work are
+    on it, so that a buffer torch hands out again is never still written to."""
+    if not _STREAM:
+        _STREAM.append(torch.cuda.Stream())
+    torch.cuda.set_stream(_STREAM[0])
+    return _STREAM[0].cuda_stream
+
+
 def prepare(case, seed):
     import openspacecharge_amd as osc
+    stream = _stream()
     prec = osc.OSC_PREC_FP32 if case["precision"] == "fp32" else osc.OSC_PREC_FP64
     if case["call"] == "stream":
         reqs = _requests(case)
@@ -190,7 +203,7 @@ def prepare(case, seed):
         pts = xyz if not case["points"] else tuple(a.cpu().numpy() for a in pts)
         q = None if q is None else q.cpu().numpy()
     else:
-        ctx.set_stream(torch.cuda.current_stream().cuda_stream)
+        ctx.set_stream(stream)
         ctx.set_async(True)
     mesh = osc.Mesh3D(nhi=(case["nx"], case["ny"], case["nz"]), gamma=GAMMA,
                       device="host" if case["host"] else "cuda")
