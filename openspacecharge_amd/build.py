@@ -30,7 +30,8 @@ HIPCC = os.path.join(ROCM, "bin", "hipcc")
 FLANG = os.path.join(ROCM, "bin", "amdflang")
 ARCH = os.environ.get("OSC_OFFLOAD_ARCH", "gfx950")
 
-HIP_SOURCES = ["context.hip", "fft_f64.hip", "fft_f32.hip", "green.hip", "solve.hip",
+HIP_SOURCES = ["context.hip", "fft_f64.hip", "fft_f32.hip", "fft_gen_f64.hip",
+               "fft_gen_f32.hip", "green.hip", "solve.hip",
                "solvers.hip", "deposit.hip", "gather.hip", "capi.hip", "server.hip",
                "noalloc.hip"]
 

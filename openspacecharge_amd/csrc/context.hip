@@ -359,17 +359,68 @@ bool fft_has_plan(int L) {
   }
 }
 
+// The prime factors of L in ascending order, split into consecutive groups of
+// kRtGroups: the fewest groups, then the smallest largest one (its registers).
 GenericPlan generic_plan(int L) {
-  GenericPlan p;
+  GenericPlan p{};
   p.L = L;
-  p.ns = 0;
-  int n = L;
-  for (int f = 2; f <= 23 && n > 1; ++f)
-    while (n % f == 0 && p.ns < 24) {
-      p.r[p.ns++] = f;
-      n /= f;
+  int f[24], nf = 0, n = L;
+  for (int q = 2; q <= 23 && n > 1; ++q)
+    while (n % q == 0 && nf < 24) {
+      f[nf++] = q;
+      n /= q;
     }
-  if (n != 1) p.ns = -1;
+  if (n != 1) {
+    p.ns = -1;
+    return p;
+  }
+  if (nf == 0) f[nf++] = 1;  // L == 1: one stage that copies
+  p.big = f[nf - 1] > 7;
+  // best[i]: stages and largest radix of the groups covering factors i ..
+  struct Best {
+    int ns, most, group, len;
+  } best[25];
+  best[nf] = {0, 0, 0, 0};
+  for (int i = nf - 1; i >= 0; --i) {
+    best[i] = {100, 0, 0, 0};
+    for (int g = 0; g < (p.big ? kRtNGroups : kRtSmall); ++g) {
+      int len = 0, R = 1;
+      bool ok = true;
+      for (int t = 0; t < 3 && ok; ++t) {
+        const int r = kRtGroups[g][t];
+        if (r == 1 && t > 0) break;
+        ok = i + len < nf && f[i + len] == r;
+        R *= r;
+        ++len;
+      }
+      if (!ok) continue;
+      const Best& t = best[i + len];
+      const Best c{t.ns + 1, std::max(t.most, R), g, len};
+      if (c.ns < best[i].ns || (c.ns == best[i].ns && c.most < best[i].most)) best[i] = c;
+    }
+  }
+  const auto magic = [](int d) {
+    return d == 1 ? 0u : uint32_t(((uint64_t(1) << 32) + d - 1) / d);
+  };
+  if (best[0].ns > int(sizeof(p.s) / sizeof(p.s[0]))) {  // L beyond any that is launched
+    p.ns = -1;
+    return p;
+  }
+  int Ns = 1;
+  for (int i = 0; i < nf; i += best[i].len) {
+    RtStage& s = p.s[p.ns++];
+    const int* r = kRtGroups[best[i].group];
+    s.group = best[i].group;
+    s.R = r[0] * r[1] * r[2];
+    s.Ns = Ns;
+    s.nbf = L / s.R;
+    s.tws[0] = L / (Ns * r[0]);
+    s.tws[1] = L / (Ns * r[0] * r[1]);
+    s.tws[2] = L / (Ns * s.R);
+    s.mNs = magic(Ns);
+    s.mnbf = magic(s.nbf);
+    Ns *= s.R;
+  }
   return p;
 }
 
@@ -377,10 +428,9 @@ bool fft_len_supported(int L) {
   if (L < 1) return false;
   if (L == 1) return true;
   if (fft_has_plan(L)) return true;
-  GenericPlan p = generic_plan(L);
-  if (p.ns < 0) return false;
-  // generic engine keeps 2 lines of L complex doubles in LDS
-  return size_t(LdsPad<double>::size(2 * kGenBX * L)) * sizeof(cpx<double>) <= 65536;
+  // the longest line: two buffers of it in 64 KB of LDS
+  if (size_t(LdsPad<double>::size(2 * L)) * sizeof(cpx<double>) > 65536) return false;
+  return generic_plan(L).ns > 0;
 }
 
 // ---------------------------------------------------------------------------

@@ -4,8 +4,8 @@
 // threads; every thread keeps E = L/TPL complex values in registers and the
 // radix stages exchange data through LDS (one buffer, read-all / barrier /
 // write-all per stage).  Plans (radix sequences) are compile-time for the
-// lengths in FftPlan; any other length uses FftGeneric (runtime radices, LDS
-// double buffer).  Both engines present the same interface:
+// lengths in FftPlan; any other length uses FftRt (its lines in LDS, prime
+// radices grouped at run time).  The compile-time engine's interface:
 //
 //   load(f)   f(b, p) -> value of line b at position p (stage-0 positions)
 //   run(lds, tw)
@@ -332,82 +332,228 @@ struct FftTile {
 };
 
 // ---------------------------------------------------------------------------
-// runtime-radix fallback (any length whose prime factors are <= 23)
+// runtime-length engine (any length whose prime factors are <= 23)
 // ---------------------------------------------------------------------------
+// A stage takes up to three consecutive prime radices of the length (ascending
+// order) in one pass over the registers of a thread: R = r1 r2 r3 values, one
+// LDS exchange, with the twiddles and the sums of each prime stage as a
+// sequence of single-prime stages has them.  The radices are compile-time
+// (rt_stage is instantiated for every group of kRtGroups), so the values stay
+// in registers; only the choice among them is made at run time.
+//
+// The engine before this kept a radix's values in arrays indexed by run-time
+// loops, which the compiler puts in scratch memory, one line per 64-thread
+// workgroup and one stage per prime: bound by scratch traffic.  In registers,
+// with several lines per workgroup and columns read by whole rows, a free FP64
+// step on a 100x75x60 mesh (10^6 particles; lines of 200, 150 and 120) takes
+// 711 us against 2845, one on 24x72x51 in FP32 339 against 737.  The order of
+// operations is the same, bit for bit.
+struct RtStage {
+  int group;      // index into kRtGroups
+  int R, Ns, nbf;  // radix, transforms done before, L / R
+  int tws[3];     // twiddle strides L / (Ns r1), L / (Ns r1 r2), L / (Ns R)
+  uint32_t mNs;   // ceil(2^32 / Ns): division of j < L by Ns (0: Ns == 1)
+  uint32_t mnbf;  // the same for nbf
+};
 struct GenericPlan {
   int L;
-  int ns;
-  int r[24];
+  int ns;  // stages; -1: a prime factor above 23
+  RtStage s[11];
+  // launch geometry, set per pass (rt_geometry): lines per workgroup as a
+  // power of two, threads, and whether the stages alternate between two
+  // buffers (some stage has more butterflies than threads)
+  int bs, nt, pp;
+  int big;  // a prime above 7: groups beyond kRtSmall
 };
+// The first kRtSmall groups serve the lengths without a prime above 7, in
+// kernels of their own: at most ten values a thread (about 100 VGPRs in FP64),
+// where radix 23 with its table of W takes 240 and leaves two waves per SIMD.
+constexpr int kRtGroups[][3] = {
+    {1, 1, 1},  {2, 1, 1},  {3, 1, 1},  {5, 1, 1},  {7, 1, 1},  {2, 2, 1},  {2, 3, 1},
+    {3, 3, 1},  {2, 5, 1},  {2, 2, 2},  {11, 1, 1}, {13, 1, 1}, {17, 1, 1}, {19, 1, 1},
+    {23, 1, 1}, {3, 5, 1},  {2, 7, 1},  {3, 7, 1},  {2, 11, 1}, {2, 13, 1}, {2, 2, 3},
+    {2, 3, 3},  {2, 2, 5},
+};
+constexpr int kRtNGroups = sizeof(kRtGroups) / sizeof(kRtGroups[0]);
+constexpr int kRtSmall = 10;
+constexpr int kRtMaxThreads = 512;
 
-// One line per group of GTPL threads; LDS holds two buffers of L per line.
-template <typename T, int DIR, int BX, int GTPL>
-struct FftGeneric {
-  static constexpr int NT = BX * GTPL;
-  int b, t;
-  int L;
-  __device__ __forceinline__ FftGeneric(int L_) : L(L_) {
-    b = threadIdx.x / GTPL;
-    t = threadIdx.x % GTPL;
+__device__ __forceinline__ int rt_div(int n, uint32_t m) {
+  return m ? int(__umulhi(uint32_t(n), m)) : n;
+}
+
+// Complex products with their contraction written out, so that a length's FP32
+// result does not change with the code around them: the real part is
+// fma(a.x, b.x, -(a.y b.y)); the imaginary part fuses a.y b.x (FUSEY) or a.x b.y.
+template <bool FUSEY, typename T>
+__device__ __forceinline__ cpx<T> mul_fused(cpx<T> a, cpx<T> b) {
+  const T p = a.y * b.y, q = FUSEY ? a.x * b.y : a.y * b.x;
+  if constexpr (sizeof(T) == 4)
+    return mk(__builtin_fmaf(a.x, b.x, -p),
+              FUSEY ? __builtin_fmaf(a.y, b.x, q) : __builtin_fmaf(a.x, b.y, q));
+  else
+    return mk(__builtin_fma(a.x, b.x, -p),
+              FUSEY ? __builtin_fma(a.y, b.x, q) : __builtin_fma(a.x, b.y, q));
+}
+
+// out(q, sum_r a[r] W_R^{rq}) for q < R, W_R^m = w[m], added in the order of r
+template <int R, int DIR, typename T, class F>
+__device__ __forceinline__ void dft_direct(const cpx<T> (&a)[R], const cpx<T> (&w)[R], F&& out) {
+#pragma unroll
+  for (int q = 0; q < R; ++q) {
+    cpx<T> acc = a[0];
+#pragma unroll
+    for (int r = 1; r < R; ++r) acc = add(acc, mul_fused<(DIR > 0)>(a[r], w[(r * q) % R]));
+    out(q, acc);
   }
-  __device__ __forceinline__ bool active() const { return b < BX; }
-  __device__ __forceinline__ int lidx(int bb, int p, int buf) const {
-    return LdsPad<T>::idx((buf * BX + bb) * L + p);
+}
+
+// BX = 1 << bs lines of L values in LDS, line b's value p at lidx(b, p): PFAST
+// (x axis) line after line, else the lines' values p side by side, as the
+// strided axes read and write them.
+template <typename T, int DIR, bool PFAST, bool BIG>
+struct FftRt {
+  const GenericPlan& pl;
+  cpx<T>* lds;
+  const cpx<T>* tw;
+  int cur = 0;  // the buffer holding the lines (with pp)
+  __device__ __forceinline__ FftRt(const GenericPlan& p, cpx<T>* l, const cpx<T>* t)
+      : pl(p), lds(l), tw(t) {}
+  __device__ __forceinline__ int at(int b, int p, int buf) const {
+    const int i = PFAST ? b * pl.L + p : (p << pl.bs) + b;
+    return LdsPad<T>::idx(i) + buf * LdsPad<T>::size(pl.L << pl.bs);
   }
-  static __host__ __device__ int lds_size(int L) { return LdsPad<T>::size(2 * BX * L); }
-
-  cpx<T>* lds_ = nullptr;
-  int cur = 0;
-
+  __device__ __forceinline__ cpx<T> get(int b, int p) const { return lds[at(b, p, cur)]; }
+  // f(b, p) for every value of every line, by the threads in memory order
   template <class F>
-  __device__ __forceinline__ void load(cpx<T>* lds, F&& f) {
-    lds_ = lds;
-    cur = 0;
-    for (int p = t; p < L; p += GTPL) lds[lidx(b, p, 0)] = f(b, p);
-  }
-  __device__ void run(const GenericPlan& pl, const cpx<T>* __restrict__ tw) {
-    __syncthreads();
-    int Ns = 1;
-    for (int s = 0; s < pl.ns; ++s) {
-      const int R = pl.r[s];
-      const int nbf = L / R;
-      const int tws = L / (Ns * R);
-      for (int j = t; j < nbf; j += GTPL) {
-        cpx<T> a[23], y[23];
-        const int k = j % Ns;
-        for (int r = 0; r < R; ++r) {
-          cpx<T> vv = lds_[lidx(b, j + r * nbf, cur)];
-          if (r > 0 && k > 0) {
-            cpx<T> w = tw[k * r * tws];
-            if (DIR > 0) w.y = -w.y;
-            vv = mul(vv, w);
-          }
-          a[r] = vv;
-        }
-        // direct DFT of size R: y[q] = sum_r a[r] W_R^{rq}, W_R^m = tw[m * L/R]
-        for (int q = 0; q < R; ++q) {
-          cpx<T> acc = a[0];
-          for (int r = 1; r < R; ++r) {
-            cpx<T> w = tw[((r * q) % R) * nbf];
-            if (DIR > 0) w.y = -w.y;
-            acc = add(acc, mul(a[r], w));
-          }
-          y[q] = acc;
-        }
-        const int od = (j / Ns) * Ns * R + k;
-        for (int r = 0; r < R; ++r) lds_[lidx(b, od + r * Ns, cur ^ 1)] = y[r];
-      }
-      cur ^= 1;
-      Ns *= R;
-      __syncthreads();
+  __device__ __forceinline__ void each(int n, F&& f) const {
+    if constexpr (PFAST) {
+      // 64 threads a line
+      for (int b = threadIdx.x >> 6; b < (1 << pl.bs); b += pl.nt >> 6)
+        for (int p = threadIdx.x & 63; p < n; p += 64) f(b, p);
+    } else {
+      for (int i = threadIdx.x; i < (n << pl.bs); i += pl.nt) f(i & ((1 << pl.bs) - 1), i >> pl.bs);
     }
   }
   template <class F>
-  __device__ __forceinline__ void store(F&& f) const {
-    for (int p = t; p < L; p += GTPL) f(b, p, lds_[lidx(b, p, cur)]);
+  __device__ __forceinline__ void load(F&& f) {
+    cur = 0;
+    each(pl.L, [&](int b, int p) { lds[at(b, p, 0)] = f(b, p); });
+    __syncthreads();
   }
-  // natural-order result already in LDS buffer `cur`
-  __device__ __forceinline__ int result_buf() const { return cur; }
+  __device__ __forceinline__ cpx<T> twd(unsigned i) const {
+    cpx<T> w = tw[i];
+    if (DIR > 0) w.y = -w.y;
+    return w;
+  }
+  template <int R1, int R2, int R3>
+  __device__ __forceinline__ void stage(const RtStage& st) {
+    constexpr int R = R1 * R2 * R3, R23 = R2 * R3;
+    const int Ns = st.Ns, nbf = st.nbf, items = nbf << pl.bs, dst = pl.pp ? cur ^ 1 : cur;
+    const int rounds = pl.pp ? (items + pl.nt - 1) / pl.nt : 1;
+    for (int it = 0; it < rounds; ++it) {
+      const int i = threadIdx.x + it * pl.nt;
+      const bool act = i < items;
+      int b, j;
+      if constexpr (PFAST) {
+        b = rt_div(i, st.mnbf);
+        j = i - b * nbf;
+      } else {
+        b = i & ((1 << pl.bs) - 1);
+        j = i >> pl.bs;
+      }
+      cpx<T> v[R];
+#pragma unroll
+      for (int m = 0; m < R; ++m) v[m] = act ? lds[at(b, j + m * nbf, cur)] : mk<T>(0, 0);
+      if (!pl.pp) __syncthreads();  // in place: every read before the first write
+      if (!act) continue;
+      const int kq = rt_div(j, st.mNs), k = j - kq * Ns, od = kq * Ns * R + k;
+      // output (q, q2, q3) of the three prime stages
+      auto put = [&](int q, int q2, int q3, cpx<T> y) {
+        lds[at(b, od + (q + R1 * (q2 + R2 * q3)) * Ns, dst)] = y;
+      };
+      {
+        cpx<T> w[R1], t[R1];
+#pragma unroll
+        for (int r = 0; r < R1; ++r) {
+          w[r] = twd(unsigned(r * (pl.L / R1)));
+          t[r] = twd(unsigned(k * r * st.tws[0]));
+        }
+#pragma unroll
+        for (int g = 0; g < R23; ++g) {
+          cpx<T> a[R1];
+          a[0] = v[g];
+#pragma unroll
+          for (int r = 1; r < R1; ++r) a[r] = mul_fused<true>(v[g + r * R23], t[r]);
+          dft_direct<R1, DIR, T>(a, w, [&](int q, cpx<T> y) {
+            if constexpr (R23 > 1) v[g + q * R23] = y;
+            else put(q, 0, 0, y);
+          });
+        }
+      }
+      if constexpr (R2 > 1) {
+        cpx<T> w[R2];
+#pragma unroll
+        for (int r = 0; r < R2; ++r) w[r] = twd(unsigned(r * (pl.L / R2)));
+#pragma unroll
+        for (int q = 0; q < R1; ++q) {
+          cpx<T> t[R2];
+#pragma unroll
+          for (int r = 1; r < R2; ++r) t[r] = twd(unsigned((k + q * Ns) * r * st.tws[1]));
+#pragma unroll
+          for (int g = 0; g < R3; ++g) {
+            cpx<T> a[R2];
+            a[0] = v[g + q * R23];
+#pragma unroll
+            for (int r = 1; r < R2; ++r) a[r] = mul_fused<true>(v[g + r * R3 + q * R23], t[r]);
+            dft_direct<R2, DIR, T>(a, w, [&](int q2, cpx<T> y) {
+              if constexpr (R3 > 1) v[g + q2 * R3 + q * R23] = y;
+              else put(q, q2, 0, y);
+            });
+          }
+        }
+      }
+      if constexpr (R3 > 1) {
+        cpx<T> w[R3];
+#pragma unroll
+        for (int r = 0; r < R3; ++r) w[r] = twd(unsigned(r * (pl.L / R3)));
+#pragma unroll
+        for (int q = 0; q < R1; ++q)
+#pragma unroll
+          for (int q2 = 0; q2 < R2; ++q2) {
+            cpx<T> a[R3];
+            a[0] = v[q2 * R3 + q * R23];
+#pragma unroll
+            for (int r = 1; r < R3; ++r)
+              a[r] = mul_fused<true>(v[r + q2 * R3 + q * R23],
+                                     twd(unsigned((k + q * Ns + q2 * Ns * R1) * r * st.tws[2])));
+            dft_direct<R3, DIR, T>(a, w, [&](int q3, cpx<T> y) { put(q, q2, q3, y); });
+          }
+      }
+    }
+    cur = dst;
+  }
+  __device__ __forceinline__ void run() {
+    for (int s = 0; s < pl.ns; ++s) {
+      const RtStage& st = pl.s[s];
+      switch (st.group) {
+#define OSC_RT(G, A, B, C)                                  \
+  case G:                                                   \
+    if constexpr (BIG || G < kRtSmall) stage<A, B, C>(st);  \
+    break;
+        OSC_RT(1, 2, 1, 1) OSC_RT(2, 3, 1, 1) OSC_RT(3, 5, 1, 1) OSC_RT(4, 7, 1, 1)
+        OSC_RT(5, 2, 2, 1) OSC_RT(6, 2, 3, 1) OSC_RT(7, 3, 3, 1) OSC_RT(8, 2, 5, 1)
+        OSC_RT(9, 2, 2, 2) OSC_RT(10, 11, 1, 1) OSC_RT(11, 13, 1, 1) OSC_RT(12, 17, 1, 1)
+        OSC_RT(13, 19, 1, 1) OSC_RT(14, 23, 1, 1) OSC_RT(15, 3, 5, 1) OSC_RT(16, 2, 7, 1)
+        OSC_RT(17, 3, 7, 1) OSC_RT(18, 2, 11, 1) OSC_RT(19, 2, 13, 1) OSC_RT(20, 2, 2, 3)
+        OSC_RT(21, 2, 3, 3) OSC_RT(22, 2, 2, 5)
+#undef OSC_RT
+        default:
+          break;
+      }
+      __syncthreads();
+    }
+  }
 };
 
 }  // namespace osc

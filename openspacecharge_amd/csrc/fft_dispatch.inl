@@ -12,8 +12,6 @@ inline dim3 grid3(int64_t x, int64_t y, int64_t z) {
 }
 inline int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
-size_t gen_lds_bytes(int L) { return size_t(LdsPad<T>::size(2 * kGenBX * L)) * sizeof(cpx<T>); }
-
 template <int L, int V>
 void axis_tv(int dir, const cpx<T>* in, cpx<T>* out, const AxisIO& a, int g1, int g2,
              const cpx<T>* tw, hipStream_t s) {
@@ -105,16 +103,8 @@ void launch_axis<T>(int L, int dir, const cpx<T>* in, cpx<T>* out, const AxisIO&
     break;
     OSC_FOR_EACH_L(OSC_CASE)
 #undef OSC_CASE
-    default: {
-      GenericPlan pl = generic_plan(L);
-      dim3 g = grid3(cdiv(a.nb, kGenBX), g1, g2);
-      if (dir < 0)
-        launch((k_axis_gen<T, -1>), g, dim3(kGenBX * kGenTPL), gen_lds_bytes(L), s, in,
-                           out, a, tw, pl);
-      else
-        launch((k_axis_gen<T, 1>), g, dim3(kGenBX * kGenTPL), gen_lds_bytes(L), s, in,
-                           out, a, tw, pl);
-    }
+    default:
+      gen_axis<T>(L, dir, in, out, a, g1, g2, tw, s);
   }
   OSC_HIP(hipGetLastError());
 }
@@ -130,12 +120,8 @@ void launch_xr2c<T>(int L, const double* in, cpx<T>* out, const R2CIO& a, const 
     break;
     OSC_FOR_EACH_L(OSC_CASE)
 #undef OSC_CASE
-    default: {
-      GenericPlan pl = generic_plan(L);
-      dim3 g = grid3(cdiv(cdiv(a.nrows, 2), kGenBX), 1, 1);
-      launch((k_xr2c_gen<T>), g, dim3(kGenBX * kGenTPL), gen_lds_bytes(L), s, in, out,
-                         a, tw, pl);
-    }
+    default:
+      gen_xr2c<T>(L, in, out, a, nullptr, tw, s);
   }
   OSC_HIP(hipGetLastError());
 }
@@ -152,7 +138,8 @@ void launch_xr2c_diff<T>(int L, const double* F, cpx<T>* out, const R2CIO& a,
     OSC_FOR_EACH_L(OSC_CASE)
 #undef OSC_CASE
     default:
-      OSC_REQUIRE(false, OSC_ERR_FFT_LENGTH, "corner-difference x pass needs a planned length");
+      OSC_REQUIRE(!cd.far, OSC_ERR_FFT_LENGTH, "far-field cells need a planned length");
+      gen_xr2c<T>(L, F, out, a, &cd, tw, s);
   }
   OSC_HIP(hipGetLastError());
 }
@@ -168,12 +155,8 @@ void launch_xc2r<T>(int L, const cpx<T>* in, const C2RIO<T>& a, int nout, const 
     break;
     OSC_FOR_EACH_L(OSC_CASE)
 #undef OSC_CASE
-    default: {
-      GenericPlan pl = generic_plan(L);
-      dim3 g = grid3(cdiv(cdiv(a.nrows, 2), kGenBX), nout, 1);
-      launch((k_xc2r_gen<T>), g, dim3(kGenBX * kGenTPL), gen_lds_bytes(L), s, in, a,
-                         tw, pl);
-    }
+    default:
+      gen_xc2r<T>(L, in, a, nout, tw, s);
   }
   OSC_HIP(hipGetLastError());
 }
@@ -201,14 +184,10 @@ void launch_zinv<T>(int L, const cpx<T>* rho, cpx<T>* out, const ZinvIO<T>& a, i
     break;
     OSC_FOR_EACH_L(OSC_CASE)
 #undef OSC_CASE
-    default: {
+    default:
       OSC_REQUIRE(!a.zreal && a.zin == 0, OSC_ERR_FFT_LENGTH,
                   "z-real Green arrays need a planned length");
-      GenericPlan pl = generic_plan(L);
-      dim3 g = grid3(cdiv(a.nb, kGenBX), Ly, nout);
-      launch((k_zinv_gen<T>), g, dim3(kGenBX * kGenTPL), gen_lds_bytes(L), s, rho, out,
-                         a, tw, pl);
-    }
+      gen_zinv<T>(L, rho, out, a, Ly, nout, tw, s);
   }
   OSC_HIP(hipGetLastError());
 }

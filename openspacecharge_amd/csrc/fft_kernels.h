@@ -149,10 +149,6 @@ struct XGeo {
   static constexpr int NT = BX * Geo<T, L>::TPL;
 };
 
-// generic engine geometry: one line per 64-thread workgroup
-constexpr int kGenTPL = 64;
-constexpr int kGenBX = 1;
-
 template <typename T>
 __device__ __forceinline__ cpx<T> ldc(const cpx<T>* p) {
   return *p;
@@ -181,25 +177,6 @@ __global__ void __launch_bounds__((BX * Geo<T, L>::TPL))
     f.load([&](int, int p) { return (ok && p < a.n_in) ? ib[p * a.s_p] : mk<T>(0, 0); });
   f.run(lds, tw);
   cpx<T>* ob = out + (ok ? bg * a.d_b + by * a.d_o1 + bz * a.d_o2 : 0);
-  f.store([&](int, int p, cpx<T> v) {
-    const int q = p - a.w0;
-    if (ok && q >= 0 && q < a.n_out) ob[q * a.d_p] = v;
-  });
-}
-
-template <typename T, int DIR>
-__global__ void __launch_bounds__(kGenBX* kGenTPL)
-    k_axis_gen(const cpx<T>* __restrict__ in, cpx<T>* out, AxisIO a, const cpx<T>* __restrict__ tw,
-               GenericPlan pl) {
-  extern __shared__ unsigned char smem_raw[];
-  cpx<T>* lds = reinterpret_cast<cpx<T>*>(smem_raw);
-  FftGeneric<T, DIR, kGenBX, kGenTPL> f(pl.L);
-  const int bg = blockIdx.x * kGenBX + f.b;
-  const bool ok = bg < a.nb;
-  const cpx<T>* ib = in + (ok ? bg * a.s_b + blockIdx.y * a.s_o1 + blockIdx.z * a.s_o2 : 0);
-  f.load(lds, [&](int, int p) { return ok ? axis_in(ib, a, pl.L, p) : mk<T>(0, 0); });
-  f.run(pl, tw);
-  cpx<T>* ob = out + (ok ? bg * a.d_b + blockIdx.y * a.d_o1 + blockIdx.z * a.d_o2 : 0);
   f.store([&](int, int p, cpx<T> v) {
     const int q = p - a.w0;
     if (ok && q >= 0 && q < a.n_out) ob[q * a.d_p] = v;
@@ -404,37 +381,6 @@ __global__ void __launch_bounds__((XGeo<T, L>::NT))
   }
 }
 
-template <typename T>
-__global__ void __launch_bounds__(kGenBX* kGenTPL)
-    k_xr2c_gen(const double* __restrict__ in, cpx<T>* __restrict__ out, R2CIO a,
-               const cpx<T>* __restrict__ tw, GenericPlan pl) {
-  extern __shared__ unsigned char smem_raw[];
-  cpx<T>* lds = reinterpret_cast<cpx<T>*>(smem_raw);
-  using F = FftGeneric<T, -1, kGenBX, kGenTPL>;
-  F f(pl.L);
-  const int L = pl.L;
-  const int64_t ra = 2 * (int64_t(blockIdx.x) * kGenBX + f.b), rb = ra + 1;
-  const bool oka = ra < a.nrows, okb = rb < a.nrows;
-  const RowPair rp = row_pair(ra, a.ny_rows);
-  const double* pa = in + (oka ? int64_t(rp.ya) * a.in_sy + int64_t(rp.za) * a.in_sz : 0);
-  const double* pb = in + (okb ? int64_t(rp.yb) * a.in_sy + int64_t(rp.zb) * a.in_sz : 0);
-  f.load(lds, [&](int, int p) {
-    T re = (oka && p < a.n_in) ? T(pa[p]) : T(0);
-    T im = (okb && p < a.n_in) ? T(pb[p]) : T(0);
-    return mk(re, im);
-  });
-  f.run(pl, tw);
-  const int buf = f.result_buf();
-  cpx<T>* oa = out + (oka ? int64_t(rp.ya) * a.out_sy + int64_t(rp.za) * a.out_sz : 0);
-  cpx<T>* ob = out + (okb ? int64_t(rp.yb) * a.out_sy + int64_t(rp.zb) * a.out_sz : 0);
-  for (int k = f.t; k <= L / 2; k += kGenTPL) {
-    cpx<T> A, B;
-    r2c_unpack(lds[f.lidx(f.b, k, buf)], lds[f.lidx(f.b, (L - k) % L, buf)], A, B);
-    if (oka) oa[k] = A;
-    if (okb) ob[k] = B;
-  }
-}
-
 // ---------------------------------------------------------------------------
 // inverse x pass: pairs of half spectra -> real rows, with FP64 epilogue
 // ---------------------------------------------------------------------------
@@ -480,34 +426,6 @@ __global__ void __launch_bounds__((XGeo<T, L>::NT))
   const cpx<T>* pb = base + (okb ? int64_t(rp.yb) * a.in_sy + int64_t(rp.zb) * a.in_sz : 0);
   f.load([&](int, int p) { return oka ? c2r_pack(pa, pb, okb, p, L) : mk<T>(0, 0); });
   f.run(lds, tw);
-  const Epilogue e = a.ep[o];
-  const int64_t offa = int64_t(rp.ya) * a.out_sy + int64_t(rp.za) * a.out_sz;
-  const int64_t offb = int64_t(rp.yb) * a.out_sy + int64_t(rp.zb) * a.out_sz;
-  f.store([&](int, int p, cpx<T> v) {
-    const int x = p - a.w0;
-    if (x < 0 || x >= a.n_out) return;
-    if (oka) epi_store(e, offa + x, double(v.x));
-    if (okb) epi_store(e, offb + x, double(v.y));
-  });
-}
-
-template <typename T>
-__global__ void __launch_bounds__(kGenBX* kGenTPL)
-    k_xc2r_gen(const cpx<T>* __restrict__ in, C2RIO<T> a, const cpx<T>* __restrict__ tw,
-               GenericPlan pl) {
-  extern __shared__ unsigned char smem_raw[];
-  cpx<T>* lds = reinterpret_cast<cpx<T>*>(smem_raw);
-  FftGeneric<T, 1, kGenBX, kGenTPL> f(pl.L);
-  const int L = pl.L;
-  const int o = blockIdx.y;
-  const int64_t ra = 2 * (int64_t(blockIdx.x) * kGenBX + f.b), rb = ra + 1;
-  const bool oka = ra < a.nrows, okb = rb < a.nrows;
-  const RowPair rp = row_pair(ra, a.ny_rows);
-  const cpx<T>* base = in + o * a.in_so;
-  const cpx<T>* pa = base + (oka ? int64_t(rp.ya) * a.in_sy + int64_t(rp.za) * a.in_sz : 0);
-  const cpx<T>* pb = base + (okb ? int64_t(rp.yb) * a.in_sy + int64_t(rp.zb) * a.in_sz : 0);
-  f.load(lds, [&](int, int p) { return oka ? c2r_pack(pa, pb, okb, p, L) : mk<T>(0, 0); });
-  f.run(pl, tw);
   const Epilogue e = a.ep[o];
   const int64_t offa = int64_t(rp.ya) * a.out_sy + int64_t(rp.za) * a.out_sz;
   const int64_t offb = int64_t(rp.yb) * a.out_sy + int64_t(rp.zb) * a.out_sz;
@@ -778,25 +696,6 @@ __global__ void __launch_bounds__((ZGeo<T, L>::NT))
         *reinterpret_cast<cpx<T>*>(ob + (c - a.w0) * a.o_sz * CB + vout) = v;
     });
   }
-}
-
-template <typename T>
-__global__ void __launch_bounds__(kGenBX* kGenTPL)
-    k_zinv_gen(const cpx<T>* __restrict__ rho, cpx<T>* __restrict__ out, ZinvIO<T> a,
-               const cpx<T>* __restrict__ tw, GenericPlan pl) {
-  extern __shared__ unsigned char smem_raw[];
-  cpx<T>* lds = reinterpret_cast<cpx<T>*>(smem_raw);
-  FftGeneric<T, 1, kGenBX, kGenTPL> f(pl.L);
-  const int kx = blockIdx.x * kGenBX + f.b, ky = blockIdx.y, o = blockIdx.z;
-  const bool ok = kx < a.nb;
-  const OutTerms<T>& ot = a.out[o];
-  f.load(lds, [&](int, int p) { return ok ? combine(rho, a, ot, kx, ky, p) : mk<T>(0, 0); });
-  f.run(pl, tw);
-  cpx<T>* ob = out + o * a.o_so + kx + ky * a.o_sy;
-  f.store([&](int, int p, cpx<T> v) {
-    const int q = p - a.w0;
-    if (ok && q >= 0 && q < a.n_out) ob[q * a.o_sz] = v;
-  });
 }
 
 }  // namespace osc

@@ -60,4 +60,18 @@ template <typename T>
 void launch_zinv(int L, const cpx<T>* rho, cpx<T>* out, const ZinvIO<T>& a, int Ly, int nout,
                  const cpx<T>* tw, hipStream_t s);
 
+// the same passes over lengths without a compile-time plan (fft_gen.inl)
+template <typename T>
+void gen_axis(int L, int dir, const cpx<T>* in, cpx<T>* out, const AxisIO& a, int g1, int g2,
+              const cpx<T>* tw, hipStream_t s);
+template <typename T>
+void gen_xr2c(int L, const double* in, cpx<T>* out, const R2CIO& a, const CornerDiff* cd,
+              const cpx<T>* tw, hipStream_t s);
+template <typename T>
+void gen_xc2r(int L, const cpx<T>* in, const C2RIO<T>& a, int nout, const cpx<T>* tw,
+              hipStream_t s);
+template <typename T>
+void gen_zinv(int L, const cpx<T>* rho, cpx<T>* out, const ZinvIO<T>& a, int Ly, int nout,
+              const cpx<T>* tw, hipStream_t s);
+
 }  // namespace osc

@@ -601,7 +601,16 @@ GreenRef green_spectrum(osc_ctx* c, const GreenSpec& s, DevBuf& keepalive) {
   GreenRef ref{};
   GreenRef* zr = fft_has_plan(s.L[2]) ? &ref : nullptr;
   const bool fast = sizeof(T) == 4;  // mirrored quarter-grid primitive (prim_mirrors)
-  if (s.kind == GK_OFFSET && fft_has_plan(s.L[0])) {
+  if (s.kind == GK_OFFSET && !fft_has_plan(s.L[0])) {
+    // the x pass of a length without a plan differences the primitive on the
+    // whole grid, without far-field cells and mirrored halves
+    {
+      ProfScope ps(c, ST_GREEN_EVAL);
+      build_offset_primitive(c, s, g.as<double>(), fast);
+    }
+    const CornerDiff cd{s.L[1], s.L[2], s.out_shift_z, s.zero_raw};
+    spectrum_forward_full<T>(c, g.as<const double>(), sp.as<cpx<T>>(), d, &cd, nullptr, zr);
+  } else if (s.kind == GK_OFFSET) {
     // the x pass takes the 8-corner difference of the primitive as it loads
     // its rows, so the difference array is never stored
     CornerDiff cd{s.L[1], s.L[2], s.out_shift_z, s.zero_raw};
