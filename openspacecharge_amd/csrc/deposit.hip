@@ -965,11 +965,9 @@ __global__ void k_node(const A* __restrict__ S, const uint8_t* __restrict__ occ,
 // not fix it) cannot change rho, which is bit-identical run to run: it is the
 // sum of the terms, each rounded to 2^-82 n max|q|, converted once.  FP32
 // deposition keeps the integer part only (terms rounded to 2^-50 n max|q|).
-constexpr int TS_T = 512, TS_P = 8192;  // threads and particles per count / scatter block
-constexpr int TS_R = 1024;              // particles per scatter round (staged in LDS)
+constexpr int TS_T = 512, TS_P = 8192;  // threads and most particles per count / scatter block
 constexpr int TA_T = 512;               // threads per accumulate workgroup
 constexpr int kTileAccWords = 5632;     // node accumulators of one workgroup (44 KB)
-static_assert(TS_P % TS_R == 0 && TS_R % TS_T == 0, "whole rounds of whole thread steps");
 static_assert(kTileMaxBins % TS_T == 0 && kTileMaxBins <= 2 * 1024, "bins per thread");
 
 __device__ __forceinline__ void tile_mesh(TileParams& p) {
@@ -1034,8 +1032,9 @@ __device__ __forceinline__ uint32_t block_excl_scan(uint32_t v, uint32_t* s) {
 __global__ void __launch_bounds__(TS_T)
     k_tile_count(const double* __restrict__ x, const double* __restrict__ y,
                  const double* __restrict__ z, const double* __restrict__ q, int64_t n,
-                 TileParams p, uint32_t* __restrict__ hist, int nb, uint32_t* __restrict__ ndrop,
-                 TilePlan* __restrict__ tp, uint64_t* __restrict__ hpart) {
+                 TileParams p, int tsp, uint32_t* __restrict__ hist, int nb,
+                 uint32_t* __restrict__ ndrop, TilePlan* __restrict__ tp,
+                 uint64_t* __restrict__ hpart) {
   __shared__ uint32_t h[kTileMaxBins];
   __shared__ double wmax[TS_T / 64];
   tile_mesh(p);
@@ -1043,8 +1042,8 @@ __global__ void __launch_bounds__(TS_T)
   __syncthreads();
   double qm = 0.0;
   uint64_t hs = 0;
-  const int64_t base = int64_t(blockIdx.x) * TS_P;
-  for (int it = 0; it < TS_P / TS_T; ++it) {
+  const int64_t base = int64_t(blockIdx.x) * tsp;
+  for (int it = 0; it < tsp / TS_T; ++it) {
     const int64_t i0w = base + int64_t(it) * TS_T;
     if (i0w >= n) break;  // uniform per block
     const int64_t i = i0w + threadIdx.x;
@@ -1080,7 +1079,7 @@ __global__ void __launch_bounds__(TS_T)
 // step 2b: one workgroup of 1024 threads, thread t owning bins 2t and 2t+1
 __global__ void __launch_bounds__(1024)
     k_tile_plan(const uint32_t* __restrict__ total, int ntiles, int64_t n, double q_each,
-                int hasq, int chunk, TilePlan* __restrict__ tp) {
+                int hasq, int chunk, int gchunk, TilePlan* __restrict__ tp) {
   __shared__ uint32_t s[3][16];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   // per bin: particles, deposit chunks, gather chunks; exclusive scans of the
@@ -1091,7 +1090,7 @@ __global__ void __launch_bounds__(1024)
     const uint32_t cnt = d <= ntiles ? total[d] : 0u;
     c[k][0] = cnt;
     c[k][1] = d < ntiles ? (cnt + uint32_t(chunk) - 1u) / uint32_t(chunk) : 0u;
-    c[k][2] = d < ntiles ? (cnt + uint32_t(kTileGatherChunk) - 1u) / uint32_t(kTileGatherChunk) : 0u;
+    c[k][2] = d < ntiles ? (cnt + uint32_t(gchunk) - 1u) / uint32_t(gchunk) : 0u;
   }
   uint32_t pre[3];
   for (int q = 0; q < 3; ++q) {
@@ -1133,17 +1132,17 @@ __global__ void __launch_bounds__(1024)
   }
 }
 
-// step 3: records and particle indices in bin order.  FP64: (x, y, z, q);
-// F32: the 16-byte (ab, de, gh, q) of the FP32 deposit and the linear cell
-// key (the sentinel nn0 nn1 nn2 off the mesh) in sk.  The block's TS_P
-// particles go in rounds of R: ranked within the round per bin, placed in
-// LDS in bin order and stored so that consecutive threads write consecutive
-// slots of a bin.  Rounds are as large as two workgroups per CU allow (2048
-// particles, 1024 with charges in FP64; with about a thousand bins shorter
-// rounds leave most bins' runs at one or two records, partial lines), the
-// particle's bin packed with its index in the block.  gofs[d] is the next
-// global slot of bin d for this block (the block's share of the bin starts
-// at bstart[d] + col[d nb + b]).
+// step 3: records in bin order, and the slot of every particle in pos (for the
+// gather's return to particle order).  FP64: (x, y, z, q); F32: the 16-byte
+// (ab, de, gh, q) of the FP32 deposit and the linear cell key (the sentinel
+// nn0 nn1 nn2 off the mesh) in sk.  The block's tsp particles go in rounds of
+// R: ranked within the round per bin, placed in LDS in bin order and stored so
+// that consecutive threads write consecutive slots of a bin.  Rounds are as
+// large as two workgroups per CU allow (2048 particles, 1024 with charges in
+// FP64; with about a thousand bins shorter rounds leave most bins' runs at one
+// or two records, partial lines).  gofs[d] is the next global slot of bin d
+// for this block (the block's share of the bin starts at bstart[d] +
+// col[d nb + b]).
 template <int T>
 __device__ __forceinline__ uint32_t block_excl_scan_t(uint32_t v, uint32_t* s) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -1165,21 +1164,22 @@ struct ScatterGeo {
   static constexpr int R = (!F32 && HASQ) ? 1024 : 2048;  // particles per round
   static constexpr int W = F32 ? 2 : (HASQ ? 4 : 3);      // staged doubles per record
 };
-static_assert(TS_P <= (1 << 13) && kTileMaxBins <= (1 << 19), "bin and index share 32 bits");
+static_assert(kTileMaxBins <= 65536, "a bin in 16 bits");
 template <bool F32, bool HASQ>
 __global__ void __launch_bounds__(TS3_T)
     k_tile_scatter(const double* __restrict__ x, const double* __restrict__ y,
                    const double* __restrict__ z, const double* __restrict__ q, int64_t n,
-                   TileParams p, const uint32_t* __restrict__ col, int nb,
+                   TileParams p, int tsp, const uint32_t* __restrict__ col, int nb,
                    const TilePlan* __restrict__ tp, double4* __restrict__ srec,
-                   uint32_t* __restrict__ sv, uint32_t* __restrict__ sk) {
+                   uint32_t* __restrict__ pos, uint32_t* __restrict__ sk) {
   constexpr int T = TS3_T, R = ScatterGeo<F32, HASQ>::R, W = ScatterGeo<F32, HASQ>::W;
   constexpr int PER = R / T, BPT = kTileMaxBins / T;
   static_assert(TS_P % R == 0 && R % T == 0 && kTileMaxBins % T == 0, "whole rounds and bins");
   __shared__ uint32_t gofs[kTileMaxBins], rc[kTileMaxBins];
   __shared__ uint16_t rs[kTileMaxBins];
   __shared__ double stage[R * W];
-  __shared__ uint32_t sbi[R], skey[F32 ? R : 1];  // bin << 13 | index in the block
+  __shared__ uint16_t sbin[R];
+  __shared__ uint32_t skey[F32 ? R : 1];
   __shared__ uint32_t sc[T / 64];
   tile_mesh(p);
   for (int d = threadIdx.x; d < kTileMaxBins; d += T) {
@@ -1188,18 +1188,16 @@ __global__ void __launch_bounds__(TS3_T)
   }
   __syncthreads();
   const uint32_t sentinel = uint32_t(p.nn[0]) * uint32_t(p.nn[1]) * uint32_t(p.nn[2]);
-  const int64_t base = int64_t(blockIdx.x) * TS_P;
-  for (int r = 0; r < TS_P / R; ++r) {
-    const int64_t rbase = base + int64_t(r) * R;
-    if (rbase >= n) break;  // uniform per block
-    const int nround = n - rbase < R ? int(n - rbase) : R;
+  const int64_t base = int64_t(blockIdx.x) * tsp, bend = base + tsp < n ? base + tsp : n;
+  for (int64_t rbase = base; rbase < bend; rbase += R) {  // uniform per block
+    const int nround = bend - rbase < R ? int(bend - rbase) : R;
     uint32_t dk[PER], rk[PER];
     double rec[PER][4];
     uint32_t key[PER];
 #pragma unroll
     for (int k = 0; k < PER; ++k) {
       const int64_t i = rbase + k * T + threadIdx.x;
-      const bool act = i < n;
+      const bool act = i < bend;
       dk[k] = 0;
       rec[k][0] = rec[k][1] = rec[k][2] = rec[k][3] = 0.0;
       key[k] = sentinel;
@@ -1246,17 +1244,18 @@ __global__ void __launch_bounds__(TS3_T)
 #pragma unroll
     for (int k = 0; k < PER; ++k) {
       const int64_t i = rbase + k * T + threadIdx.x;
-      if (i < n) {
+      if (i < bend) {
         const uint32_t ls = rs[dk[k]] + rk[k];
+        pos[i] = gofs[dk[k]] + rk[k];
 #pragma unroll
         for (int w = 0; w < W; ++w) stage[W * ls + w] = rec[k][w];
         if (F32) skey[ls] = key[k];
-        sbi[ls] = (dk[k] << 13) | uint32_t(i - base);
+        sbin[ls] = uint16_t(dk[k]);
       }
     }
     __syncthreads();
     for (int j = threadIdx.x; j < nround; j += T) {
-      const uint32_t d = sbi[j] >> 13;
+      const uint32_t d = sbin[j];
       const uint32_t g = gofs[d] + (uint32_t(j) - rs[d]);
       if (F32) {
         reinterpret_cast<double2*>(srec)[g] = make_double2(stage[2 * j], stage[2 * j + 1]);
@@ -1265,7 +1264,6 @@ __global__ void __launch_bounds__(TS3_T)
         srec[g] = make_double4(stage[W * j], stage[W * j + 1], stage[W * j + 2],
                                HASQ ? stage[W * j + 3] : 0.0);
       }
-      sv[g] = uint32_t(base) + (sbi[j] & 8191u);
     }
     __syncthreads();
     for (int d = threadIdx.x; d < kTileMaxBins; d += T) {
@@ -1385,8 +1383,15 @@ __global__ void __launch_bounds__(TA_T)
 }
 
 // step 5: node (i, j, k) of the mesh lies in the tiles a = i >> tb and, on a
-// tile face (i a multiple of the tile width), a - 1, per axis
-template <bool F32>
+// tile face (i a multiple of the tile width), a - 1, per axis.  Bound by the
+// latency of the chunk blocks' loads where a node has many of them (a corner
+// of eight central tiles): LPN lanes share a node, lane q of them taking the
+// chunks q, q + LPN, ... of each tile (integer sums: any order).  Eight lanes
+// on meshes of at most kNodesSplit nodes, where one lane per node leaves CUs
+// idle; above it the loads of one lane per node, contiguous over a wave, fill
+// the chip.
+constexpr uint32_t kNodesSplit = 1u << 19;
+template <bool F32, int LPN>
 __global__ void k_tile_nodes(const unsigned long long* __restrict__ part,
                              const TilePlan* __restrict__ tp, TileParams p,
                              double* __restrict__ rho) {
@@ -1395,7 +1400,13 @@ __global__ void k_tile_nodes(const unsigned long long* __restrict__ part,
   const int W = F32 ? 1 : 2;
   const double unscale = tp->unscale;
   const bool bad = tp->bad != 0;
-  for (uint32_t g = blockIdx.x * blockDim.x + threadIdx.x; g < ntot; g += gridDim.x * blockDim.x) {
+  const uint32_t q = threadIdx.x / (blockDim.x / LPN);  // lane of the node
+  const uint32_t per = blockDim.x / LPN;
+  __shared__ unsigned long long sum[LPN > 1 ? 2 * kThreads : 1];
+  // uniform trip count: every thread meets the barriers
+  for (uint32_t g0 = blockIdx.x * per; g0 < ntot; g0 += gridDim.x * per) {
+    const uint32_t g = g0 + threadIdx.x % per;
+    const bool act = g < ntot;
     const int k = int(g / (nx * ny)), r = int(g - uint32_t(k) * nx * ny);
     const int j = r / int(nx), i = r - j * int(nx);
     const int ci[3] = {i, j, k};
@@ -1403,6 +1414,7 @@ __global__ void k_tile_nodes(const unsigned long long* __restrict__ part,
     for (int a = 0; a < 3; ++a) {
       const int t = ci[a] >> p.tb[a];
       nta[a] = 0;
+      if (!act) continue;
       if (t < p.nt[a]) ta[a][nta[a]++] = t;
       if ((ci[a] & ((1 << p.tb[a]) - 1)) == 0 && t >= 1) ta[a][nta[a]++] = t - 1;
     }
@@ -1417,10 +1429,10 @@ __global__ void k_tile_nodes(const unsigned long long* __restrict__ part,
           // four chunk blocks at a time, their loads in flight together
           // (integer sums: the order does not matter)
           const uint32_t c1 = tp->wl[t + 1];
-          uint32_t c = tp->wl[t];
-          const int64_t cs = int64_t(p.nodes) * W;
-          for (; c + 4 <= c1; c += 4) {
-            const unsigned long long* blk = part + int64_t(c) * cs + local;
+          uint32_t c = tp->wl[t] + q;
+          const int64_t cw = int64_t(p.nodes) * W, cs = cw * LPN;
+          for (; c + 3 * LPN < c1; c += 4 * LPN) {
+            const unsigned long long* blk = part + int64_t(c) * cw + local;
             const unsigned long long h0 = blk[0], h1 = blk[cs], h2 = blk[2 * cs], h3 = blk[3 * cs];
             H += (h0 + h1) + (h2 + h3);
             if (!F32) {
@@ -1429,12 +1441,25 @@ __global__ void k_tile_nodes(const unsigned long long* __restrict__ part,
               L += (l0 + l1) + (l2 + l3);
             }
           }
-          for (; c < c1; ++c) {
-            const unsigned long long* blk = part + int64_t(c) * cs + local;
+          for (; c < c1; c += LPN) {
+            const unsigned long long* blk = part + int64_t(c) * cw + local;
             H += blk[0];
             if (!F32) L += blk[p.nodes];
           }
         }
+    if constexpr (LPN > 1) {
+      sum[threadIdx.x] = H;
+      sum[kThreads + threadIdx.x] = L;
+      __syncthreads();
+      if (q == 0)
+        for (uint32_t u = 1; u < LPN; ++u) {
+          H += sum[threadIdx.x + u * per];
+          L += sum[kThreads + threadIdx.x + u * per];
+        }
+      __syncthreads();
+      if (q) continue;
+    }
+    if (!act) continue;
     double v = double((long long)H);
     if (!F32) v = v + double((long long)L) * 2.3283064365386963e-10;  // 2^-32
     rho[g] = bad ? __builtin_nan("") : v * unscale;
@@ -1667,7 +1692,16 @@ static void deposit_tiled(osc_ctx* c, const DepositArgs& a, double* rho, SortedP
   cp.hasq = a.q != nullptr;
   cp.q_each = a.q_each;
   const int nbins = tp.ntiles + 1;
-  const int nb = int((n + TS_P - 1) / TS_P);
+  // Particles per count / scatter block: 8192 keeps the runs of a bin long
+  // (the scatter's stores) once there are two blocks per CU; below, enough
+  // blocks to reach every CU matter more
+  int tsp = TS_T;
+  while (tsp < TS_P && int64_t(tsp) * 512 < n) tsp <<= 1;
+  const int nb = int((n + tsp - 1) / tsp);
+  // particles per gather item, by the same rule (an item stages its tile's
+  // nodes first): 512 to 4096
+  int gchunk = 512;
+  while (gchunk < kTileGatherChunk && int64_t(gchunk) * 1024 < n) gchunk <<= 1;
   // chunks: about 512 work items for the whole bunch, 1024 to 32768 particles
   int chunk = 1024;
   while (chunk < 32768 && int64_t(chunk) * 512 < n) chunk <<= 1;
@@ -1686,7 +1720,7 @@ static void deposit_tiled(osc_ctx* c, const DepositArgs& a, double* rho, SortedP
     ProfScope ps(c, ST_DEP_KEYS);
     DevBuf hpart(c->pool, a.hash ? sizeof(uint64_t) * size_t(nb) : 0);
     hipLaunchKernelGGL(k_tile_count, dim3(nb), dim3(TS_T), 0, c->stream, a.x, a.y, a.z, a.q, n,
-                       tp, hist.as<uint32_t>(), nb, cnt, pl, hpart.as<uint64_t>());
+                       tp, tsp, hist.as<uint32_t>(), nb, cnt, pl, hpart.as<uint64_t>());
     OSC_HIP(hipGetLastError());
     if (a.hash) {
       hipLaunchKernelGGL(k_hash_sum, dim3(1), dim3(kThreads), 0, c->stream,
@@ -1700,12 +1734,12 @@ static void deposit_tiled(osc_ctx* c, const DepositArgs& a, double* rho, SortedP
                        total.as<uint32_t>());
     OSC_HIP(hipGetLastError());
     hipLaunchKernelGGL(k_tile_plan, dim3(1), dim3(1024), 0, c->stream, total.as<const uint32_t>(),
-                       tp.ntiles, n, a.q_each, int(a.q != nullptr), chunk, pl);
+                       tp.ntiles, n, a.q_each, int(a.q != nullptr), chunk, gchunk, pl);
     OSC_HIP(hipGetLastError());
     uint32_t* skp = f32 ? sk.as<uint32_t>() : nullptr;
     auto scatter = [&](auto kern) {
       hipLaunchKernelGGL(kern, dim3(nb), dim3(TS3_T), 0, c->stream, a.x, a.y, a.z, a.q, n, tp,
-                         hist.as<const uint32_t>(), nb, pl, srec.as<double4>(), sv.as<uint32_t>(),
+                         tsp, hist.as<const uint32_t>(), nb, pl, srec.as<double4>(), sv.as<uint32_t>(),
                          skp);
     };
     if (f32 && a.q)
@@ -1734,12 +1768,11 @@ static void deposit_tiled(osc_ctx* c, const DepositArgs& a, double* rho, SortedP
   }
   {
     ProfScope ps(c, ST_DEP_NODES);
-    if (f32)
-      hipLaunchKernelGGL(k_tile_nodes<true>, dim3(nblk(ntot)), dim3(kThreads), 0, c->stream,
-                         part.as<const unsigned long long>(), pl, tp, rho);
-    else
-      hipLaunchKernelGGL(k_tile_nodes<false>, dim3(nblk(ntot)), dim3(kThreads), 0, c->stream,
-                         part.as<const unsigned long long>(), pl, tp, rho);
+    const bool split = ntot <= int64_t(kNodesSplit);
+    auto* k = f32 ? (split ? k_tile_nodes<true, 8> : k_tile_nodes<true, 1>)
+                  : (split ? k_tile_nodes<false, 8> : k_tile_nodes<false, 1>);
+    hipLaunchKernelGGL(k, dim3(nblk(split ? 8 * ntot : ntot)), dim3(kThreads), 0, c->stream,
+                       part.as<const unsigned long long>(), pl, tp, rho);
     OSC_HIP(hipGetLastError());
   }
   if (keep) {
@@ -1753,8 +1786,7 @@ static void deposit_tiled(osc_ctx* c, const DepositArgs& a, double* rho, SortedP
     keep->tile.md = nullptr;
     keep->plan = std::move(plan);
     keep->total = std::move(total);
-    keep->chunk = chunk;
-    keep->nwork = nwork;
+    keep->gchunk = gchunk;
   }
 }
 

@@ -626,32 +626,47 @@ __global__ void __launch_bounds__(kThreads)
 // ---------------------------------------------------------------------------
 // tile gather: the particles of the tiled deposit, in bin order
 // ---------------------------------------------------------------------------
-constexpr int TG_T = 1024;
-
-// One workgroup per gather item (kTileGatherChunk particles of one tile's
-// bin): the E and B values of the tile's nodes are staged in LDS as node
-// records of 7 values (FP64; F32: the values of the FP32 node records; the
-// odd stride in 4-byte words spreads random nodes over the LDS banks), then
-// each particle sums its 8 nodes from there in the upstream
-// order and leaves (E, B, clamped, 0) in the 64-byte record out8[sv[s]] for
-// k_unpack.  FP64: cell and weights from the coordinates by the
-// interpolate_field rule, the values of k_interp_cells; F32: the deposit's cell
-// key and FP32 weights, the values of k_interp_cells32.  Tiles holding fewer
-// than kTileGatherStage particles, and particles whose cell lies outside the
-// tile (a gather mesh other than the deposit's), read the planar fields.
-constexpr int TG_PER = kTileGatherChunk / TG_T;
+// Geometry of the tile gather.  Tiles of 8^3 cells (729 nodes) take 40 KB of
+// LDS (FP32: 20 KB), so that three (seven) workgroups of 256 share a CU and
+// one's node loads overlap another's sums, in items down to 512 particles;
+// larger tiles need most of the LDS for one workgroup of 1024.
+template <bool F32, bool SMALL>
+struct TileGatherGeo {
+  static constexpr int T = SMALL ? 256 : 1024;
+  static constexpr int PER = SMALL ? 2 : 4;  // particles in flight per thread
+  static constexpr int kNodes = 729;         // most nodes of a SMALL tile
+  static constexpr int kBytes = SMALL ? (kNodes * 7 * (F32 ? 4 : 8) + 7) / 8 * 8
+                                      : (F32 ? kTileGatherBytes32 : kTileGatherBytes64);
+  static_assert(512 % (T * PER) == 0 || kTileGatherChunk % (T * PER) == 0, "whole rounds");
+};
 constexpr int kTileGatherStage = 512;
-static_assert(kTileGatherChunk % TG_T == 0, "whole particles per thread");
-template <bool F32>
-__global__ void __launch_bounds__(TG_T)
-    k_tile_gather(const double* __restrict__ ef, const double* __restrict__ bf, int wantE,
-                  int wantB, TileParams tg, const TilePlan* __restrict__ tp,
-                  const uint32_t* __restrict__ total, const double4* __restrict__ srec,
-                  const uint32_t* __restrict__ sk, const uint32_t* __restrict__ sv, IP p,
-                  double* __restrict__ out8, uint32_t* __restrict__ nclamp) {
+
+// One workgroup per gather item (gchunk particles of one tile's bin): the E
+// and B values of the tile's nodes are staged in LDS as node records of 7
+// values (FP64; F32: the values of the FP32 node records; the odd stride in
+// 4-byte words spreads random nodes over the LDS banks), then each particle
+// sums its 8 nodes from there in the upstream order and leaves its values (E
+// and B, or the one asked for) at its slot of out, in bin order: contiguous
+// stores, which k_tile_return takes to particle order.  (Storing each result
+// as a 64-byte record at its particle's place instead cost a random line per
+// particle and a pass over 64 bytes of each after it.)  FP64: cell and weights
+// from the coordinates by the interpolate_field rule, the values of
+// k_interp_cells; F32: the deposit's cell key and FP32 weights, the values of
+// k_interp_cells32.  Tiles holding fewer than kTileGatherStage particles, and
+// particles whose cell lies outside the tile (a gather mesh other than the
+// deposit's), read the planar fields.
+template <bool F32, bool SMALL, int NV>
+__global__ void __launch_bounds__((TileGatherGeo<F32, SMALL>::T))
+    k_tile_gather(const double* __restrict__ ef, const double* __restrict__ bf, TileParams tg,
+                  int gchunk, const TilePlan* __restrict__ tp, const uint32_t* __restrict__ total,
+                  const double4* __restrict__ srec, const uint32_t* __restrict__ sk, IP p,
+                  typename std::conditional<F32, float, double>::type* __restrict__ out,
+                  uint32_t* __restrict__ nclamp) {
   using A = typename std::conditional<F32, float, double>::type;
+  using G = TileGatherGeo<F32, SMALL>;
   constexpr int NS = 7;  // LDS values per node record
-  __shared__ double lds_raw[(F32 ? kTileGatherBytes32 : kTileGatherBytes64) / 8];
+  constexpr int T = G::T, PER = G::PER;
+  __shared__ double lds_raw[G::kBytes / 8];
   __shared__ int s_t;
   __shared__ uint32_t cnt;
   A* L = reinterpret_cast<A*>(lds_raw);
@@ -680,95 +695,89 @@ __global__ void __launch_bounds__(TG_T)
   const uint32_t count = total[t];
   const bool staged = count >= uint32_t(kTileGatherStage);  // uniform
   if (staged) {
-    for (int node = threadIdx.x; node < nodes; node += TG_T) {
+    for (int node = threadIdx.x; node < nodes; node += T) {
       const int lk = node / tn01, rr = node - lk * tn01, lj = rr / tn0, li = rr - lj * tn0;
       const int gi = ox + li, gj = oy + lj, gk = oz + lk;
       const bool in = gi < p.nn[0] && gj < p.nn[1] && gk < p.nn[2];
       const int64_t g = in ? gi + sy * gj + sz * gk : 0;
-      A v[6];
+      A v[NV];
 #pragma unroll
-      for (int c = 0; c < 6; ++c) {
-        const double* F = c < 3 ? ef : bf;
-        v[c] = A((in && (c < 3 ? wantE : wantB)) ? F[(c % 3) * nt + g] : 0.0);
-      }
+      for (int c = 0; c < NV; ++c) v[c] = A(in ? (c < 3 ? ef : bf)[(c % 3) * nt + g] : 0.0);
 #pragma unroll
-      for (int c = 0; c < 6; ++c) L[NS * node + c] = v[c];
+      for (int c = 0; c < NV; ++c) L[NS * node + c] = v[c];
     }
     __syncthreads();
   }
-  const int64_t s0 = int64_t(tp->bstart[t]) +
-                     int64_t(int(blockIdx.x) - int(tp->gwl[t])) * kTileGatherChunk;
-  const int64_t send = int64_t(tp->bstart[t]) + count;
+  const int64_t sbeg = int64_t(tp->bstart[t]) + int64_t(int(blockIdx.x) - int(tp->gwl[t])) * gchunk;
+  const int64_t sbin = int64_t(tp->bstart[t]) + count;
+  const int64_t send = sbeg + gchunk < sbin ? sbeg + gchunk : sbin;
   const int wx = 1 << tg.tb[0], wy = 1 << tg.tb[1], wz = 1 << tg.tb[2];
-  // the thread's particles: records first, so that their loads overlap
-  double4 rec[TG_PER];
-  uint32_t key[TG_PER], dst[TG_PER];
-#pragma unroll
-  for (int k = 0; k < TG_PER; ++k) {
-    const int64_t s = s0 + k * TG_T + threadIdx.x;
-    rec[k] = make_double4(0.0, 0.0, 0.0, 0.0);
-    key[k] = 0;
-    dst[k] = 0;
-    if (s < send) {
-      if (F32) {
-        const float4 r = reinterpret_cast<const float4*>(srec)[s];
-        rec[k] = make_double4(r.x, r.y, r.z, 0.0);
-        key[k] = sk[s];
-      } else {
-        rec[k] = srec[s];
-      }
-      dst[k] = sv[s];
-    }
-  }
   uint32_t mine = 0;
+  for (int64_t s0 = sbeg; s0 < send; s0 += T * PER) {
+    // the thread's particles: records first, so that their loads overlap
+    double4 rec[PER];
+    uint32_t key[PER];
 #pragma unroll
-  for (int k = 0; k < TG_PER; ++k) {
-    const int64_t s = s0 + k * TG_T + threadIdx.x;
-    if (s >= send) continue;
-    A ab, de, gh;
-    int i0, j0, k0;
-    bool fl = false;
-    if (F32) {
-      const uint32_t nx = uint32_t(p.nn[0]), ny = uint32_t(p.nn[1]);
-      i0 = int(key[k] % nx);
-      j0 = int((key[k] / nx) % ny);
-      k0 = int(key[k] / (nx * ny));
-      ab = A(rec[k].x);
-      de = A(rec[k].y);
-      gh = A(rec[k].z);
-    } else {
-      const double xr = rec[k].x, yr = rec[k].y, zr = rec[k].z;
-      const int ip = clamp_idx(xr, p.mn[0], p.hinv[0], p.nhi[0], fl);
-      const int jp = clamp_idx(yr, p.mn[1], p.hinv[1], p.nhi[1], fl);
-      const int kp = clamp_idx(zr, p.mn[2], p.hinv[2], p.nhi[2], fl);
-      ab = A(((p.mn[0] - xr) + ip * p.delta[0]) * p.hinv[0]);
-      de = A(((p.mn[1] - yr) + jp * p.delta[1]) * p.hinv[1]);
-      gh = A(((p.mn[2] - zr) + kp * p.delta[2]) * p.hinv[2]);
-      i0 = ip - p.nlo[0];
-      j0 = jp - p.nlo[1];
-      k0 = kp - p.nlo[2];
-      i0 = i0 < 0 ? 0 : (i0 > p.nn[0] - 2 ? p.nn[0] - 2 : i0);
-      j0 = j0 < 0 ? 0 : (j0 > p.nn[1] - 2 ? p.nn[1] - 2 : j0);
-      k0 = k0 < 0 ? 0 : (k0 > p.nn[2] - 2 ? p.nn[2] - 2 : k0);
+    for (int k = 0; k < PER; ++k) {
+      const int64_t s = s0 + k * T + threadIdx.x;
+      rec[k] = make_double4(0.0, 0.0, 0.0, 0.0);
+      key[k] = 0;
+      if (s < send) {
+        if (F32) {
+          const float4 r = reinterpret_cast<const float4*>(srec)[s];
+          rec[k] = make_double4(r.x, r.y, r.z, 0.0);
+          key[k] = sk[s];
+        } else {
+          rec[k] = srec[s];
+        }
+      }
     }
-    mine += fl ? 1u : 0u;
-    const int li = i0 - ox, lj = j0 - oy, lk = k0 - oz;
-    A v[6] = {A(0), A(0), A(0), A(0), A(0), A(0)};
-    if (staged && li >= 0 && li < wx && lj >= 0 && lj < wy && lk >= 0 && lk < wz) {
-      const int q0 = li + tn0 * lj + tn01 * lk;
 #pragma unroll
-      for (int c = 0; c < 6; ++c)
-        if (c < 3 ? wantE : wantB)
+    for (int k = 0; k < PER; ++k) {
+      const int64_t s = s0 + k * T + threadIdx.x;
+      if (s >= send) continue;
+      A ab, de, gh;
+      int i0, j0, k0;
+      bool fl = false;
+      if (F32) {
+        const uint32_t nx = uint32_t(p.nn[0]), ny = uint32_t(p.nn[1]);
+        i0 = int(key[k] % nx);
+        j0 = int((key[k] / nx) % ny);
+        k0 = int(key[k] / (nx * ny));
+        ab = A(rec[k].x);
+        de = A(rec[k].y);
+        gh = A(rec[k].z);
+      } else {
+        const double xr = rec[k].x, yr = rec[k].y, zr = rec[k].z;
+        const int ip = clamp_idx(xr, p.mn[0], p.hinv[0], p.nhi[0], fl);
+        const int jp = clamp_idx(yr, p.mn[1], p.hinv[1], p.nhi[1], fl);
+        const int kp = clamp_idx(zr, p.mn[2], p.hinv[2], p.nhi[2], fl);
+        ab = A(((p.mn[0] - xr) + ip * p.delta[0]) * p.hinv[0]);
+        de = A(((p.mn[1] - yr) + jp * p.delta[1]) * p.hinv[1]);
+        gh = A(((p.mn[2] - zr) + kp * p.delta[2]) * p.hinv[2]);
+        i0 = ip - p.nlo[0];
+        j0 = jp - p.nlo[1];
+        k0 = kp - p.nlo[2];
+        i0 = i0 < 0 ? 0 : (i0 > p.nn[0] - 2 ? p.nn[0] - 2 : i0);
+        j0 = j0 < 0 ? 0 : (j0 > p.nn[1] - 2 ? p.nn[1] - 2 : j0);
+        k0 = k0 < 0 ? 0 : (k0 > p.nn[2] - 2 ? p.nn[2] - 2 : k0);
+      }
+      mine += fl ? 1u : 0u;
+      const int li = i0 - ox, lj = j0 - oy, lk = k0 - oz;
+      A v[NV];
+      if (staged && li >= 0 && li < wx && lj >= 0 && lj < wy && lk >= 0 && lk < wz) {
+        const int q0 = li + tn0 * lj + tn01 * lk;
+#pragma unroll
+        for (int c = 0; c < NV; ++c)
           v[c] = wsum8_any<A>(
               [&](int r2, int d) {
                 return L[NS * (q0 + d + ((r2 & 1) ? tn0 : 0) + ((r2 & 2) ? tn01 : 0)) + c];
               },
               ab, de, gh);
-    } else {
-      const int64_t b = i0 + sy * j0 + sz * k0;
+      } else {
+        const int64_t b = i0 + sy * j0 + sz * k0;
 #pragma unroll
-      for (int c = 0; c < 6; ++c)
-        if (c < 3 ? wantE : wantB) {
+        for (int c = 0; c < NV; ++c) {
           const double* F = (c < 3 ? ef : bf) + (c % 3) * nt;
           v[c] = wsum8_any<A>(
               [&](int r2, int d) {
@@ -776,82 +785,137 @@ __global__ void __launch_bounds__(TG_T)
               },
               ab, de, gh);
         }
+      }
+#pragma unroll
+      for (int c = 0; c < NV; ++c) out[NV * s + c] = v[c];
     }
-    double2* o = reinterpret_cast<double2*>(out8 + 8 * int64_t(dst[k]));
-    o[0] = make_double2(double(v[0]), double(v[1]));
-    o[1] = make_double2(double(v[2]), double(v[3]));
-    o[2] = make_double2(double(v[4]), double(v[5]));
-    o[3] = make_double2(fl ? 1.0 : 0.0, 0.0);
   }
   if (mine) atomicAdd(&cnt, mine);
   __syncthreads();
   if (threadIdx.x == 0 && cnt) atomicAdd(nclamp, cnt);
 }
 
-// The off-mesh bin of the tiled deposit (slots bstart[ntiles] on): the
-// interpolate_field clamp rule from the coordinates (FP64: the record; F32:
-// x, y, z of the particle, the weights rounded as in k_interp_cells32),
-// the planar fields read directly.
-template <bool F32>
+// The results of k_tile_gather (val, NV values per slot) in particle order:
+// each wave reads the records of 64 consecutive particles (their slots from
+// pos; a scatter block's particles of one bin lie side by side, so the lines
+// are shared by the waves around) into LDS and stores them as contiguous runs
+// of E and B.  A particle of the off-mesh bin (slots from bstart[ntiles] on)
+// has no value there: it takes the interpolate_field clamp rule from its
+// coordinates here, the planar fields read directly (FP32: the weights
+// rounded as in k_interp_cells32).  Flags, where asked for: FP64 by the
+// clamp rule from the coordinates, F32 (the deposit's own mesh) the off-mesh
+// particles'.  E or B null: val holds the other's three values.
+template <bool F32, int NV>
 __global__ void __launch_bounds__(kThreads)
-    k_tile_gather_off(const double* __restrict__ ef, const double* __restrict__ bf, int wantE,
-                      int wantB, int ntiles, const TilePlan* __restrict__ tp,
-                      const uint32_t* __restrict__ total, const double4* __restrict__ srec,
-                      const uint32_t* __restrict__ sv, const double* __restrict__ x,
-                      const double* __restrict__ y, const double* __restrict__ z, IP p,
-                      double* __restrict__ out8, uint32_t* __restrict__ nclamp) {
+    k_tile_return(const typename std::conditional<F32, float, double>::type* __restrict__ val,
+                  const uint32_t* __restrict__ pos, int64_t n, const double* __restrict__ ef,
+                  const double* __restrict__ bf, int ntiles, const TilePlan* __restrict__ tp,
+                  const double* __restrict__ x, const double* __restrict__ y,
+                  const double* __restrict__ z, IP p, double* __restrict__ E,
+                  double* __restrict__ B, int8_t* __restrict__ clamped,
+                  uint32_t* __restrict__ nclamp) {
   using A = typename std::conditional<F32, float, double>::type;
-  __shared__ uint32_t cnt;
-  if (threadIdx.x == 0) cnt = 0;
-  __syncthreads();
+  // an odd stride in 4-byte (FP64: 8-byte) words against bank conflicts
+  constexpr int NP = NV + 1 - NV % 2;
+  __shared__ A stage[kThreads / 64][64 * NP];
+  const int lane = threadIdx.x & 63;
+  A* w = stage[threadIdx.x >> 6];
+  const uint32_t off = tp->bstart[ntiles];
   const int64_t sy = p.nn[0], sz = int64_t(p.nn[0]) * p.nn[1], nt = sz * p.nn[2];
-  const int64_t s0 = tp->bstart[ntiles], s1 = s0 + total[ntiles];
-  uint32_t mine = 0;
-  for (int64_t s = s0 + blockIdx.x * int64_t(blockDim.x) + threadIdx.x; s < s1;
-       s += int64_t(gridDim.x) * blockDim.x) {
-    const uint32_t dst = sv[s];
-    double xi, yi, zi;
-    if (F32) {
-      xi = x[dst];
-      yi = y[dst];
-      zi = z[dst];
-    } else {
-      const double4 r = srec[s];
-      xi = r.x;
-      yi = r.y;
-      zi = r.z;
-    }
-    bool fl = false;
-    const int ip = clamp_idx(xi, p.mn[0], p.hinv[0], p.nhi[0], fl);
-    const int jp = clamp_idx(yi, p.mn[1], p.hinv[1], p.nhi[1], fl);
-    const int kp = clamp_idx(zi, p.mn[2], p.hinv[2], p.nhi[2], fl);
-    const A ab = A(((p.mn[0] - xi) + ip * p.delta[0]) * p.hinv[0]);
-    const A de = A(((p.mn[1] - yi) + jp * p.delta[1]) * p.hinv[1]);
-    const A gh = A(((p.mn[2] - zi) + kp * p.delta[2]) * p.hinv[2]);
-    int i0 = ip - p.nlo[0], j0 = jp - p.nlo[1], k0 = kp - p.nlo[2];
-    i0 = i0 < 0 ? 0 : (i0 > p.nn[0] - 2 ? p.nn[0] - 2 : i0);
-    j0 = j0 < 0 ? 0 : (j0 > p.nn[1] - 2 ? p.nn[1] - 2 : j0);
-    k0 = k0 < 0 ? 0 : (k0 > p.nn[2] - 2 ? p.nn[2] - 2 : k0);
-    const int64_t b = i0 + sy * j0 + sz * k0;
-    A v[6] = {A(0), A(0), A(0), A(0), A(0), A(0)};
+  for (int64_t i0 = blockIdx.x * int64_t(blockDim.x) + (threadIdx.x & ~63); i0 < n;
+       i0 += int64_t(gridDim.x) * blockDim.x) {  // uniform per wave
+    const int nrec = n - i0 < 64 ? int(n - i0) : 64;
+    const int64_t i = i0 + lane;
+    bool fl = false, outside = false;
+    if (lane < nrec) {
+      const uint32_t s = pos[i];
+      outside = s >= off;
+      A v[NV];
+      if (!outside) {
 #pragma unroll
-    for (int c = 0; c < 6; ++c)
-      if (c < 3 ? wantE : wantB) {
-        const double* F = (c < 3 ? ef : bf) + (c % 3) * nt;
-        v[c] = wsum8_any<A>(
-            [&](int rr, int d) { return A(F[b + d + ((rr & 1) ? sy : 0) + ((rr & 2) ? sz : 0)]); },
-            ab, de, gh);
+        for (int c = 0; c < NV; ++c) v[c] = val[int64_t(NV) * s + c];
+        if (!F32 && clamped) {
+          (void)clamp_idx(x[i], p.mn[0], p.hinv[0], p.nhi[0], fl);
+          (void)clamp_idx(y[i], p.mn[1], p.hinv[1], p.nhi[1], fl);
+          (void)clamp_idx(z[i], p.mn[2], p.hinv[2], p.nhi[2], fl);
+        }
+      } else {
+        const double xi = x[i], yi = y[i], zi = z[i];
+        const int ip = clamp_idx(xi, p.mn[0], p.hinv[0], p.nhi[0], fl);
+        const int jp = clamp_idx(yi, p.mn[1], p.hinv[1], p.nhi[1], fl);
+        const int kp = clamp_idx(zi, p.mn[2], p.hinv[2], p.nhi[2], fl);
+        const A ab = A(((p.mn[0] - xi) + ip * p.delta[0]) * p.hinv[0]);
+        const A de = A(((p.mn[1] - yi) + jp * p.delta[1]) * p.hinv[1]);
+        const A gh = A(((p.mn[2] - zi) + kp * p.delta[2]) * p.hinv[2]);
+        int ii = ip - p.nlo[0], jj = jp - p.nlo[1], kk = kp - p.nlo[2];
+        ii = ii < 0 ? 0 : (ii > p.nn[0] - 2 ? p.nn[0] - 2 : ii);
+        jj = jj < 0 ? 0 : (jj > p.nn[1] - 2 ? p.nn[1] - 2 : jj);
+        kk = kk < 0 ? 0 : (kk > p.nn[2] - 2 ? p.nn[2] - 2 : kk);
+        const int64_t b = ii + sy * jj + sz * kk;
+#pragma unroll
+        for (int c = 0; c < NV; ++c) {
+          const double* F = (c < 3 ? ef : bf) + (c % 3) * nt;
+          v[c] = wsum8_any<A>(
+              [&](int rr, int d) {
+                return A(F[b + d + ((rr & 1) ? sy : 0) + ((rr & 2) ? sz : 0)]);
+              },
+              ab, de, gh);
+        }
       }
-    mine += fl ? 1u : 0u;
-    double2* o = reinterpret_cast<double2*>(out8 + 8 * int64_t(dst));
-    o[0] = make_double2(double(v[0]), double(v[1]));
-    o[1] = make_double2(double(v[2]), double(v[3]));
-    o[2] = make_double2(double(v[4]), double(v[5]));
-    o[3] = make_double2(fl ? 1.0 : 0.0, 0.0);
+#pragma unroll
+      for (int c = 0; c < NV; ++c) w[NP * lane + c] = v[c];
+      if (clamped) clamped[i] = fl ? 1 : 0;
+    }
+    // the clamped off-mesh particles (k_tile_gather counts its own)
+    const uint64_t bal = __ballot(fl && outside);
+    if (bal && lane == 0) atomicAdd(nclamp, uint32_t(__popcll(bal)));
+    wave_lds_sync();
+    double* first = E ? E : B;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      const int e = lane + 64 * k;  // value of the chunk: record e / 3, component e % 3
+      if (e / 3 < nrec) first[3 * i0 + e] = double(w[(e / 3) * NP + e % 3]);
+    }
+    if constexpr (NV == 6)
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        const int e = lane + 64 * k;
+        if (e / 3 < nrec) B[3 * i0 + e] = double(w[(e / 3) * NP + 3 + e % 3]);
+      }
+    wave_lds_sync();  // read before the next chunk overwrites the stage
   }
-  if (mine) atomicAdd(&cnt, mine);
-  __syncthreads();
-  if (threadIdx.x == 0 && cnt) atomicAdd(nclamp, cnt);
+}
+
+// gather of a tiled deposit's particles: k_tile_gather, k_tile_return
+template <bool F32, int NV>
+void tile_gather(osc_ctx* c, const SortedParticles& sp, const double* ef, const double* bf,
+                 const IP& p, const double* x, const double* y, const double* z, double* E,
+                 double* B, int8_t* clamped, uint32_t* cnt) {
+  using A = typename std::conditional<F32, float, double>::type;
+  const int64_t n = sp.n;
+  DevBuf val(c->pool, sizeof(A) * NV * n);
+  const TilePlan* tpl = sp.plan.as<const TilePlan>();
+  // one field only: in the place of E
+  const double* f0 = E ? ef : bf;
+  {
+    ProfScope ps(c, ST_GATHER);
+    // at most one partial chunk per tile beyond the full ones
+    const int64_t items = (n + sp.gchunk - 1) / sp.gchunk + sp.tile.ntiles;
+    const bool small = sp.tile.nodes <= TileGatherGeo<F32, true>::kNodes;
+    hipLaunchKernelGGL((small ? k_tile_gather<F32, true, NV> : k_tile_gather<F32, false, NV>),
+                       dim3(unsigned(items)),
+                       dim3(small ? TileGatherGeo<F32, true>::T : TileGatherGeo<F32, false>::T), 0,
+                       c->stream, f0, bf, sp.tile, sp.gchunk, tpl, sp.total.as<const uint32_t>(),
+                       sp.srec.as<const double4>(), sp.sk.as<const uint32_t>(), p, val.as<A>(),
+                       cnt);
+    OSC_HIP(hipGetLastError());
+  }
+  ProfScope po(c, ST_GATHER_OUT);
+  const int64_t nb = std::min<int64_t>((n + kThreads - 1) / kThreads, 65536 * 8);
+  hipLaunchKernelGGL((k_tile_return<F32, NV>), dim3(unsigned(nb)), dim3(kThreads), 0, c->stream,
+                     val.as<const A>(), sp.sv.as<const uint32_t>(), n, f0, bf, sp.tile.ntiles, tpl,
+                     x, y, z, p, E, B, clamped, cnt);
+  OSC_HIP(hipGetLastError());
 }
 
 }  // namespace
@@ -884,46 +948,23 @@ void interpolate_sorted(osc_ctx* c, const InterpArgs& a, const double* ef, const
   fill_u32(c, cnt, 1, 0u);
   if (sp.tiled) {
     // bin order of the tiled deposit: each tile's nodes staged in LDS
-    OSC_REQUIRE(!sp.f32 || (x && y && z), OSC_ERR_ARG, "FP32 gather: coordinates needed");
-    const int64_t n = sp.n;
-    if (n <= 0) return;
-    DevBuf out8(c->pool, sizeof(double) * 8 * n);
-    const TilePlan* tpl = sp.plan.as<const TilePlan>();
-    const uint32_t* tot = sp.total.as<const uint32_t>();
-    const int wantE = int(E && ef), wantB = int(B && bf);
-    // gather items: at most one partial chunk per tile beyond the full ones
-    const int64_t gitems = (n + kTileGatherChunk - 1) / kTileGatherChunk + sp.tile.ntiles;
-    {
-      ProfScope ps(c, ST_GATHER);
-      if (sp.f32) {
-        hipLaunchKernelGGL(k_tile_gather<true>, dim3(unsigned(gitems)), dim3(TG_T), 0, c->stream,
-                           ef, bf, wantE, wantB, sp.tile, tpl, tot,
-                           sp.srec.as<const double4>(), sp.sk.as<const uint32_t>(),
-                           sp.sv.as<const uint32_t>(), p, out8.as<double>(), cnt);
-        OSC_HIP(hipGetLastError());
-        hipLaunchKernelGGL(k_tile_gather_off<true>, dim3(64), dim3(kThreads), 0, c->stream, ef, bf,
-                           wantE, wantB, sp.tile.ntiles, tpl, tot, sp.srec.as<const double4>(),
-                           sp.sv.as<const uint32_t>(), x, y, z, p, out8.as<double>(), cnt);
-      } else {
-        hipLaunchKernelGGL(k_tile_gather<false>, dim3(unsigned(gitems)), dim3(TG_T), 0,
-                           c->stream, ef, bf, wantE, wantB, sp.tile, tpl, tot,
-                           sp.srec.as<const double4>(), static_cast<const uint32_t*>(nullptr),
-                           sp.sv.as<const uint32_t>(), p, out8.as<double>(), cnt);
-        OSC_HIP(hipGetLastError());
-        hipLaunchKernelGGL(k_tile_gather_off<false>, dim3(64), dim3(kThreads), 0, c->stream, ef,
-                           bf, wantE, wantB, sp.tile.ntiles, tpl, tot, sp.srec.as<const double4>(),
-                           sp.sv.as<const uint32_t>(), static_cast<const double*>(nullptr),
-                           static_cast<const double*>(nullptr), static_cast<const double*>(nullptr),
-                           p, out8.as<double>(), cnt);
-      }
+    OSC_REQUIRE(x && y && z, OSC_ERR_ARG, "tile gather: coordinates needed");
+    if (sp.n <= 0) return;
+    double* Eo = ef ? E : nullptr;
+    double* Bo = bf ? B : nullptr;
+    if (!Eo && !Bo) {  // flags and their count only
+      const int64_t nb = std::min<int64_t>((sp.n + kThreads - 1) / kThreads, 65536 * 8);
+      hipLaunchKernelGGL(k_interp, dim3(unsigned(nb)), dim3(kThreads), 0, c->stream, nullptr,
+                         nullptr, sp.n, x, y, z, p, nullptr, nullptr, clamped, cnt);
       OSC_HIP(hipGetLastError());
+      return;
     }
-    ProfScope po(c, ST_GATHER_OUT);
-    const int64_t nb = std::min<int64_t>((n + kThreads - 1) / kThreads, 65536 * 8);
-    hipLaunchKernelGGL(k_unpack, dim3(unsigned(nb)), dim3(kThreads), kUnpackOccLds, c->stream,
-                       out8.as<const double>(), n, (E && ef) ? E : nullptr,
-                       (B && bf) ? B : nullptr, clamped);
-    OSC_HIP(hipGetLastError());
+    if (Eo && Bo)
+      (sp.f32 ? tile_gather<true, 6> : tile_gather<false, 6>)(c, sp, ef, bf, p, x, y, z, Eo, Bo,
+                                                              clamped, cnt);
+    else
+      (sp.f32 ? tile_gather<true, 3> : tile_gather<false, 3>)(c, sp, ef, bf, p, x, y, z, Eo, Bo,
+                                                              clamped, cnt);
     return;
   }
   if (!packed && sp.n < 2 * nt) {
@@ -1046,7 +1087,7 @@ int64_t interpolate(osc_ctx* c, const InterpArgs& a, const double* ef, const dou
       DevBuf rec(c->pool, sizeof(double) * 8 * nt);
       if (!c->kept.tiled) pack_nodes(c, a, ef, bf, rec.as<double>());
       if (deposit_hash_matches(c)) {
-        interpolate_sorted(c, a, ef, bf, c->kept, E, B, clamped, rec.as<const double>());
+        interpolate_sorted(c, a, ef, bf, c->kept, E, B, clamped, rec.as<const double>(), x, y, z);
         return 0;
       }
       SortedParticles sp;

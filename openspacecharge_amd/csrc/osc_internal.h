@@ -164,7 +164,7 @@ constexpr int kTileMaxBins = 2048;
 // LDS of the tile gather's node records (E and B of every node of a tile, 7
 // values per node: FP64 and FP32)
 constexpr int kTileGatherBytes64 = 155648, kTileGatherBytes32 = 79872;
-// particles per work item of the tile gather
+// most particles per work item of the tile gather
 constexpr int kTileGatherChunk = 4096;
 struct TileParams {
   double mn[3], dinv[3], d[3];
@@ -178,7 +178,7 @@ struct TileParams {
 struct TilePlan {
   uint32_t bstart[kTileMaxBins + 1];  // first slot of every bin
   uint32_t wl[kTileMaxBins + 1];      // first work item of every tile; wl[ntiles] = all
-  uint32_t gwl[kTileMaxBins + 1];     // the same for the gather's items of kTileGatherChunk
+  uint32_t gwl[kTileMaxBins + 1];     // the same for the gather's items of gchunk
   double scale, unscale;              // 2^E, 2^-E
   int bad;                            // a charge or the bound n max|q| is not finite
   int pad;
@@ -189,7 +189,8 @@ struct TilePlan {
 // deposit (for a following gather) or by sort_for_gather
 struct SortedParticles {
   int64_t n = 0;
-  DevBuf sv;    // original particle index of each sorted slot (u32)
+  DevBuf sv;    // original particle index of each sorted slot (u32); tiled: the
+                // slot of each particle instead
   DevBuf srec;  // 32-byte records (x, y, z, q) in sorted order (double4), or with
                 // f32 16-byte records (ab, de, gh, q) of the FP32 deposit (float4)
   bool f32 = false;
@@ -200,8 +201,7 @@ struct SortedParticles {
   bool tiled = false;
   TileParams tile{};
   DevBuf plan, total;
-  int chunk = 0;
-  int64_t nwork = 0;
+  int gchunk = 0;  // particles per work item of the gather
 };
 
 constexpr int kMeshDev = 256, kCounterBytes = 512;
