@@ -1,5 +1,6 @@
 // Green-function builders (FP64, on the device), their R2C spectra, the
 // spectrum cache, and conversions to the upstream full-spectrum convention.
+#include "fast_math.h"
 #include "igf_math.h"
 #include "osc_internal.h"
 
@@ -88,6 +89,75 @@ __global__ void __launch_bounds__(64)
     if (!((half >> mod) & 1) || c == L[mod] / 2 - 1) {
       F[at + step] = -g;
       if (wev) F[ev + step] = -g;
+    }
+  }
+}
+
+// The primitives of up to three E components (F[ic - 1], null: not wanted) on
+// the whole offset grid at upstream's coordinates: F = prim(u, v, w) * factor,
+// as k_prim_offset without mirrors.  Bound by the FP64 instructions of the
+// logarithms, arc tangents, roots and quotients: xlafun2_tab takes the first
+// two from fast_math.h, the components' three roots -- of sums in different
+// orders, which may differ by an ulp that the cancelling logarithms magnify,
+// so each component keeps its own -- come from one root and two corrections,
+// and a thread marches kPrimZ planes, its table and row products staying.
+// 256^3 grid, three components: 0.188 ms (about 400 vector instructions a node
+// and 0.4 GB stored), where three launches of k_prim_offset take 0.476 ms
+// (about 350 FP64 instructions a value each).
+constexpr int kPrimZ = 4;
+struct Prim3 {
+  double* F[3];
+  double factor[3];
+};
+// CHECK: coordinates the host has not seen, or at which a root, a logarithm or
+// a quotient may leave the range of the plain instruction sequences (plain_grid)
+template <bool CHECK>
+__global__ void __launch_bounds__(256)
+    k_prim3(Prim3 o, int L0, int L1, int L2, double dx, double dy, double dz, double umin,
+            double vmin, double wmin, const MeshDev* __restrict__ md, double gamma, int img,
+            const FastMathTab* __restrict__ table) {
+  __shared__ FastMathTab tab;
+  {
+    const unsigned* src = reinterpret_cast<const unsigned*>(table);
+    unsigned* dst = reinterpret_cast<unsigned*>(&tab);
+    for (int t = threadIdx.y * 64 + threadIdx.x; t < int(sizeof(FastMathTab) / 4); t += 256) dst[t] = src[t];
+  }
+  __syncthreads();
+  const int i = blockIdx.x * 64 + threadIdx.x, j = blockIdx.y * 4 + threadIdx.y;
+  if (i >= L0 || j >= L1) return;
+  if (md) {  // the spacing from the device record, as k_prim_offset
+    dx = md->d[0];
+    dy = md->d[1];
+    dz = md->d[2] * gamma;
+    o.factor[0] = o.factor[1] = gamma / (dx * dy * dz);
+    o.factor[2] = 1.0 / (dx * dy * dz);
+    umin = (0.5 - double(L0 / 2)) * dx;
+    vmin = (0.5 - double(L1 / 2)) * dy;
+    wmin = (0.5 - double(L2 / 2)) * dz;
+    umin = umin + 0.0;
+    vmin = vmin + 0.0;
+    double oz = 0.0;
+    if (img) oz = oz + 2 * md->mn[2] + (md->mx[2] - md->mn[2]);
+    wmin = wmin + oz * gamma;
+  }
+  const double v = double(j) * dy + vmin, u = double(i) * dx + umin;
+  const double uu = u * u, vv = v * v;
+  const int k1 = min((int(blockIdx.z) + 1) * kPrimZ, L2);
+  for (int k = int(blockIdx.z) * kPrimZ; k < k1; ++k) {
+    const double w = double(k) * dz + wmin, ww = w * w;
+    const int64_t at = i + int64_t(L0) * (j + int64_t(L1) * k);
+    // r of xlafun2(u, v, w), (v, w, u) and (w, u, v)
+    const double s0 = uu + vv + ww;
+    double h = 0.0;
+    const double r0 = CHECK ? sqrt(s0) : fm_sqrt(s0, h);
+    if (o.F[0]) o.F[0][at] = xlafun2_tab<CHECK>(u, v, w, r0, tab) * o.factor[0];
+    if (o.F[1]) {
+      const double s = vv + ww + uu, r = CHECK ? sqrt(s) : fast_sqrt_near(s, r0, h);
+      o.F[1][at] = xlafun2_tab<CHECK>(v, w, u, r, tab) * o.factor[1];
+    }
+    if (o.F[2]) {
+      const double s = ww + uu + vv, r = CHECK ? sqrt(s) : fast_sqrt_near(s, r0, h);
+      o.F[2][at] = xlafun2_tab<CHECK>(w, u, v, r, tab) * o.factor[2];
     }
   }
 }
@@ -331,12 +401,74 @@ static void prim_mirrors(const GreenSpec& s, bool fast, int& mev, int& mod) {
   }
 }
 
+// Whether every coordinate i d + mn of the grid is far enough from the limits of
+// doubles, and from the axes, for k_prim3 without checks: magnitudes in
+// 1e+-60 (their products and squares in range) and at most one axis with
+// coordinates under 1e-5 of the largest radius, so that r + y and r - z, about
+// (x^2 + z^2) / (2 r) where they cancel, stay 1e-10 r or more, a million
+// roundings of r (or they are exact: x = z = 0 does not occur).
+static bool plain_grid(const int L[3], const double d[3], const double mn[3]) {
+  double near[3], far[3];
+  for (int a = 0; a < 3; ++a) {
+    near[a] = INFINITY;
+    far[a] = 0.0;
+    for (int i = 0; i < L[a]; ++i) {
+      const double x = std::fabs(double(i) * d[a] + mn[a]);
+      if (!(x < 1e60)) return false;
+      near[a] = std::min(near[a], x);
+      far[a] = std::max(far[a], x);
+    }
+  }
+  const double r = std::sqrt(far[0] * far[0] + far[1] * far[1] + far[2] * far[2]);
+  int small = 0;
+  for (int a = 0; a < 3; ++a) {
+    if (!(far[a] > 1e-60)) return false;
+    small += !(near[a] > 1e-5 * r && near[a] > 1e-60);
+  }
+  return small <= 1;
+}
+
+// Primitives on the whole grid at upstream's coordinates (k_prim3): of the
+// components with F[ic - 1] set, all of one offset-kind specification s but
+// for its component.
+static void launch_prim3(osc_ctx* c, const GreenSpec& s, double* const F[3]) {
+  const double dx = s.delta[0], dy = s.delta[1], dz = s.delta[2] * s.gamma;
+  Prim3 o{};
+  for (int a = 0; a < 3; ++a) {
+    o.F[a] = F[a];
+    o.factor[a] = a < 2 ? s.gamma / (dx * dy * dz) : 1.0 / (dx * dy * dz);
+  }
+  double umin = (0.5 - double(s.L[0] / 2)) * dx;
+  double vmin = (0.5 - double(s.L[1] / 2)) * dy;
+  double wmin = (0.5 - double(s.L[2] / 2)) * dz;
+  umin = umin + s.offset[0];
+  vmin = vmin + s.offset[1];
+  wmin = wmin + s.offset[2] * s.gamma;
+  const MeshDev* md = c->green_md;
+  OSC_REQUIRE(!md || (s.offset[0] == 0.0 && s.offset[1] == 0.0), OSC_ERR_ARG,
+              "device-side Green parameters: unsupported offset");
+  const dim3 g(unsigned((s.L[0] + 63) / 64), unsigned((s.L[1] + 3) / 4),
+               unsigned((s.L[2] + kPrimZ - 1) / kPrimZ));
+  const double d[3] = {dx, dy, dz}, mn[3] = {umin, vmin, wmin};
+  const bool plain = !md && plain_grid(s.L, d, mn);
+  launch(plain ? k_prim3<false> : k_prim3<true>, g, dim3(64, 4), 0, c->stream, o, s.L[0], s.L[1], s.L[2], dx, dy, dz, umin, vmin,
+         wmin, md, s.gamma, int(md && s.out_shift_z != 0),
+         static_cast<const FastMathTab*>(c->fast_tab));
+  OSC_HIP(hipGetLastError());
+}
+
 // primitive F of an offset-kind Green function (open_spacecharge_mod.f90:662-691).
 // lower_halves: the reader (the corner-difference x pass) loads only the
 // lower half, plus one plane, along mirrored y and z axes (unshifted z), so
 // the mirror images beyond that are not stored.
 static void build_offset_primitive(osc_ctx* c, const GreenSpec& s, double* F, bool fast,
                                    bool lower_halves = false, int zlo = 0, int zhi = -1) {
+  if (!fast && s.icomp >= 1) {
+    double* one[3] = {nullptr, nullptr, nullptr};
+    one[s.icomp - 1] = F;
+    launch_prim3(c, s, one);
+    return;
+  }
   if (zhi < 0 && zlo == 0) zhi = s.L[2] - 1;  // every plane
   const double dx = s.delta[0], dy = s.delta[1], dz = s.delta[2] * s.gamma;
   const double factor =
@@ -571,13 +703,42 @@ static void far_field_setup(osc_ctx* c, const GreenSpec& s, bool fast, CornerDif
 // a compile-time plan the z transform is left to conv_solve, which takes it
 // line by line inside the multiply (the array is z-real, GreenRef::zr).
 // Cached per precision under the full specification.
-template <typename T>
-GreenRef green_spectrum(osc_ctx* c, const GreenSpec& s, DevBuf& keepalive) {
-  const SpecDims d = SpecDims::of(s.L);
-  const int64_t N = int64_t(s.L[0]) * s.L[1] * s.L[2];
+static std::string green_key(const osc_ctx* c, const GreenSpec& s, bool fast) {
   std::string key(reinterpret_cast<const char*>(&s), sizeof(s));
   // spectra built with far-field cells are kept apart from exact ones
-  if (s.kind == GK_OFFSET && far_field_applies(c, s, sizeof(T) == 4)) key.push_back('F');
+  if (s.kind == GK_OFFSET && far_field_applies(c, s, fast)) key.push_back('F');
+  return key;
+}
+
+// The real primitives of s's three E components in one kernel, into F (three
+// arrays of the grid, component after component), if the FP64 spectra of all
+// three have to be built: green_spectrum takes them from there.
+template <typename T>
+bool green_primitives(osc_ctx* c, const GreenSpec& s, DevBuf& F) {
+  if (sizeof(T) == 4 || s.kind != GK_OFFSET) return false;
+  if (c->gcache.enable && !c->green_md)
+    for (int ic = 1; ic <= 3; ++ic) {
+      GreenSpec t = s;
+      t.icomp = ic;
+      auto it = c->gcache.map.find(green_key(c, t, false));
+      if (it != c->gcache.map.end() && it->second->f64.p) return false;
+    }
+  const int64_t N = int64_t(s.L[0]) * s.L[1] * s.L[2];
+  F = DevBuf(c->pool, sizeof(double) * 3 * N);
+  double* p[3];
+  for (int a = 0; a < 3; ++a) p[a] = F.as<double>() + a * N;
+  ProfScope ps(c, ST_GREEN_EVAL);
+  launch_prim3(c, s, p);
+  return true;
+}
+template bool green_primitives<double>(osc_ctx*, const GreenSpec&, DevBuf&);
+template bool green_primitives<float>(osc_ctx*, const GreenSpec&, DevBuf&);
+
+template <typename T>
+GreenRef green_spectrum(osc_ctx* c, const GreenSpec& s, DevBuf& keepalive, const double* prim) {
+  const SpecDims d = SpecDims::of(s.L);
+  const int64_t N = int64_t(s.L[0]) * s.L[1] * s.L[2];
+  const std::string key = green_key(c, s, sizeof(T) == 4);
   GreenCache& gc = c->gcache;
   GreenCache::Entry* hit = nullptr;
   // a captured solve builds its spectra on every replay (the spacing is only
@@ -596,7 +757,8 @@ GreenRef green_spectrum(osc_ctx* c, const GreenSpec& s, DevBuf& keepalive) {
     }
     ++gc.misses;
   }
-  DevBuf g(c->pool, sizeof(double) * N);
+  DevBuf g(c->pool, prim ? 0 : sizeof(double) * N);
+  double* F = g.as<double>();
   DevBuf sp(c->pool, sizeof(cpx<T>) * d.size());
   GreenRef ref{};
   GreenRef* zr = fft_has_plan(s.L[2]) ? &ref : nullptr;
@@ -604,21 +766,21 @@ GreenRef green_spectrum(osc_ctx* c, const GreenSpec& s, DevBuf& keepalive) {
   if (s.kind == GK_OFFSET && !fft_has_plan(s.L[0])) {
     // the x pass of a length without a plan differences the primitive on the
     // whole grid, without far-field cells and mirrored halves
-    {
+    if (!prim) {
       ProfScope ps(c, ST_GREEN_EVAL);
-      build_offset_primitive(c, s, g.as<double>(), fast);
+      build_offset_primitive(c, s, F, fast);
     }
     const CornerDiff cd{s.L[1], s.L[2], s.out_shift_z, s.zero_raw};
-    spectrum_forward_full<T>(c, g.as<const double>(), sp.as<cpx<T>>(), d, &cd, nullptr, zr);
+    spectrum_forward_full<T>(c, prim ? prim : F, sp.as<cpx<T>>(), d, &cd, nullptr, zr);
   } else if (s.kind == GK_OFFSET) {
     // the x pass takes the 8-corner difference of the primitive as it loads
     // its rows, so the difference array is never stored
     CornerDiff cd{s.L[1], s.L[2], s.out_shift_z, s.zero_raw};
     int zlo, zhi;
     far_field_setup(c, s, fast, cd, zlo, zhi);
-    if (zlo <= zhi) {
+    if (!prim && zlo <= zhi) {
       ProfScope ps(c, ST_GREEN_EVAL);
-      build_offset_primitive(c, s, g.as<double>(), fast, true, zlo, zhi);
+      build_offset_primitive(c, s, F, fast, true, zlo, zhi);
     }
     // the corner difference of a primitive that is even along an axis is odd
     // about L/2 - 1 there, and even where the primitive is odd
@@ -627,10 +789,10 @@ GreenRef green_spectrum(osc_ctx* c, const GreenSpec& s, DevBuf& keepalive) {
     int sym[3] = {0, 0, 0};
     if (mev >= 0) sym[mev] = -1;
     if (mod >= 0) sym[mod] = 1;
-    spectrum_forward_full<T>(c, g.as<const double>(), sp.as<cpx<T>>(), d, &cd, sym, zr);
+    spectrum_forward_full<T>(c, prim ? prim : F, sp.as<cpx<T>>(), d, &cd, sym, zr);
   } else {
-    build_green_real(c, s, g.as<double>(), fast);
-    spectrum_forward_full<T>(c, g.as<const double>(), sp.as<cpx<T>>(), d, nullptr, nullptr, zr);
+    build_green_real(c, s, F, fast);
+    spectrum_forward_full<T>(c, F, sp.as<cpx<T>>(), d, nullptr, nullptr, zr);
   }
   g.reset();
   ref.g = sp.p;
@@ -660,8 +822,8 @@ GreenRef green_spectrum(osc_ctx* c, const GreenSpec& s, DevBuf& keepalive) {
   }
   return ref;
 }
-template GreenRef green_spectrum<double>(osc_ctx*, const GreenSpec&, DevBuf&);
-template GreenRef green_spectrum<float>(osc_ctx*, const GreenSpec&, DevBuf&);
+template GreenRef green_spectrum<double>(osc_ctx*, const GreenSpec&, DevBuf&, const double*);
+template GreenRef green_spectrum<float>(osc_ctx*, const GreenSpec&, DevBuf&, const double*);
 
 // full upstream array F_s[g](k) = F_-[g](sigma_s k), sigma flipping axes with s=+1
 void half_to_upstream(osc_ctx* c, const cpx<double>* spec_dev, const SpecDims& d, const int s[3],

@@ -255,6 +255,7 @@ struct osc_ctx {
   bool kept_ok = false;
   std::unique_ptr<osc::HostRing> ring;  // pageable host transfers (created on first use)
   void* counters = nullptr;  // small device scratch for counters (persistent)
+  void* fast_tab = nullptr;  // the FastMathTab of fast_math.h, behind the counters
   osc::MeshDev* mesh_host = nullptr;  // pinned copy of the device mesh
   hipEvent_t mesh_ev = nullptr;        // recorded after the copy is queued
   // pinned copies of the deposit's and the query's content hashes (in the
@@ -415,7 +416,12 @@ void pipe_spectrum(osc_ctx* c, const GreenSpec& s, const SpecDims& d, cpx<double
 // spectrum of a Green function in precision T (z-real when the z length has a
 // compile-time plan); cached by spec
 template <typename T>
-GreenRef green_spectrum(osc_ctx* c, const GreenSpec& s, DevBuf& keepalive);
+GreenRef green_spectrum(osc_ctx* c, const GreenSpec& s, DevBuf& keepalive,
+                        const double* prim = nullptr);
+// the primitives of s's three E components for green_spectrum's prim (one
+// array of the grid each), where that pays; false: none
+template <typename T>
+bool green_primitives(osc_ctx* c, const GreenSpec& s, DevBuf& F);
 // forward R2C of a real (L0,L1,L2) FP64 array into a half spectrum of precision T
 // (with cd: g is a primitive and the x pass takes its corner difference;
 // sym: per-axis mirror symmetry of that difference, 0 / +1 even / -1 odd;

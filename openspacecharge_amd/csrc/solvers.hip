@@ -91,6 +91,21 @@ struct Specs {
     }
     return green_spectrum<T>(c, s, keep[slot]);
   }
+  // the three E components of the offset-kind specification s, in slots
+  // slot .. slot + 2
+  void get3(osc_ctx* c, GreenSpec s, size_t slot, GreenRef out[3]) {
+    if (!pinned) {
+      pinned = c;
+      c->gcache.pin();
+    }
+    DevBuf F;
+    const int64_t N = int64_t(s.L[0]) * s.L[1] * s.L[2];
+    const double* p = green_primitives<T>(c, s, F) ? F.as<const double>() : nullptr;
+    for (int a = 0; a < 3; ++a) {
+      s.icomp = a + 1;
+      out[a] = green_spectrum<T>(c, s, keep[slot + a], p ? p + a * N : nullptr);
+    }
+  }
 };
 
 void mesh_n(const osc_mesh& m, int n[3]) {
@@ -114,10 +129,11 @@ void solver2_t(osc_ctx* c, const int n[3], const double* rho, double gamma, cons
   Specs<T> sp(4);
   std::vector<OutSpec> outs;
   if (phi) outs.push_back(out1(sp.get(c, offset_spec(L, delta, gamma, 0, off, 0), 0), s1, phi));
-  if (ef)
-    for (int ic = 1; ic <= 3; ++ic)
-      outs.push_back(out1(sp.get(c, offset_spec(L, delta, gamma, ic, off, 0), ic), s1,
-                          ef + (ic - 1) * nt));
+  if (ef) {
+    GreenRef G[3];
+    sp.get3(c, offset_spec(L, delta, gamma, 1, off, 0), 1, G);
+    for (int ic = 0; ic < 3; ++ic) outs.push_back(out1(G[ic], s1, ef + ic * nt));
+  }
   if (!outs.empty()) conv_solve<T>(c, rho, n, d, win, outs);
 }
 
@@ -142,8 +158,7 @@ void sc3d_t(osc_ctx* c, const osc_mesh& m, const double* rho, const double* offs
   }
   Specs<T> sp(6);
   GreenRef G[3];
-  for (int ic = 1; ic <= 3; ++ic)
-    G[ic - 1] = sp.get(c, offset_spec(L, m.delta, m.gamma, ic, off, 0), ic - 1);
+  sp.get3(c, offset_spec(L, m.delta, m.gamma, 1, off, 0), 0, G);
   std::vector<OutSpec> outs;
   if (!at_cathode) {
     for (int ic = 0; ic < 3; ++ic) outs.push_back(out1(G[ic], s1, ef + ic * nt));
@@ -156,8 +171,7 @@ void sc3d_t(osc_ctx* c, const osc_mesh& m, const double* rho, const double* offs
     double offi[3] = {off[0], off[1], off[2]};
     offi[2] = offi[2] + 2 * m.min[2] + (m.max[2] - m.min[2]);
     GreenRef H[3];
-    for (int ic = 1; ic <= 3; ++ic)
-      H[ic - 1] = sp.get(c, offset_spec(L, m.delta, m.gamma, ic, offi, n[2] - 1), 3 + ic - 1);
+    sp.get3(c, offset_spec(L, m.delta, m.gamma, 1, offi, n[2] - 1), 3, H);
     for (int ic = 0; ic < 3; ++ic) outs.push_back(out2(G[ic], H[ic], -1.0, 4, s1, ef + ic * nt));
     if (calc_b) {
       // Bx = -(beta/c)(Ey_free - Ey_img), By = (beta/c)(Ex_free - Ex_img) (:459-460, 483-484)
