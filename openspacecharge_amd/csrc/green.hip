@@ -186,32 +186,119 @@ __global__ void __launch_bounds__(64)
 }
 
 // legacy loops: osc_getgrnfree (core:476-493), osc_getgrnimageshift
-// (core:1157-1174), osc_getgrnimageconvcorr (core:1207-1226)
-__global__ void k_green_legacy(double* __restrict__ G, GreenSpec s) {
-  const int L0 = s.L[0], L1 = s.L[1], L2 = s.L[2];
-  const int64_t N = int64_t(L0) * L1 * L2;
-  const double dx = s.delta[0], dy = s.delta[1], dz = s.delta[2];
+// (core:1157-1174), osc_getgrnimageconvcorr (core:1207-1226): the cell of
+// index (ii, jj, kq) at
+__host__ __device__ __forceinline__ double legacy_u(const GreenSpec& s, int ii) {
+  return double(s.lo[0] + (ii + s.shift[0]) % s.L[0]) * s.delta[0];
+}
+__host__ __device__ __forceinline__ double legacy_v(const GreenSpec& s, int jj) {
+  return double(s.lo[1] + (jj + s.shift[1]) % s.L[1]) * s.delta[1];
+}
+__host__ __device__ __forceinline__ double legacy_w(const GreenSpec& s, int kq) {
+  int kk = (kq - s.out_shift_z) % s.L[2];
+  if (kk < 0) kk += s.L[2];
+  const double dz = s.delta[2];
+  if (s.kind == GK_IMG_CONVCORR)
+    return (s.lo[2] + kk) * dz + 2.0 * s.umin[2] - 2.0 * s.nlo3 * s.delta[2];
+  double w = (s.lo[2] + (kk + s.shift[2]) % s.L[2]) * dz;
+  if (s.kind == GK_IMG_SHIFT) w = w + s.zshft;
+  return w;
+}
+
+// igfflag 0: 1/r at the cell (E components are 0: never requested upstream)
+__global__ void k_green_coulomb(double* __restrict__ G, GreenSpec s) {
+  const int64_t N = int64_t(s.L[0]) * s.L[1] * s.L[2];
   for (int64_t idx = blockIdx.x * int64_t(blockDim.x) + threadIdx.x; idx < N;
        idx += int64_t(gridDim.x) * blockDim.x) {
-    const int ii = int(idx % L0);
-    const int jj = int((idx / L0) % L1);
-    const int kq = int(idx / (int64_t(L0) * L1));
-    int kk = (kq - s.out_shift_z) % L2;
-    if (kk < 0) kk += L2;
-    double w;
-    if (s.kind == GK_IMG_CONVCORR) {
-      const int kp = s.lo[2] + kk;
-      w = kp * dz + 2.0 * s.umin[2] - 2.0 * s.nlo3 * s.delta[2];
-    } else {
-      const int kp = s.lo[2] + (kk + s.shift[2]) % L2;
-      w = kp * dz;
-      if (s.kind == GK_IMG_SHIFT) w = w + s.zshft;
+    const double u = legacy_u(s, int(idx % s.L[0])), v = legacy_v(s, int((idx / s.L[0]) % s.L[1]));
+    const double w = legacy_w(s, int(idx / (int64_t(s.L[0]) * s.L[1])));
+    G[idx] = s.icomp == 0 ? coulombfun(u, v, w, s.gamma) : 0.0;
+  }
+}
+
+// Integrated legacy Green functions: per cell the 8-corner sums of xlafun,
+// ylafun and zlafun (core:243-428; G[a] null: not wanted), or with PHI of
+// lafun (core:205-238) into G[0].  Bound by the FP64 instructions of the
+// corners' logarithms and arc tangents.  The three components have one root
+// and three logarithms between them, so one thread forms them together with
+// the functions of fast_math.h; it marches `nk` planes, and where the upper
+// corners of a cell have the bits of the next one's lower corners (both are
+// rounded from their own cell's centre, about half of them agree) they are
+// not evaluated again.  Upstream's terms z - x atan(z/x) of xlafun (and their
+// like) do not depend on the component's second coordinate: the corner sum
+// cancels them, and they are left out.  128^3 cells, three components: 0.094 ms,
+// where a launch per component, every corner and term on its own in
+// the device library's functions, took 0.64 ms.
+struct Legacy3 {
+  double* G[3];
+  double div[3];
+};
+template <bool CHECK>
+__device__ __forceinline__ double legacy_term(double a, double arg, double log_arg) {
+  // a log(arg), with the guards of upstream's E functions (core:386-387)
+  return CHECK && arg == 0.0 ? 0.0 : a * log_arg;
+}
+template <bool CHECK, bool PHI>
+__device__ __forceinline__ void legacy_corner(double x, double y, double z, const FastMathTab& tab,
+                                              double f[PHI ? 1 : 3]) {
+  const double s = x * x + y * y + z * z;
+  double h = 0.0;
+  const double r = CHECK ? sqrt(s) : fm_sqrt(s, h);
+  const double ax = fast_atan<CHECK>(y * z, x * r, tab), lx = fast_log<CHECK>(x + r, tab);
+  const double ay = fast_atan<CHECK>(z * x, y * r, tab), ly = fast_log<CHECK>(y + r, tab);
+  const double az = fast_atan<CHECK>(x * y, z * r, tab), lz = fast_log<CHECK>(z + r, tab);
+  if constexpr (PHI) {
+    f[0] = -(0.5 * (z * z) * az) - 0.5 * (y * y) * ay - 0.5 * (x * x) * ax + y * z * lx +
+           x * z * ly + x * y * lz;
+  } else {
+    f[0] = x * ax - legacy_term<CHECK>(z, y + r, ly) - legacy_term<CHECK>(y, z + r, lz);
+    f[1] = y * ay - legacy_term<CHECK>(x, z + r, lz) - legacy_term<CHECK>(z, x + r, lx);
+    f[2] = z * az - legacy_term<CHECK>(y, x + r, lx) - legacy_term<CHECK>(x, y + r, ly);
+  }
+}
+template <bool CHECK, bool PHI>
+__global__ void __launch_bounds__(256)
+    k_green_legacy(Legacy3 o, GreenSpec s, int nk, const FastMathTab* __restrict__ table) {
+  constexpr int NC = PHI ? 1 : 3;
+  __shared__ FastMathTab tab;
+  {
+    const unsigned* src = reinterpret_cast<const unsigned*>(table);
+    unsigned* dst = reinterpret_cast<unsigned*>(&tab);
+    for (int t = threadIdx.y * 64 + threadIdx.x; t < int(sizeof(FastMathTab) / 4); t += 256) dst[t] = src[t];
+  }
+  __syncthreads();
+  const int i = blockIdx.x * 64 + threadIdx.x, j = blockIdx.y * 4 + threadIdx.y;
+  if (i >= s.L[0] || j >= s.L[1]) return;
+  const double u = legacy_u(s, i), v = legacy_v(s, j);
+  const double x1 = u - 0.5 * s.delta[0], x2 = u + 0.5 * s.delta[0];
+  const double y1 = v - 0.5 * s.delta[1], y2 = v + 0.5 * s.delta[1];
+  // corners (x1,y1), (x2,y1), (x1,y2), (x2,y2) at the lower and upper z
+  double lo[4][NC], up[4][NC];
+  auto plane = [&](double z, double (&f)[4][NC]) {
+    legacy_corner<CHECK, PHI>(x1, y1, z, tab, f[0]);
+    legacy_corner<CHECK, PHI>(x2, y1, z, tab, f[1]);
+    legacy_corner<CHECK, PHI>(x1, y2, z, tab, f[2]);
+    legacy_corner<CHECK, PHI>(x2, y2, z, tab, f[3]);
+  };
+  const int k0 = int(blockIdx.z) * nk, k1 = min(k0 + nk, s.L[2]);
+  double zl = 0.0;
+  for (int k = k0; k < k1; ++k) {
+    const double w = legacy_w(s, k);
+    const double z1 = (w - 0.5 * s.delta[2]) * s.gamma, z2 = (w + 0.5 * s.delta[2]) * s.gamma;
+    if (k == k0 || z1 != zl) plane(z1, lo);
+    plane(z2, up);
+    const int64_t at = i + int64_t(s.L[0]) * (j + int64_t(s.L[1]) * k);
+    const bool self = !PHI && x1 < 0.0 && x2 > 0.0 && y1 < 0.0 && y2 > 0.0 && z1 < 0.0 && z2 > 0.0;
+#pragma unroll
+    for (int a = 0; a < NC; ++a) {
+      const double g = up[3][a] - up[2][a] - up[1][a] - lo[3][a] - lo[0][a] + up[0][a] + lo[2][a] + lo[1][a];
+      if (o.G[a]) o.G[a][at] = self ? 0.0 / o.div[a] : g / o.div[a];
     }
-    const int jp = s.lo[1] + (jj + s.shift[1]) % L1;
-    const double v = jp * dy;
-    const int ip = s.lo[0] + (ii + s.shift[0]) % L0;
-    const double u = ip * dx;
-    G[idx] = igf_legacy(s.igf, s.icomp, u, v, w, s.gamma, dx, dy, dz);
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+      for (int a = 0; a < NC; ++a) lo[q][a] = up[q][a];
+    zl = z2;
   }
 }
 
@@ -401,19 +488,20 @@ static void prim_mirrors(const GreenSpec& s, bool fast, int& mev, int& mod) {
   }
 }
 
-// Whether every coordinate i d + mn of the grid is far enough from the limits of
-// doubles, and from the axes, for k_prim3 without checks: magnitudes in
-// 1e+-60 (their products and squares in range) and at most one axis with
-// coordinates under 1e-5 of the largest radius, so that r + y and r - z, about
-// (x^2 + z^2) / (2 r) where they cancel, stay 1e-10 r or more, a million
-// roundings of r (or they are exact: x = z = 0 does not occur).
-static bool plain_grid(const int L[3], const double d[3], const double mn[3]) {
+// Whether every coordinate (n[a] of them along axis a, at(a, i)) is far enough
+// from the limits of doubles, and from the axes, for the kernels without checks:
+// magnitudes in 1e+-60 (their products and squares in range) and at most one
+// axis with coordinates under 1e-5 of the largest radius, so that r + y and
+// r - z, about (x^2 + z^2) / (2 r) where they cancel, stay 1e-10 r or more, a
+// million roundings of r (or they are exact: x = z = 0 does not occur).
+template <typename At>
+static bool plain_grid(const int n[3], At at) {
   double near[3], far[3];
   for (int a = 0; a < 3; ++a) {
     near[a] = INFINITY;
     far[a] = 0.0;
-    for (int i = 0; i < L[a]; ++i) {
-      const double x = std::fabs(double(i) * d[a] + mn[a]);
+    for (int i = 0; i < n[a]; ++i) {
+      const double x = std::fabs(at(a, i));
       if (!(x < 1e60)) return false;
       near[a] = std::min(near[a], x);
       far[a] = std::max(far[a], x);
@@ -426,6 +514,34 @@ static bool plain_grid(const int L[3], const double d[3], const double mn[3]) {
     small += !(near[a] > 1e-5 * r && near[a] > 1e-60);
   }
   return small <= 1;
+}
+
+// The integrated legacy Green functions of the components with G[ic - 1] set
+// (phi: the potential's into G[0]) of one legacy-kind specification s
+static void launch_legacy(osc_ctx* c, const GreenSpec& s, bool phi, double* const G[3]) {
+  Legacy3 o{};
+  const double dx = s.delta[0], dy = s.delta[1], dz = s.delta[2];
+  for (int a = 0; a < 3; ++a) {
+    o.G[a] = G[a];
+    // icomp past the components is answered as the third without its gamma
+    const bool third = a == 2 && (s.icomp < 0 || s.icomp > 3);
+    o.div[a] = (phi || a == 2) && !third ? dx * dy * dz * s.gamma : dx * dy * dz;
+  }
+  const int n[3] = {2 * s.L[0], 2 * s.L[1], 2 * s.L[2]};
+  const bool plain = plain_grid(n, [&](int a, int i) {
+    const double at = a == 0 ? legacy_u(s, i / 2) : (a == 1 ? legacy_v(s, i / 2) : legacy_w(s, i / 2));
+    const double e = (i & 1) ? at + 0.5 * s.delta[a] : at - 0.5 * s.delta[a];
+    return a == 2 ? e * s.gamma : e;
+  });
+  // planes per thread: eight where that still gives every CU four workgroups
+  const unsigned gx = unsigned((s.L[0] + 63) / 64), gy = unsigned((s.L[1] + 3) / 4);
+  int nk = 8;
+  while (nk > 1 && int64_t(gx) * gy * ((s.L[2] + nk - 1) / nk) < 1024) nk /= 2;
+  auto kern = phi ? (plain ? k_green_legacy<false, true> : k_green_legacy<true, true>)
+                  : (plain ? k_green_legacy<false, false> : k_green_legacy<true, false>);
+  launch(kern, dim3(gx, gy, unsigned((s.L[2] + nk - 1) / nk)), dim3(64, 4), 0, c->stream, o, s, nk,
+         static_cast<const FastMathTab*>(c->fast_tab));
+  OSC_HIP(hipGetLastError());
 }
 
 // Primitives on the whole grid at upstream's coordinates (k_prim3): of the
@@ -450,7 +566,7 @@ static void launch_prim3(osc_ctx* c, const GreenSpec& s, double* const F[3]) {
   const dim3 g(unsigned((s.L[0] + 63) / 64), unsigned((s.L[1] + 3) / 4),
                unsigned((s.L[2] + kPrimZ - 1) / kPrimZ));
   const double d[3] = {dx, dy, dz}, mn[3] = {umin, vmin, wmin};
-  const bool plain = !md && plain_grid(s.L, d, mn);
+  const bool plain = !md && plain_grid(s.L, [&](int a, int i) { return double(i) * d[a] + mn[a]; });
   launch(plain ? k_prim3<false> : k_prim3<true>, g, dim3(64, 4), 0, c->stream, o, s.L[0], s.L[1], s.L[2], dx, dy, dz, umin, vmin,
          wmin, md, s.gamma, int(md && s.out_shift_z != 0),
          static_cast<const FastMathTab*>(c->fast_tab));
@@ -584,8 +700,12 @@ void build_green_real(osc_ctx* c, const GreenSpec& s, double* g, bool fast) {
     const dim3 g3(unsigned((s.L[0] + 63) / 64), unsigned((s.L[1] + 3) / 4), unsigned(s.L[2]));
     launch(k_green_pipe, g3, dim3(256), 0, c->stream, g, s, cu, rows);
     OSC_HIP(hipGetLastError());
+  } else if (s.igf != 0) {
+    double* G[3] = {nullptr, nullptr, nullptr};
+    G[s.icomp >= 0 && s.icomp <= 2 ? std::max(0, s.icomp - 1) : 2] = g;
+    launch_legacy(c, s, s.icomp == 0, G);
   } else {
-    launch(k_green_legacy, dim3(nblk(N)), dim3(kThreads), 0, c->stream, g, s);
+    launch(k_green_coulomb, dim3(nblk(N)), dim3(kThreads), 0, c->stream, g, s);
     OSC_HIP(hipGetLastError());
   }
 }
@@ -710,25 +830,27 @@ static std::string green_key(const osc_ctx* c, const GreenSpec& s, bool fast) {
   return key;
 }
 
-// The real primitives of s's three E components in one kernel, into F (three
-// arrays of the grid, component after component), if the FP64 spectra of all
-// three have to be built: green_spectrum takes them from there.
+// The real arrays of s's three E components in one kernel, into F (three
+// arrays of the grid, component after component), if the spectra of all three
+// have to be built: the primitives of an FP64 offset-kind specification, the
+// Green functions of a legacy-kind one.  green_spectrum takes them from there.
 template <typename T>
 bool green_primitives(osc_ctx* c, const GreenSpec& s, DevBuf& F) {
-  if (sizeof(T) == 4 || s.kind != GK_OFFSET) return false;
+  if (s.kind == GK_OFFSET ? sizeof(T) == 4 : s.igf == 0) return false;
   if (c->gcache.enable && !c->green_md)
     for (int ic = 1; ic <= 3; ++ic) {
       GreenSpec t = s;
       t.icomp = ic;
-      auto it = c->gcache.map.find(green_key(c, t, false));
-      if (it != c->gcache.map.end() && it->second->f64.p) return false;
+      auto it = c->gcache.map.find(green_key(c, t, sizeof(T) == 4));
+      if (it != c->gcache.map.end() && (sizeof(T) == 4 ? it->second->f32 : it->second->f64).p) return false;
     }
   const int64_t N = int64_t(s.L[0]) * s.L[1] * s.L[2];
   F = DevBuf(c->pool, sizeof(double) * 3 * N);
   double* p[3];
   for (int a = 0; a < 3; ++a) p[a] = F.as<double>() + a * N;
   ProfScope ps(c, ST_GREEN_EVAL);
-  launch_prim3(c, s, p);
+  if (s.kind == GK_OFFSET) launch_prim3(c, s, p);
+  else launch_legacy(c, s, false, p);
   return true;
 }
 template bool green_primitives<double>(osc_ctx*, const GreenSpec&, DevBuf&);
@@ -791,8 +913,8 @@ GreenRef green_spectrum(osc_ctx* c, const GreenSpec& s, DevBuf& keepalive, const
     if (mod >= 0) sym[mod] = 1;
     spectrum_forward_full<T>(c, prim ? prim : F, sp.as<cpx<T>>(), d, &cd, sym, zr);
   } else {
-    build_green_real(c, s, F, fast);
-    spectrum_forward_full<T>(c, F, sp.as<cpx<T>>(), d, nullptr, nullptr, zr);
+    if (!prim) build_green_real(c, s, F, fast);
+    spectrum_forward_full<T>(c, prim ? prim : F, sp.as<cpx<T>>(), d, nullptr, nullptr, zr);
   }
   g.reset();
   ref.g = sp.p;

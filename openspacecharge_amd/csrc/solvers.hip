@@ -91,7 +91,7 @@ struct Specs {
     }
     return green_spectrum<T>(c, s, keep[slot]);
   }
-  // the three E components of the offset-kind specification s, in slots
+  // the three E components of the offset- or legacy-kind specification s, in slots
   // slot .. slot + 2
   void get3(osc_ctx* c, GreenSpec s, size_t slot, GreenRef out[3]) {
     if (!pinned) {
@@ -210,10 +210,9 @@ int legacy_free_t(osc_ctx* c, const osc_mesh& m, const double* rho, int direct, 
     fd_gradient(c, phi, n, m.delta, m.gamma, ef);
     bfield_core(c, ef, nt, m.gamma, bf);
   } else {
-    for (int ic = 1; ic <= 3; ++ic) {
-      GreenSpec s = legacy_spec(m.nlo, m.nhi, m.npad, m.delta, m.gamma, ic, igf);
-      outs.push_back(out1(sp.get(c, s, ic - 1), s1, ef + (ic - 1) * nt));
-    }
+    GreenRef G[3];
+    sp.get3(c, legacy_spec(m.nlo, m.nhi, m.npad, m.delta, m.gamma, 1, igf), 0, G);
+    for (int ic = 0; ic < 3; ++ic) outs.push_back(out1(G[ic], s1, ef + ic * nt));
     set_b(outs[0], bf + nt, 1, 1.0, beta0, kClightDp);   // By =  Ex*beta0/c
     set_b(outs[1], bf, 1, -1.0, beta0, kClightDp);       // Bx = -Ey*beta0/c
     conv_solve<T>(c, rho, n, d, win, outs);
@@ -270,10 +269,8 @@ int cathode_t(osc_ctx* c, const osc_mesh& m, double* rho, int direct, int igf, i
   } else {
     GreenRef G[3];
     GreenRef H[3];
-    for (int ic = 1; ic <= 3; ++ic) {
-      G[ic - 1] = sp.get(c, legacy_spec(m.nlo, m.nhi, m.npad, m.delta, m.gamma, ic, igf), ic - 1);
-      H[ic - 1] = sp.get(c, image_spec(ic), 3 + ic - 1);
-    }
+    sp.get3(c, legacy_spec(m.nlo, m.nhi, m.npad, m.delta, m.gamma, 1, igf), 0, G);
+    sp.get3(c, image_spec(1), 3, H);
     for (int ic = 0; ic < 3; ++ic) outs.push_back(out2(G[ic], H[ic], -1.0, 4, s1, ef + ic * nt));
     OutSpec bx = out2(G[1], H[1], 1.0, 4, s1, nullptr);
     set_b(bx, bf, 1, -1.0, beta0, kClightDp);  // -(Ey + 2 Ey_img)*beta0/c
