@@ -58,8 +58,10 @@ void xr2c_t(const double* in, cpx<T>* out, const R2CIO& a, const cpx<T>* tw, hip
 template <int L>
 void xc2r_t(const cpx<T>* in, const C2RIO<T>& a, int nout, const cpx<T>* tw, hipStream_t s) {
   constexpr int BX = XGeo<T, L>::BX, NT = XGeo<T, L>::NT;
-  dim3 g = grid3(cdiv(cdiv(a.nrows, 2), BX), nout, 1);
-  launch((k_xc2r<T, L>), g, dim3(NT), 0, s, in, a, tw);
+  if (a.npair > 0)
+    launch((k_xc2r<T, L, true>), grid3(cdiv(a.nrows, BX), a.npair, 1), dim3(NT), 0, s, in, a, tw);
+  else
+    launch((k_xc2r<T, L, false>), grid3(cdiv(cdiv(a.nrows, 2), BX), nout, 1), dim3(NT), 0, s, in, a, tw);
 }
 // k_zconv's per-thread byte offsets (line b < BX, position t < TPL of a
 // column block) must fit in 32 bits
@@ -79,8 +81,13 @@ void zinv_t(const cpx<T>* rho, cpx<T>* out, const ZinvIO<T>& a, int Ly, int nout
   if (a.zreal && a.zin > 0) {
     OSC_REQUIRE(zconv_fits_t<L>(a), OSC_ERR_ARG, "fused z convolution: offsets exceed 32 bits");
     const int nxb = int(cdiv(a.nb, ZGeo<T, L>::BX));
-    launch((k_zconv<T, L>), grid3(int64_t(nxb) * Ly, 1, 1), dim3(ZGeo<T, L>::NT), 0,
-                       s, rho, out, a, tw, nxb);
+    ZinvIO<T> b = a;
+    // phases that add into one output follow each other
+    const int launches = a.nphase == 2 && a.acc ? 2 : 1;
+    b.nphase = a.nphase / launches;
+    const dim3 g1 = grid3(int64_t(nxb) * Ly * b.nphase, 1, 1);
+    for (b.phase0 = 0; b.phase0 < launches; ++b.phase0)
+      launch((k_zconv<T, L>), g1, dim3(ZGeo<T, L>::NT), 0, s, rho, out, b, tw, nxb);
   } else if (a.zreal) {
     const int nxb = int(cdiv(a.nb, ZGeo<T, L>::BX));
     const int64_t units = int64_t(nxb) * Ly;
@@ -156,6 +163,7 @@ void launch_xc2r<T>(int L, const cpx<T>* in, const C2RIO<T>& a, int nout, const 
     OSC_FOR_EACH_L(OSC_CASE)
 #undef OSC_CASE
     default:
+      OSC_REQUIRE(a.npair == 0, OSC_ERR_FFT_LENGTH, "pairs of parts need a planned length");
       gen_xc2r<T>(L, in, a, nout, tw, s);
   }
   OSC_HIP(hipGetLastError());

@@ -51,10 +51,11 @@ struct R2CIO {
 // Epilogue of the inverse x pass for one output field: e = s1*val is stored
 // to dst1 (if any); dst2 (if any) receives bmode 0: s2*e, or
 // bmode 1: ((sgn*e)*beta)/c   (the two B-field formulas of the upstream code).
+// Of a pair of parts (C2RIO::npair) val is the first plus sb times the second.
 struct Epilogue {
   double* dst1;
   double* dst2;
-  double s1, s2, beta, c;
+  double s1, s2, beta, c, sb;
   int bmode, pad_;
 };
 
@@ -68,7 +69,11 @@ struct C2RIO {
   int64_t in_sy, in_sz, in_so;
   int64_t out_sy, out_sz;
   int64_t nrows;
-  int ny_rows, w0, n_out, pad_;
+  int ny_rows, w0, n_out;
+  // > 0: the spectra are npair first parts and then their npair second parts;
+  // a complex line carries a row of both, and pair o has the epilogues ep[2 o]
+  // and ep[2 o + 1] (no destination: none)
+  int npair;
   Epilogue ep[kMaxOut];
 };
 
@@ -96,11 +101,16 @@ struct ZinvIO {
   // and y only; its z transform is taken per line inside the multiply
   // (k_zinv_g)
   int zreal;
-  // > 0 (with zreal, every output one term with mir == 0): rho_hat has had
-  // its x and y passes only, with zin stored z planes (the rest zero); its z
-  // pass is taken inside the multiply, once per column for all outputs
-  // (k_zconv)
-  int zin;
+  // > 0 (with zreal): rho_hat has had its x and y passes only, with zin stored
+  // z planes (the rest zero); its z pass is taken inside the multiply, once
+  // per column and phase (k_zconv).  Term t of an output belongs to phase t:
+  // one phase, every output one term without mirrors; or two, the second's
+  // terms mirrored in z.
+  int zin, nphase;
+  int phase0;  // k_zconv: the first of the nphase phases of this launch
+  // two phases: the second's result is added to the first's output (acc, a
+  // launch for each), or stored as output o + nout
+  int acc;
   OutTerms<T> out[kMaxOut];
 };
 
@@ -410,7 +420,9 @@ __device__ __forceinline__ void epi_store(const Epilogue& e, int64_t off, double
   if (e.dst2) e.dst2[off] = e.bmode == 0 ? e.s2 * v : ((e.s2 * v) * e.beta) / e.c;
 }
 
-template <typename T, int L>
+// PAIR: a line is a row of the two parts of pair o (C2RIO::npair), whose sums
+// and differences the epilogues take: each part is transformed once for both.
+template <typename T, int L, bool PAIR>
 __global__ void __launch_bounds__((XGeo<T, L>::NT))
     k_xc2r(const cpx<T>* __restrict__ in, C2RIO<T> a, const cpx<T>* __restrict__ tw) {
   constexpr int BX = XGeo<T, L>::BX;
@@ -418,6 +430,24 @@ __global__ void __launch_bounds__((XGeo<T, L>::NT))
   __shared__ cpx<T> lds[F::LDS];
   F f;
   const int o = blockIdx.y;
+  if constexpr (PAIR) {
+    const int64_t r = int64_t(blockIdx.x) * BX + f.b;
+    const bool ok = r < a.nrows;
+    const RowPair rp = row_pair(r, a.ny_rows);
+    const cpx<T>* pa = in + o * a.in_so + (ok ? int64_t(rp.ya) * a.in_sy + int64_t(rp.za) * a.in_sz : 0);
+    const cpx<T>* pb = pa + a.npair * a.in_so;
+    f.load([&](int, int p) { return ok ? c2r_pack(pa, pb, true, p, L) : mk<T>(0, 0); });
+    f.run(lds, tw);
+    const int64_t off = int64_t(rp.ya) * a.out_sy + int64_t(rp.za) * a.out_sz;
+    f.store([&](int, int p, cpx<T> v) {
+      const int x = p - a.w0;
+      if (!ok || x < 0 || x >= a.n_out) return;
+      const double va = double(v.x), vb = double(v.y);
+      epi_store(a.ep[2 * o], off + x, va + a.ep[2 * o].sb * vb);
+      epi_store(a.ep[2 * o + 1], off + x, va + a.ep[2 * o + 1].sb * vb);
+    });
+    return;
+  }
   const int64_t ra = 2 * (int64_t(blockIdx.x) * BX + f.b), rb = ra + 1;
   const bool oka = ra < a.nrows, okb = rb < a.nrows;
   const RowPair rp = row_pair(ra, a.ny_rows);
@@ -605,10 +635,19 @@ __device__ __forceinline__ const cpx<T>& at_off(const char* base, uint32_t vo) {
 
 // The forward z pass of rho_hat and, for every output, the z transform of its
 // z-real Green line, the multiply and the inverse z pass, per (kx, ky) column:
-// rho_hat's column (ZinvIO::zin stored planes) is read once and its spectrum
-// kept in registers across the outputs, and the forward and Green spectra
-// meet in registers (same tile, same element positions).  Every output is a
-// single term without mirrors.  One workgroup per (x block, ky) unit.
+// rho_hat's column (ZinvIO::zin stored planes) is read once per phase and its
+// spectrum kept in registers across the outputs, and the forward and Green
+// spectra meet in registers (same tile, same element positions).  The second
+// phase (image charges) reads the column mirrored, element p from L - p, which
+// is the mirror of its spectrum.  One workgroup per (x block, ky) unit and phase.
+//
+// Two phases instead of one transform of each output's sum over full spectra
+// (k_zinv): at 128x128x256 in FP64 the z passes of the six Green functions and
+// rho (272 MB read and written each) and the sums took 2.31 ms; this kernel
+// takes 0.82 ms (2.7 GB, 3.3 TB/s), the inverse y pass carrying six parts
+// instead of five sums.  Keeping both phases' spectra, or the loop over them,
+// in one workgroup needs 157 VGPRs (three waves per SIMD); one output per
+// workgroup, for small meshes, changes nothing (32^3 .. 64x64x128).
 //
 // Addressing: element (line b, position t + c) of a column block is at a
 // uniform base (block, c) plus the per-thread byte offset of (b, t), computed
@@ -619,6 +658,7 @@ __device__ __forceinline__ const cpx<T>& at_off(const char* base, uint32_t vo) {
 // output positions are its input positions), with or without reading the
 // next Green line during the inverse transform, needs about 150 VGPRs
 // (3 waves per SIMD instead of 4) and is 5-10 % slower.
+//
 template <typename T, int L>
 __global__ void __launch_bounds__((ZGeo<T, L>::NT))
     k_zconv(const cpx<T>* __restrict__ rho, cpx<T>* __restrict__ out, ZinvIO<T> a,
@@ -630,8 +670,10 @@ __global__ void __launch_bounds__((ZGeo<T, L>::NT))
   constexpr int64_t CB = sizeof(cpx<T>);
   static_assert(FF::LDS == FI::LDS, "forward and inverse tiles differ");
   __shared__ cpx<T> lds[FF::LDS];
+  // the phases of a column are consecutive logical workgroups (one L2)
   const int lw = int(xcd_block(blockIdx.x, gridDim.x));
-  const int xb = lw % nxb, ky = lw / nxb;
+  const int ph = a.phase0 + lw % a.nphase, unit = lw / a.nphase;
+  const int xb = unit % nxb, ky = unit / nxb;
   FF fr;
   const int b = fr.b, t = fr.t;
   const bool ok = xb * BX + b < a.nb;
@@ -641,13 +683,22 @@ __global__ void __launch_bounds__((ZGeo<T, L>::NT))
   const uint32_t vm = uint32_t((b + (TPL - 1 - t) * a.sz) * CB);
   const uint32_t vout = uint32_t((b + t * a.o_sz) * CB);
   const char* rb = reinterpret_cast<const char*>(rho + col0);
-  fr.load_c([&](int c) {
-    return (ok && t + c < a.zin) ? at_off<T>(rb + c * a.sz * CB, vo) : mk<T>(0, 0);
-  });
+  if (ph) {
+    // element p from L-p = (L+1-TPL-c) + (TPL-1-t), element 0 from itself
+    fr.load_c([&](int c) {
+      const int p = t + c;
+      if (p == 0) return ok ? at_off<T>(rb, vo) : mk<T>(0, 0);
+      return (ok && L - p < a.zin) ? at_off<T>(rb + (L + 1 - TPL - c) * a.sz * CB, vm) : mk<T>(0, 0);
+    });
+  } else {
+    fr.load_c([&](int c) {
+      return (ok && t + c < a.zin) ? at_off<T>(rb + c * a.sz * CB, vo) : mk<T>(0, 0);
+    });
+  }
   fr.run(lds, tw);
 #pragma clang loop unroll(disable)
   for (int o = 0; o < a.nout; ++o) {
-    const Term<T> tm = a.out[o].t[0];
+    const Term<T> tm = a.out[o].t[ph];
     const char* gb = reinterpret_cast<const char*>(tm.g + col0);
     // the tiles' LDS index arithmetic stays inside the loop (hoisted, it would
     // hold two transforms' worth of addresses in registers across it)
@@ -688,13 +739,23 @@ __global__ void __launch_bounds__((ZGeo<T, L>::NT))
     fi.load([&](int bb, int p) { return lds[FI::lidx(bb, p)]; });
     __syncthreads();
     fi.run(lds, tw);
-    char* ob = reinterpret_cast<char*>(out + o * a.o_so + col0 - int64_t(ky) * a.sy +
-                                       int64_t(ky) * a.o_sy);
-    fi.store_c([&](int c, cpx<T> v) {
-      const int q = t + c - a.w0;
-      if (ok && q >= 0 && q < a.n_out)
-        *reinterpret_cast<cpx<T>*>(ob + (c - a.w0) * a.o_sz * CB + vout) = v;
-    });
+    char* ob = reinterpret_cast<char*>(out + (ph && !a.acc ? o + a.nout : o) * a.o_so + col0 -
+                                       int64_t(ky) * a.sy + int64_t(ky) * a.o_sy);
+    if (a.acc && ph) {
+      fi.store_c([&](int c, cpx<T> v) {
+        const int q = t + c - a.w0;
+        if (ok && q >= 0 && q < a.n_out) {
+          cpx<T>* dst = reinterpret_cast<cpx<T>*>(ob + (c - a.w0) * a.o_sz * CB + vout);
+          *dst = add(*dst, v);
+        }
+      });
+    } else {
+      fi.store_c([&](int c, cpx<T> v) {
+        const int q = t + c - a.w0;
+        if (ok && q >= 0 && q < a.n_out)
+          *reinterpret_cast<cpx<T>*>(ob + (c - a.w0) * a.o_sz * CB + vout) = v;
+      });
+    }
   }
 }
 

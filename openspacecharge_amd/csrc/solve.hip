@@ -149,9 +149,36 @@ void conv_solve(osc_ctx* c, const double* rho, const int n[3], const SpecDims& d
   // rho_hat's z pass inside the multiply (once per column for all outputs)
   ZinvIO<T> zs{};
   zs.sz = zs.o_sz = KXP * L1;
-  bool zconv = fft_has_plan(L2) && zconv_fits<T>(L2, zs);
-  for (const OutSpec& os : outs)
+  bool zconv = fft_has_plan(L2) && zconv_fits<T>(L2, zs), two = zconv;
+  for (const OutSpec& os : outs) {
     zconv = zconv && os.nt == 1 && os.t[0].mir == 0 && os.t[0].g.zr;
+    // ... as do sums of such a term and an image term mirrored in z (two phases)
+    two = two && os.nt == 2 && os.t[0].mir == 0 && os.t[0].sgn == 1.0 && os.t[1].mir == 4 &&
+          os.t[0].g.zr && os.t[1].g.zr;
+  }
+  // two phases: outputs over the same two Green arrays (E and B of a
+  // component) are sums and differences of the same two parts, which then stay
+  // apart until the x pass; without such outputs the multiply adds them
+  std::vector<std::vector<int>> pairs;
+  bool apart = false;
+  if (two) {
+    for (int o = 0; o < int(outs.size()); ++o) {
+      size_t q = 0;
+      while (q < pairs.size() && (outs[pairs[q][0]].t[0].g.g != outs[o].t[0].g.g ||
+                                  outs[pairs[q][0]].t[1].g.g != outs[o].t[1].g.g))
+        ++q;
+      if (q == pairs.size()) pairs.emplace_back();
+      pairs[q].push_back(o);
+      apart = apart || pairs[q].size() > 1;
+      two = two && pairs[q].size() <= 2;
+    }
+    two = two && (!apart || (fft_has_plan(L0) && 2 * pairs.size() <= size_t(kMaxOut)));
+  }
+  if (!two) {
+    pairs.clear();
+    apart = false;
+  }
+  zconv = zconv || two;
   if (!zconv) {
     AxisIO az{};
     az.s_b = az.d_b = 1;
@@ -165,7 +192,8 @@ void conv_solve(osc_ctx* c, const double* rho, const int n[3], const SpecDims& d
     launch_axis<T>(L2, -1, sp, sp, az, L1, 1, twiddles<T>(c, L2), s);
   }
   // inverse: combine + z, y (window), x (window + epilogue)
-  const int nout = int(outs.size());
+  const int nsum = two ? int(pairs.size()) : int(outs.size());
+  const int nout = apart ? 2 * nsum : nsum;  // arrays through the y pass
   const int64_t so = KXP * L1 * nz;
   DevBuf Tb(c->pool, sizeof(cpx<T>) * so * nout);
   cpx<T>* tp = Tb.as<cpx<T>>();
@@ -180,19 +208,22 @@ void conv_solve(osc_ctx* c, const double* rho, const int n[3], const SpecDims& d
   zi.nb = d.KX;
   zi.w0 = win[2];
   zi.n_out = nz;
-  zi.nout = nout;
+  zi.nout = nsum;
   zi.zreal = outs[0].t[0].g.zr;
   zi.zin = zconv ? nz : 0;
+  zi.nphase = two ? 2 : 1;
+  zi.acc = !apart;
   bool multi = false;
-  for (int o = 0; o < nout; ++o) {
-    zi.out[o].nt = outs[o].nt;
-    multi = multi || outs[o].nt > 1;
-    for (int t = 0; t < outs[o].nt; ++t) {
-      const GreenRef& gr = outs[o].t[t].g;
+  for (int o = 0; o < nsum; ++o) {
+    const OutSpec& os = outs[two ? pairs[o][0] : o];
+    zi.out[o].nt = os.nt;
+    multi = multi || (os.nt > 1 && !two);
+    for (int t = 0; t < os.nt; ++t) {
+      const GreenRef& gr = os.t[t].g;
       OSC_REQUIRE(gr.zr == zi.zreal, OSC_ERR_ARG, "Green arrays of one solve differ in z form");
       zi.out[o].t[t].g = static_cast<const cpx<T>*>(gr.g);
-      zi.out[o].t[t].sgn = T(outs[o].t[t].sgn);
-      zi.out[o].t[t].mir = outs[o].t[t].mir;
+      zi.out[o].t[t].sgn = T(apart ? 1.0 : os.t[t].sgn);
+      zi.out[o].t[t].mir = os.t[t].mir;
       zi.out[o].t[t].zmh = gr.zmh;
       zi.out[o].t[t].zms = gr.zms;
     }
@@ -203,7 +234,7 @@ void conv_solve(osc_ctx* c, const double* rho, const int n[3], const SpecDims& d
   if (zi.zreal && multi) {
     std::map<const void*, const cpx<T>*> done;
     ProfScope ps(c, ST_GREEN_FFT);
-    for (int o = 0; o < nout; ++o)
+    for (int o = 0; o < nsum; ++o)
       for (int t = 0; t < zi.out[o].nt; ++t) {
         Term<T>& tm = zi.out[o].t[t];
         auto it = done.find(tm.g);
@@ -230,7 +261,7 @@ void conv_solve(osc_ctx* c, const double* rho, const int n[3], const SpecDims& d
   }
   {
     ProfScope ps(c, ST_INV_ZMUL);
-    launch_zinv<T>(L2, sp, tp, zi, L1, nout, twiddles<T>(c, L2), s);
+    launch_zinv<T>(L2, sp, tp, zi, L1, nsum, twiddles<T>(c, L2), s);
   }
   AxisIO ai{};
   ai.s_b = ai.d_b = 1;
@@ -255,7 +286,18 @@ void conv_solve(osc_ctx* c, const double* rho, const int n[3], const SpecDims& d
   cr.ny_rows = ny;
   cr.w0 = win[0];
   cr.n_out = nx;
-  for (int o = 0; o < nout; ++o) cr.ep[o] = outs[o].ep;
+  cr.npair = apart ? nsum : 0;
+  for (int o = 0; o < nsum; ++o) {
+    if (!apart) {
+      cr.ep[o] = outs[two ? pairs[o][0] : o].ep;
+      continue;
+    }
+    for (size_t q = 0; q < 2; ++q) {
+      Epilogue& e = cr.ep[2 * o + q];
+      e = q < pairs[o].size() ? outs[pairs[o][q]].ep : Epilogue{};
+      if (q < pairs[o].size()) e.sb = outs[pairs[o][q]].t[1].sgn;
+    }
+  }
   {
     ProfScope ps(c, ST_INV_X);
     launch_xc2r<T>(L0, tp, cr, nout, twiddles<T>(c, L0), s);
