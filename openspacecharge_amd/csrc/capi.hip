@@ -50,19 +50,6 @@ int check_len(osc_ctx* c, const int L[3]) {
   return OSC_OK;
 }
 
-// the table of fast_math.h into the context's device copy, behind the counters,
-// on its own stream (the host's table stays, and osc_ctx_set_stream waits for
-// the stream it leaves, so nothing has to wait here)
-hipError_t upload_fast_table(osc_ctx* c) {
-  static const FastMathTab table = [] {
-    FastMathTab t;
-    fast_math_table(t);
-    return t;
-  }();
-  c->fast_tab = static_cast<char*>(c->counters) + kCounterBytes;
-  return hipMemcpyAsync(c->fast_tab, &table, sizeof(table), hipMemcpyHostToDevice, c->own);
-}
-
 __global__ void k_real_to_cplx(const double* __restrict__ g, double* __restrict__ out, int64_t n) {
   for (int64_t i = blockIdx.x * int64_t(blockDim.x) + threadIdx.x; i < n;
        i += int64_t(gridDim.x) * blockDim.x) {
@@ -106,8 +93,7 @@ OSC_API int osc_ctx_create(int device, osc_ctx** out) {
   c->device = device;
   DeviceGuard g(device);
   if (hipStreamCreateWithFlags(&c->own, hipStreamNonBlocking) != hipSuccess ||
-      hipMalloc(&c->counters, kCounterBytes + sizeof(FastMathTab)) != hipSuccess ||
-      upload_fast_table(c) != hipSuccess ||
+      hipMalloc(&c->counters, kCounterBytes) != hipSuccess || !(c->fast_tab = fast_table(device)) ||
       hipHostMalloc(reinterpret_cast<void**>(&c->mesh_host), kPinnedBytes,
                     hipHostMallocDefault) != hipSuccess ||
       hipEventCreateWithFlags(&c->mesh_ev, hipEventDisableTiming) != hipSuccess ||

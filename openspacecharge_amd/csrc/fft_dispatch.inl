@@ -12,12 +12,18 @@ inline dim3 grid3(int64_t x, int64_t y, int64_t z) {
 }
 inline int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
+inline bool mirrored(const AxisIO& a) {
+  bool m = a.batch == 0 && a.mh > 0;
+  for (int o = 0; o < a.batch; ++o) m = m || a.bmh[o] > 0;
+  return m;
+}
+
 template <int L, int V>
 void axis_tv(int dir, const cpx<T>* in, cpx<T>* out, const AxisIO& a, int g1, int g2,
              const cpx<T>* tw, hipStream_t s) {
   constexpr int BX = AxisTiles<T, L>::bx(V), NT = BX * Geo<T, L>::TPL;
   dim3 g = grid3(cdiv(a.nb, BX), g1, g2);
-  if (dir < 0 && a.mh > 0)
+  if (mirrored(a))
     launch((k_axis<T, L, -1, true, BX>), g, dim3(NT), 0, s, in, out, a, tw);
   else if (dir < 0)
     launch((k_axis<T, L, -1, false, BX>), g, dim3(NT), 0, s, in, out, a, tw);
@@ -28,7 +34,7 @@ void axis_tv(int dir, const cpx<T>* in, cpx<T>* out, const AxisIO& a, int g1, in
 template <int L>
 void axis_t(int dir, const cpx<T>* in, cpx<T>* out, const AxisIO& a, int g1, int g2,
             const cpx<T>* tw, hipStream_t s) {
-  const int kind = dir > 0 ? 2 : (a.mh > 0 ? 1 : 0);
+  const int kind = dir > 0 ? 2 : (mirrored(a) ? 1 : 0);
   const int64_t lines = int64_t(a.nb) * g1 * g2;
   bool distinct[3];
   for (int v = 0; v < 3; ++v) distinct[v] = v == 1 || AxisTiles<T, L>::bx(v) != AxisTiles<T, L>::bx(1);
@@ -45,15 +51,22 @@ void axis_t(int dir, const cpx<T>* in, cpx<T>* out, const AxisIO& a, int g1, int
   }
   tune.done(s);
 }
+// rows of the widest array of a batch
+inline int64_t batch_rows(const R2CBatch<T>& b) {
+  int64_t n = 0;
+  for (int q = 0; q < b.n; ++q) n = b.a[q].nrows > n ? b.a[q].nrows : n;
+  return n;
+}
 template <int L>
-void xr2c_t(const double* in, cpx<T>* out, const R2CIO& a, const cpx<T>* tw, hipStream_t s,
-            const CornerDiff* cd) {
+void xr2c_t(const R2CBatch<T>& b, bool diff, const cpx<T>* tw, hipStream_t s) {
   constexpr int BX = XGeo<T, L>::BX, NT = XGeo<T, L>::NT;
-  dim3 g = grid3(cdiv(cdiv(a.nrows, 2), BX), 1, 1);
-  if (cd)
-    launch((k_xr2c<T, L, true>), g, dim3(NT), 0, s, in, out, a, tw, *cd);
-  else
-    launch((k_xr2c<T, L, false>), g, dim3(NT), 0, s, in, out, a, tw, CornerDiff{});
+  const dim3 g = grid3(cdiv(cdiv(batch_rows(b), 2), BX), b.n, 1);
+  if (b.n > 1) {
+    launch((diff ? k_xr2c<T, L, true, 3> : k_xr2c<T, L, false, 3>), g, dim3(NT), 0, s, b, tw);
+  } else {
+    const R2CBatch<T, 1> one{{b.in[0]}, {b.out[0]}, {b.a[0]}, {b.cd[0]}, 1};
+    launch((diff ? k_xr2c<T, L, true, 1> : k_xr2c<T, L, false, 1>), g, dim3(NT), 0, s, one, tw);
+  }
 }
 template <int L>
 void xc2r_t(const cpx<T>* in, const C2RIO<T>& a, int nout, const cpx<T>* tw, hipStream_t s) {
@@ -101,8 +114,12 @@ void zinv_t(const cpx<T>* rho, cpx<T>* out, const ZinvIO<T>& a, int Ly, int nout
 template <>
 void launch_axis<T>(int L, int dir, const cpx<T>* in, cpx<T>* out, const AxisIO& a, int g1, int g2,
                     const cpx<T>* tw, hipStream_t s) {
-  OSC_REQUIRE(a.mh == 0 || (dir < 0 && 2 * a.mh == L), OSC_ERR_ARG,
-              "half-stored input lines are for forward passes over even lengths");
+  OSC_REQUIRE(a.batch == 0 || (a.batch == g2 && g2 <= 3), OSC_ERR_ARG, "bad batch");
+  for (int o = 0; o < (a.batch ? a.batch : 1); ++o) {
+    const int mh = a.batch ? a.bmh[o] : a.mh;
+    OSC_REQUIRE(mh == 0 || (dir < 0 && 2 * mh == L), OSC_ERR_ARG,
+                "half-stored input lines are for forward passes over even lengths");
+  }
   switch (L) {
 #define OSC_CASE(LL)                           \
   case LL:                                     \
@@ -117,36 +134,21 @@ void launch_axis<T>(int L, int dir, const cpx<T>* in, cpx<T>* out, const AxisIO&
 }
 
 template <>
-void launch_xr2c<T>(int L, const double* in, cpx<T>* out, const R2CIO& a, const cpx<T>* tw,
-                    hipStream_t s) {
-  OSC_REQUIRE(a.nrows < (int64_t(1) << 31), OSC_ERR_ARG, "x pass: too many rows for 32-bit indices");
+void launch_xr2c<T>(int L, const R2CBatch<T>& b, bool diff, const cpx<T>* tw, hipStream_t s) {
+  OSC_REQUIRE(b.n >= 1 && b.n <= 3, OSC_ERR_ARG, "bad batch");
+  OSC_REQUIRE(batch_rows(b) < (int64_t(1) << 31), OSC_ERR_ARG,
+              "x pass: too many rows for 32-bit indices");
   switch (L) {
-#define OSC_CASE(LL)                         \
-  case LL:                                   \
-    xr2c_t<LL>(in, out, a, tw, s, nullptr);  \
+#define OSC_CASE(LL)           \
+  case LL:                     \
+    xr2c_t<LL>(b, diff, tw, s); \
     break;
     OSC_FOR_EACH_L(OSC_CASE)
 #undef OSC_CASE
     default:
-      gen_xr2c<T>(L, in, out, a, nullptr, tw, s);
-  }
-  OSC_HIP(hipGetLastError());
-}
-
-template <>
-void launch_xr2c_diff<T>(int L, const double* F, cpx<T>* out, const R2CIO& a,
-                         const CornerDiff& cd, const cpx<T>* tw, hipStream_t s) {
-  OSC_REQUIRE(a.nrows < (int64_t(1) << 31), OSC_ERR_ARG, "x pass: too many rows for 32-bit indices");
-  switch (L) {
-#define OSC_CASE(LL)                     \
-  case LL:                               \
-    xr2c_t<LL>(F, out, a, tw, s, &cd);   \
-    break;
-    OSC_FOR_EACH_L(OSC_CASE)
-#undef OSC_CASE
-    default:
-      OSC_REQUIRE(!cd.far, OSC_ERR_FFT_LENGTH, "far-field cells need a planned length");
-      gen_xr2c<T>(L, F, out, a, &cd, tw, s);
+      for (int q = 0; diff && q < b.n; ++q)
+        OSC_REQUIRE(!b.cd[q].far, OSC_ERR_FFT_LENGTH, "far-field cells need a planned length");
+      gen_xr2c<T>(L, b, diff, tw, s);
   }
   OSC_HIP(hipGetLastError());
 }

@@ -27,12 +27,20 @@ __global__ void __launch_bounds__(kRtMaxThreads)
   const uint32_t gx = gridDim.x, gy = gridDim.y;
   const uint32_t lw = xcd_block(blockIdx.x + gx * (blockIdx.y + gy * blockIdx.z), gx * gy * gridDim.z);
   const int b0 = int(lw % gx) << pl.bs, by = int((lw / gx) % gy), bz = int(lw / (gx * gy));
-  const cpx<T>* ib = in + b0 * a.s_b + by * a.s_o1 + bz * a.s_o2;
+  int64_t src = bz * a.s_o2, dst = bz * a.d_o2;
+  int mh = a.mh, ms = a.ms;
+  if (a.batch) {
+    if (by >= a.n1[bz]) return;
+    src = dst = a.at[bz];
+    mh = a.bmh[bz];
+    ms = a.bms[bz];
+  }
+  const cpx<T>* ib = in + b0 * a.s_b + by * a.s_o1 + src;
   f.load([&](int b, int p) {
-    return b0 + b < a.nb ? axis_in(ib + b * a.s_b, a, pl.L, p) : mk<T>(0, 0);
+    return b0 + b < a.nb ? axis_in(ib + b * a.s_b, a, mh, ms, pl.L, p) : mk<T>(0, 0);
   });
   f.run();
-  cpx<T>* ob = out + b0 * a.d_b + by * a.d_o1 + bz * a.d_o2;
+  cpx<T>* ob = out + b0 * a.d_b + by * a.d_o1 + dst;
   f.each(a.n_out, [&](int b, int q) {
     if (b0 + b < a.nb) ob[b * a.d_b + q * a.d_p] = f.get(b, q + a.w0);
   });
@@ -40,9 +48,12 @@ __global__ void __launch_bounds__(kRtMaxThreads)
 
 template <typename T, bool DIFF, bool BIG>
 __global__ void __launch_bounds__(kRtMaxThreads)
-    k_xr2c_gen(const double* __restrict__ in, cpx<T>* __restrict__ out, R2CIO a,
-               const cpx<T>* __restrict__ tw, GenericPlan pl, CornerDiff cd) {
+    k_xr2c_gen(R2CBatch<T> bt, const cpx<T>* __restrict__ tw, GenericPlan pl) {
   extern __shared__ unsigned char smem_raw[];
+  const double* __restrict__ in = bt.in[blockIdx.y];
+  cpx<T>* __restrict__ out = bt.out[blockIdx.y];
+  const R2CIO& a = bt.a[blockIdx.y];
+  const CornerDiff& cd = bt.cd[blockIdx.y];
   FftRt<T, -1, true, BIG> f(pl, reinterpret_cast<cpx<T>*>(smem_raw), tw);
   const int L = pl.L;
   const int64_t r0 = 2 * (int64_t(blockIdx.x) << pl.bs);
@@ -161,15 +172,16 @@ void gen_axis<OscReal>(int L, int dir, const cpx<OscReal>* in, cpx<OscReal>* out
 }
 
 template <>
-void gen_xr2c<OscReal>(int L, const double* in, cpx<OscReal>* out, const R2CIO& a,
-                       const CornerDiff* cd, const cpx<OscReal>* tw, hipStream_t s) {
+void gen_xr2c<OscReal>(int L, const R2CBatch<OscReal>& b, bool diff, const cpx<OscReal>* tw,
+                       hipStream_t s) {
   using T = OscReal;
-  const int64_t lines = cdiv(a.nrows, 2);
+  int64_t lines = 0;
+  for (int q = 0; q < b.n; ++q) lines = std::max(lines, cdiv(b.a[q].nrows, 2));
   const GenericPlan pl = rt_plan(L, lines);
-  const dim3 g = grid3(cdiv(lines, 1 << pl.bs), 1, 1);
-  auto* k = pl.big ? (cd ? k_xr2c_gen<T, true, true> : k_xr2c_gen<T, false, true>)
-                   : (cd ? k_xr2c_gen<T, true, false> : k_xr2c_gen<T, false, false>);
-  launch(k, g, dim3(pl.nt), rt_lds_bytes(pl), s, in, out, a, tw, pl, cd ? *cd : CornerDiff{});
+  const dim3 g = grid3(cdiv(lines, 1 << pl.bs), b.n, 1);
+  auto* k = pl.big ? (diff ? k_xr2c_gen<T, true, true> : k_xr2c_gen<T, false, true>)
+                   : (diff ? k_xr2c_gen<T, true, false> : k_xr2c_gen<T, false, false>);
+  launch(k, g, dim3(pl.nt), rt_lds_bytes(pl), s, b, tw, pl);
 }
 
 template <>

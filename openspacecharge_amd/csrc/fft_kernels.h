@@ -24,16 +24,23 @@ struct AxisIO {
   // line being mirror-symmetric about L/2 - 1: element p in [mh, L-2] is
   // ms * element L-2-p and element L-1 is zero
   int mh, ms;
+  // batch > 0: the blocks o2 are arrays of their own, at[o2] elements from the
+  // first (input and output), with o1 < n1[o2] and their own mh and ms.  (Not
+  // by these arrays always: arguments at a place that depends on the workgroup
+  // cost it a round trip to memory before its first load, 1 to 2 % of a pass.)
+  int batch;
+  int n1[3], bmh[3], bms[3];
+  int64_t at[3];
 };
 
 // element p of an axis input line (see AxisIO::mh)
 template <typename T>
-__device__ __forceinline__ cpx<T> axis_in(const cpx<T>* ib, const AxisIO& a, int L, int p) {
+__device__ __forceinline__ cpx<T> axis_in(const cpx<T>* ib, const AxisIO& a, int mh, int ms, int L, int p) {
   if (p >= a.n_in) return mk<T>(0, 0);
-  if (a.mh > 0 && p >= a.mh) {
+  if (mh > 0 && p >= mh) {
     if (p == L - 1) return mk<T>(0, 0);
     const cpx<T> v = ib[(L - 2 - p) * a.s_p];
-    return a.ms < 0 ? mk<T>(-v.x, -v.y) : v;
+    return ms < 0 ? mk<T>(-v.x, -v.y) : v;
   }
   return ib[p * a.s_p];
 }
@@ -167,7 +174,7 @@ __device__ __forceinline__ cpx<T> ldc(const cpx<T>* p) {
 // ---------------------------------------------------------------------------
 // strided line FFT (y or z axis, or x with s_p = 1)
 // ---------------------------------------------------------------------------
-// MIR: the input lines are stored as halves (AxisIO::mh)
+// MIR: input lines may be stored as halves (AxisIO::mh)
 template <typename T, int L, int DIR, bool MIR, int BX = Geo<T, L>::BX>
 __global__ void __launch_bounds__((BX * Geo<T, L>::TPL))
     k_axis(const cpx<T>* __restrict__ in, cpx<T>* out, AxisIO a, const cpx<T>* __restrict__ tw) {
@@ -178,15 +185,23 @@ __global__ void __launch_bounds__((BX * Geo<T, L>::TPL))
   const uint32_t gx = gridDim.x, gy = gridDim.y;
   const uint32_t lw = xcd_block(blockIdx.x + gx * (blockIdx.y + gy * blockIdx.z), gx * gy * gridDim.z);
   const int bx = int(lw % gx), by = int((lw / gx) % gy), bz = int(lw / (gx * gy));
+  int64_t src = bz * a.s_o2, dst = bz * a.d_o2;
+  int mh = a.mh, ms = a.ms;
+  if (a.batch) {
+    if (by >= a.n1[bz]) return;
+    src = dst = a.at[bz];
+    mh = a.bmh[bz];
+    ms = a.bms[bz];
+  }
   const int bg = bx * BX + f.b;
   const bool ok = bg < a.nb;
-  const cpx<T>* ib = in + (ok ? bg * a.s_b + by * a.s_o1 + bz * a.s_o2 : 0);
+  const cpx<T>* ib = in + (ok ? bg * a.s_b + by * a.s_o1 + src : 0);
   if constexpr (MIR)
-    f.load([&](int, int p) { return ok ? axis_in(ib, a, L, p) : mk<T>(0, 0); });
+    f.load([&](int, int p) { return ok ? axis_in(ib, a, mh, ms, L, p) : mk<T>(0, 0); });
   else
     f.load([&](int, int p) { return (ok && p < a.n_in) ? ib[p * a.s_p] : mk<T>(0, 0); });
   f.run(lds, tw);
-  cpx<T>* ob = out + (ok ? bg * a.d_b + by * a.d_o1 + bz * a.d_o2 : 0);
+  cpx<T>* ob = out + (ok ? bg * a.d_b + by * a.d_o1 + dst : 0);
   f.store([&](int, int p, cpx<T> v) {
     const int q = p - a.w0;
     if (ok && q >= 0 && q < a.n_out) ob[q * a.d_p] = v;
@@ -307,15 +322,36 @@ __device__ __forceinline__ double diff_elem(const double* q, const R2CIO& a, con
   return cd.zero_raw ? 0.0 : q[p];
 }
 
-template <typename T, int L, bool DIFF>
+// Up to three arrays of one x pass (the Green functions of a solve's components)
+template <typename T, int N = 3>
+struct R2CBatch {
+  const double* in[N];
+  cpx<T>* out[N];
+  R2CIO a[N];
+  CornerDiff cd[N];
+  int n;
+};
+
+// DIFF: bound by the loads of the corner difference (four rows of the primitive
+// per row, eight elements per element): 256^3 grid in FP64, 89 us a component.
+// Sharing the primitive's row between the two rows of a line (12 loads instead
+// of 16) and a contiguous range of the rows per XCD gain together in one pass
+// over three components (268 -> 251 us) and nothing in a component's own.
+// N arrays: one's arguments are at fixed places (5 % of the pass).
+template <typename T, int L, bool DIFF, int N>
 __global__ void __launch_bounds__((XGeo<T, L>::NT))
-    k_xr2c(const double* __restrict__ in, cpx<T>* __restrict__ out, R2CIO a,
-           const cpx<T>* __restrict__ tw, CornerDiff cd) {
+    k_xr2c(R2CBatch<T, N> bt, const cpx<T>* __restrict__ tw) {
   constexpr int BX = XGeo<T, L>::BX;
   using F = FftTile<T, L, -1, BX, true>;
   __shared__ cpx<T> lds[F::LDS];
+  const uint32_t blk = blockIdx.x, arr = N > 1 ? blockIdx.y : 0;
+  const R2CIO& a = bt.a[arr];
+  const CornerDiff& cd = bt.cd[arr];
+  if (N > 1 && 2 * int64_t(blk) * BX >= a.nrows) return;
+  const double* __restrict__ in = bt.in[arr];
+  cpx<T>* __restrict__ out = bt.out[arr];
   F f;
-  const int64_t ra = 2 * (int64_t(blockIdx.x) * BX + f.b), rb = ra + 1;
+  const int64_t ra = 2 * (int64_t(blk) * BX + f.b), rb = ra + 1;
   const bool oka = ra < a.nrows, okb = rb < a.nrows;
   const RowPair rp = row_pair(ra, a.ny_rows);
   if constexpr (DIFF) {

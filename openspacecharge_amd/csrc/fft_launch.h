@@ -42,13 +42,10 @@ GenericPlan generic_plan(int L);
 template <typename T>
 void launch_axis(int L, int dir, const cpx<T>* in, cpx<T>* out, const AxisIO& a, int g1, int g2,
                  const cpx<T>* tw, hipStream_t s);
+// the x pass of up to three arrays; diff: over the corner differences of
+// primitives (far-field cells: lengths with a plan only)
 template <typename T>
-void launch_xr2c(int L, const double* in, cpx<T>* out, const R2CIO& a, const cpx<T>* tw,
-                 hipStream_t s);
-// x pass over the corner difference of a primitive F (lengths with a plan only)
-template <typename T>
-void launch_xr2c_diff(int L, const double* F, cpx<T>* out, const R2CIO& a, const CornerDiff& cd,
-                      const cpx<T>* tw, hipStream_t s);
+void launch_xr2c(int L, const R2CBatch<T>& b, bool diff, const cpx<T>* tw, hipStream_t s);
 template <typename T>
 void launch_xc2r(int L, const cpx<T>* in, const C2RIO<T>& a, int nout, const cpx<T>* tw,
                  hipStream_t s);
@@ -65,8 +62,7 @@ template <typename T>
 void gen_axis(int L, int dir, const cpx<T>* in, cpx<T>* out, const AxisIO& a, int g1, int g2,
               const cpx<T>* tw, hipStream_t s);
 template <typename T>
-void gen_xr2c(int L, const double* in, cpx<T>* out, const R2CIO& a, const CornerDiff* cd,
-              const cpx<T>* tw, hipStream_t s);
+void gen_xr2c(int L, const R2CBatch<T>& b, bool diff, const cpx<T>* tw, hipStream_t s);
 template <typename T>
 void gen_xc2r(int L, const cpx<T>* in, const C2RIO<T>& a, int nout, const cpx<T>* tw,
               hipStream_t s);

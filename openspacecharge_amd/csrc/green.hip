@@ -1,5 +1,7 @@
 // Green-function builders (FP64, on the device), their R2C spectra, the
 // spectrum cache, and conversions to the upstream full-spectrum convention.
+#include <mutex>
+
 #include "fast_math.h"
 #include "igf_math.h"
 #include "osc_internal.h"
@@ -14,6 +16,8 @@ inline int64_t nblk(int64_t n, int t = kThreads) {
   int64_t b = (n + t - 1) / t;
   return b > 65536 * 8 ? 65536 * 8 : b;
 }
+
+__device__ FastMathTab g_fast_tab;
 
 // primitive of osc_get_cgrn_freespace on the offset grid
 // (open_spacecharge_mod.f90:674-691): F = prim(u,v,w) * factor.
@@ -33,12 +37,28 @@ inline int64_t nblk(int64_t n, int t = kThreads) {
 // dz, factor and the minima are formed here with the host's operations in
 // the host's order (build_offset_primitive); img selects the z offset of the
 // cathode image solve, 2 min(3) + (max(3) - min(3)) (open_spacecharge_mod.f90:472-476).
+//
+// One launch for up to three components (PrimOne), their planes one after
+// another along the grid's z: on small meshes each has less than a wave per CU.
+struct PrimOne {
+  double* F;
+  double factor;
+  int icomp, mev, mod, half, zlo, zhi, zbase, nz;
+};
+struct PrimBatch {
+  PrimOne c[3];
+};
 __global__ void __launch_bounds__(64)
-    k_prim_offset(double* __restrict__ F, int L0, int L1, int L2, double dx, double dy, double dz,
-                  double umin, double vmin, double wmin, double factor, int icomp, int mev,
-                  int mod, int half, int zlo, int zhi, int zbase,
-                  const MeshDev* __restrict__ md, double gamma, int img) {
-  const int i = blockIdx.x * 64 + threadIdx.x, j = blockIdx.y, k = zbase + int(blockIdx.z);
+    k_prim_offset(PrimBatch pb, int L0, int L1, int L2, double dx, double dy, double dz,
+                  double umin, double vmin, double wmin, const MeshDev* __restrict__ md,
+                  double gamma, int img) {
+  int q = 0, zq = int(blockIdx.z);
+  while (q < 2 && zq >= pb.c[q].nz) zq -= pb.c[q++].nz;
+  const PrimOne& o = pb.c[q];
+  double* __restrict__ F = o.F;
+  double factor = o.factor;
+  const int icomp = o.icomp, mev = o.mev, mod = o.mod, half = o.half, zlo = o.zlo, zhi = o.zhi;
+  const int i = blockIdx.x * 64 + threadIdx.x, j = blockIdx.y, k = o.zbase + zq;
   if (md) {
     dx = md->d[0];
     dy = md->d[1];
@@ -54,7 +74,7 @@ __global__ void __launch_bounds__(64)
     wmin = wmin + oz * gamma;
   }
   const bool m0 = mev == 0 || mod == 0, m1 = mev == 1 || mod == 1, m2 = mev == 2 || mod == 2;
-  if (i >= (m0 ? L0 / 2 : L0)) return;
+  if (i >= (m0 ? L0 / 2 : L0) || j >= (m1 ? L1 / 2 : L1)) return;
   // only the planes [zlo, zhi] are read (the near cells of a far-field build):
   // a plane outside is evaluated when its mirror image is inside
   if (k < zlo || k > zhi) {
@@ -464,6 +484,22 @@ __global__ void k_convert(const cpx<double>* __restrict__ in, cpx<float>* __rest
 
 }  // namespace
 
+const void* fast_table(int device) {
+  static std::mutex mu;
+  static std::map<int, void*> made;
+  std::lock_guard<std::mutex> lk(mu);
+  void*& p = made[device];
+  if (p) return p;
+  FastMathTab t;
+  fast_math_table(t);
+  void* d = nullptr;
+  // (a copy that has ended on return, for the streams of every context)
+  if (hipGetSymbolAddress(&d, HIP_SYMBOL(g_fast_tab)) != hipSuccess ||
+      hipMemcpy(d, &t, sizeof(t), hipMemcpyHostToDevice) != hipSuccess)
+    return nullptr;
+  return p = d;
+}
+
 // Axes along which the solve-path primitive of an E component is mirrored
 // (k_prim_offset): mev, where xlafun2 is even (its first argument), and mod,
 // where it is odd (its third argument); -1 where the axis has an offset or odd
@@ -573,61 +609,74 @@ static void launch_prim3(osc_ctx* c, const GreenSpec& s, double* const F[3]) {
   OSC_HIP(hipGetLastError());
 }
 
-// primitive F of an offset-kind Green function (open_spacecharge_mod.f90:662-691).
+// The primitives of n components of an offset-kind Green function
+// (open_spacecharge_mod.f90:662-691), component icomp[q] into F[q].
 // lower_halves: the reader (the corner-difference x pass) loads only the
 // lower half, plus one plane, along mirrored y and z axes (unshifted z), so
-// the mirror images beyond that are not stored.
-static void build_offset_primitive(osc_ctx* c, const GreenSpec& s, double* F, bool fast,
-                                   bool lower_halves = false, int zlo = 0, int zhi = -1) {
-  if (!fast && s.icomp >= 1) {
-    double* one[3] = {nullptr, nullptr, nullptr};
-    one[s.icomp - 1] = F;
-    launch_prim3(c, s, one);
+// the mirror images beyond that are not stored.  [zlo, zhi]: the planes wanted.
+static void build_offset_primitives(osc_ctx* c, const GreenSpec& s, int n, const int icomp[],
+                                    double* const F[], bool fast, bool lower_halves, int zlo,
+                                    int zhi) {
+  if (!fast && icomp[0] >= 1) {
+    double* comp[3] = {nullptr, nullptr, nullptr};
+    for (int q = 0; q < n; ++q) comp[icomp[q] - 1] = F[q];
+    launch_prim3(c, s, comp);
     return;
   }
-  if (zhi < 0 && zlo == 0) zhi = s.L[2] - 1;  // every plane
   const double dx = s.delta[0], dy = s.delta[1], dz = s.delta[2] * s.gamma;
-  const double factor =
-      (s.icomp == 1 || s.icomp == 2) ? s.gamma / (dx * dy * dz) : 1.0 / (dx * dy * dz);
   double umin = (0.5 - double(s.L[0] / 2)) * dx;
   double vmin = (0.5 - double(s.L[1] / 2)) * dy;
   double wmin = (0.5 - double(s.L[2] / 2)) * dz;
   umin = umin + s.offset[0];
   vmin = vmin + s.offset[1];
   wmin = wmin + s.offset[2] * s.gamma;
-  const dim3 g3(unsigned((s.L[0] + 63) / 64), unsigned(s.L[1]), unsigned(s.L[2]));
-  // the FP32 solve path evaluates E components on a quarter of the grid (even
-  // mirror along their own axis, odd mirror along the axis of xlafun2's third
-  // argument, see k_prim_offset); every other build keeps upstream's
-  // coordinate arithmetic on the whole grid
-  int mev, mod;
-  prim_mirrors(s, fast, mev, mod);
-  dim3 gp = g3;
-  if (mev == 0 || mod == 0) gp.x = unsigned((s.L[0] / 2 + 63) / 64);
-  if (mev == 1 || mod == 1) gp.y = unsigned(s.L[1] / 2);
-  // the planes launched: those of [zlo, zhi], or of the lower half whose
-  // mirror images are in it
-  int zbase = zlo, ztop = zhi;
-  if (mev == 2 || mod == 2) {
-    zbase = std::max(0, std::min(zlo, s.L[2] - 1 - zhi));
-    ztop = std::min(s.L[2] / 2 - 1, std::max(zhi, s.L[2] - 1 - zlo));
-  }
-  if (ztop < zbase) return;
-  gp.z = unsigned(ztop - zbase + 1);
   // a solve being captured for replay takes the spacing from the device mesh
   // record; only the zero offset of the free solve and the image offset of
   // the cathode solve occur there
   const MeshDev* md = c->green_md;
   OSC_REQUIRE(!md || (s.offset[0] == 0.0 && s.offset[1] == 0.0), OSC_ERR_ARG,
               "device-side Green parameters: unsupported offset");
-  int half = 0;
-  if (lower_halves) {
-    if (mev == 1 || mod == 1) half |= 2;
-    if ((mev == 2 || mod == 2) && s.out_shift_z == 0) half |= 4;
+  PrimBatch pb{};
+  dim3 g(1, 1, 0);
+  int m = 0;
+  for (int q = 0; q < n; ++q) {
+    // the FP32 solve path evaluates E components on a quarter of the grid (even
+    // mirror along their own axis, odd mirror along the axis of xlafun2's third
+    // argument, see k_prim_offset); every other build keeps upstream's
+    // coordinate arithmetic on the whole grid
+    GreenSpec t = s;
+    t.icomp = icomp[q];
+    PrimOne o{};
+    prim_mirrors(t, fast, o.mev, o.mod);
+    o.F = F[q];
+    o.icomp = icomp[q];
+    o.factor = (icomp[q] == 1 || icomp[q] == 2) ? s.gamma / (dx * dy * dz) : 1.0 / (dx * dy * dz);
+    o.zlo = zlo;
+    o.zhi = zhi;
+    // the planes launched: those of [zlo, zhi], or of the lower half whose
+    // mirror images are in it
+    int ztop = zhi;
+    o.zbase = zlo;
+    if (o.mev == 2 || o.mod == 2) {
+      o.zbase = std::max(0, std::min(zlo, s.L[2] - 1 - zhi));
+      ztop = std::min(s.L[2] / 2 - 1, std::max(zhi, s.L[2] - 1 - zlo));
+    }
+    o.nz = ztop - o.zbase + 1;
+    if (o.nz <= 0) continue;
+    if (lower_halves) {
+      if (o.mev == 1 || o.mod == 1) o.half |= 2;
+      if ((o.mev == 2 || o.mod == 2) && s.out_shift_z == 0) o.half |= 4;
+    }
+    const int nx = o.mev == 0 || o.mod == 0 ? s.L[0] / 2 : s.L[0];
+    const int ny = o.mev == 1 || o.mod == 1 ? s.L[1] / 2 : s.L[1];
+    g.x = std::max(g.x, unsigned((nx + 63) / 64));
+    g.y = std::max(g.y, unsigned(ny));
+    g.z += unsigned(o.nz);
+    pb.c[m++] = o;
   }
-  launch(k_prim_offset, gp, dim3(64), 0, c->stream, F, s.L[0], s.L[1], s.L[2], dx, dy,
-                     dz, umin, vmin, wmin, factor, s.icomp, mev, mod, half, zlo, zhi, zbase,
-                     md, s.gamma, int(md && s.out_shift_z != 0));
+  if (m == 0) return;
+  launch(k_prim_offset, g, dim3(64), 0, c->stream, pb, s.L[0], s.L[1], s.L[2], dx, dy, dz, umin,
+         vmin, wmin, md, s.gamma, int(md && s.out_shift_z != 0));
   OSC_HIP(hipGetLastError());
 }
 
@@ -676,7 +725,8 @@ void build_green_real(osc_ctx* c, const GreenSpec& s, double* g, bool fast) {
   if (s.kind == GK_OFFSET) {
     // osc_get_cgrn_freespace (open_spacecharge_mod.f90:633-707)
     DevBuf F(c->pool, sizeof(double) * N);
-    build_offset_primitive(c, s, F.as<double>(), fast);
+    double* const one[1] = {F.as<double>()};
+    build_offset_primitives(c, s, 1, &s.icomp, one, fast, false, 0, s.L[2] - 1);
     const dim3 g3(unsigned((s.L[0] + 63) / 64), unsigned(s.L[1]), unsigned(s.L[2]));
     launch(k_diff_offset, g3, dim3(64), 0, c->stream, F.as<const double>(), g, s.L[0],
                        s.L[1], s.L[2], s.out_shift_z, s.zero_raw);
@@ -710,31 +760,52 @@ void build_green_real(osc_ctx* c, const GreenSpec& s, double* g, bool fast) {
   }
 }
 
-// With a corner difference and sym (per axis: 0, +1 even, -1 odd about
+// With corner differences and sym (per array and axis: 0, +1 even, -1 odd about
 // L/2 - 1, last plane zero), lines along y and z are computed only for the
 // lower half of a symmetric axis until that axis is transformed, whose pass
 // rebuilds the upper half as it loads (AxisIO::mh).
 template <typename T>
-void spectrum_forward_full(osc_ctx* c, const double* g, cpx<T>* spec, const SpecDims& d,
-                           const CornerDiff* cd, const int* sym, GreenRef* zr) {
+static void spectra_forward(osc_ctx* c, int n, const double* const g[], cpx<T>* const spec[],
+                            const SpecDims& d, const CornerDiff* cd, const int (*sym)[3],
+                            GreenRef* const* zr) {
   const int L0 = d.L[0], L1 = d.L[1], L2 = d.L[2];
   ProfScope ps(c, ST_GREEN_FFT);
-  const bool hy = cd && sym && sym[1] != 0 && L1 % 2 == 0;
-  const bool hz = cd && sym && sym[2] != 0 && L2 % 2 == 0 && cd->sh == 0;
-  const int Yh = hy ? L1 / 2 : L1, Zh = hz ? L2 / 2 : L2;
-  R2CIO r{};
-  r.in_sy = L0;
-  r.in_sz = int64_t(L0) * L1;
-  r.out_sy = d.KXP;
-  r.out_sz = int64_t(d.KXP) * L1;
-  r.nrows = int64_t(Yh) * Zh;
-  r.ny_rows = Yh;
-  r.n_in = L0;
-  if (cd)
-    launch_xr2c_diff<T>(L0, g, spec, r, *cd, twiddles<T>(c, L0), c->stream);
-  else
-    launch_xr2c<T>(L0, g, spec, r, twiddles<T>(c, L0), c->stream);
-  AxisIO ay{};
+  R2CBatch<T> rb{};
+  rb.n = n;
+  AxisIO ay{}, az{};
+  int zmost = 0;
+  for (int q = 0; q < n; ++q) {
+    const bool hy = cd && sym && sym[q][1] != 0 && L1 % 2 == 0;
+    const bool hz = cd && sym && sym[q][2] != 0 && L2 % 2 == 0 && cd[q].sh == 0;
+    const int Yh = hy ? L1 / 2 : L1, Zh = hz ? L2 / 2 : L2;
+    R2CIO& r = rb.a[q];
+    r.in_sy = L0;
+    r.in_sz = int64_t(L0) * L1;
+    r.out_sy = d.KXP;
+    r.out_sz = int64_t(d.KXP) * L1;
+    r.nrows = int64_t(Yh) * Zh;
+    r.ny_rows = Yh;
+    r.n_in = L0;
+    rb.in[q] = g[q];
+    rb.out[q] = spec[q];
+    if (cd) rb.cd[q] = cd[q];
+    // spectrum q in elements from the first (of one allocation size: aligned alike)
+    ay.at[q] = az.at[q] = (reinterpret_cast<intptr_t>(spec[q]) - reinterpret_cast<intptr_t>(spec[0])) /
+                          intptr_t(sizeof(cpx<T>));
+    ay.n1[q] = Zh;
+    az.n1[q] = L1;
+    zmost = std::max(zmost, Zh);
+    ay.bmh[q] = hy ? L1 / 2 : 0;
+    ay.bms[q] = hy ? sym[q][1] : 0;
+    az.bmh[q] = hz ? L2 / 2 : 0;
+    az.bms[q] = hz ? sym[q][2] : 0;
+  }
+  for (AxisIO* a : {&ay, &az}) {
+    a->batch = n > 1 ? n : 0;
+    a->mh = a->bmh[0];
+    a->ms = a->bms[0];
+  }
+  launch_xr2c<T>(L0, rb, cd != nullptr, twiddles<T>(c, L0), c->stream);
   ay.s_b = ay.d_b = 1;
   ay.s_p = ay.d_p = d.KXP;
   ay.s_o1 = ay.d_o1 = int64_t(d.KXP) * L1;
@@ -742,17 +813,15 @@ void spectrum_forward_full(osc_ctx* c, const double* g, cpx<T>* spec, const Spec
   ay.n_in = L1;
   ay.w0 = 0;
   ay.n_out = L1;
-  ay.mh = hy ? L1 / 2 : 0;
-  ay.ms = hy ? sym[1] : 0;
-  launch_axis<T>(L1, -1, spec, spec, ay, Zh, 1, twiddles<T>(c, L1), c->stream);
+  launch_axis<T>(L1, -1, spec[0], spec[0], ay, zmost, n, twiddles<T>(c, L1), c->stream);
   if (zr) {
-    zr->g = spec;
-    zr->zr = 1;
-    zr->zmh = hz ? L2 / 2 : 0;
-    zr->zms = hz ? sym[2] : 0;
+    for (int q = 0; q < n; ++q) {
+      zr[q]->zr = 1;
+      zr[q]->zmh = az.bmh[q];
+      zr[q]->zms = az.bms[q];
+    }
     return;
   }
-  AxisIO az{};
   az.s_b = az.d_b = 1;
   az.s_p = az.d_p = int64_t(d.KXP) * L1;
   az.s_o1 = az.d_o1 = d.KXP;
@@ -760,14 +829,12 @@ void spectrum_forward_full(osc_ctx* c, const double* g, cpx<T>* spec, const Spec
   az.n_in = L2;
   az.w0 = 0;
   az.n_out = L2;
-  az.mh = hz ? L2 / 2 : 0;
-  az.ms = hz ? sym[2] : 0;
-  launch_axis<T>(L2, -1, spec, spec, az, L1, 1, twiddles<T>(c, L2), c->stream);
+  launch_axis<T>(L2, -1, spec[0], spec[0], az, L1, n, twiddles<T>(c, L2), c->stream);
 }
-template void spectrum_forward_full<double>(osc_ctx*, const double*, cpx<double>*, const SpecDims&,
-                                            const CornerDiff*, const int*, GreenRef*);
-template void spectrum_forward_full<float>(osc_ctx*, const double*, cpx<float>*, const SpecDims&,
-                                           const CornerDiff*, const int*, GreenRef*);
+
+void spectrum_forward_full(osc_ctx* c, const double* g, cpx<double>* spec, const SpecDims& d) {
+  spectra_forward<double>(c, 1, &g, &spec, d, nullptr, nullptr, nullptr);
+}
 
 void convert_spectrum(osc_ctx* c, const cpx<double>* in, cpx<float>* out, int64_t n) {
   ProfScope ps(c, ST_GREEN_FFT);
@@ -830,99 +897,29 @@ static std::string green_key(const osc_ctx* c, const GreenSpec& s, bool fast) {
   return key;
 }
 
-// The real arrays of s's three E components in one kernel, into F (three
-// arrays of the grid, component after component), if the spectra of all three
-// have to be built: the primitives of an FP64 offset-kind specification, the
-// Green functions of a legacy-kind one.  green_spectrum takes them from there.
+// the array of key in the cache, if it is there
 template <typename T>
-bool green_primitives(osc_ctx* c, const GreenSpec& s, DevBuf& F) {
-  if (s.kind == GK_OFFSET ? sizeof(T) == 4 : s.igf == 0) return false;
-  if (c->gcache.enable && !c->green_md)
-    for (int ic = 1; ic <= 3; ++ic) {
-      GreenSpec t = s;
-      t.icomp = ic;
-      auto it = c->gcache.map.find(green_key(c, t, sizeof(T) == 4));
-      if (it != c->gcache.map.end() && (sizeof(T) == 4 ? it->second->f32 : it->second->f64).p) return false;
-    }
-  const int64_t N = int64_t(s.L[0]) * s.L[1] * s.L[2];
-  F = DevBuf(c->pool, sizeof(double) * 3 * N);
-  double* p[3];
-  for (int a = 0; a < 3; ++a) p[a] = F.as<double>() + a * N;
-  ProfScope ps(c, ST_GREEN_EVAL);
-  if (s.kind == GK_OFFSET) launch_prim3(c, s, p);
-  else launch_legacy(c, s, false, p);
+static bool cached_spectrum(osc_ctx* c, const std::string& key, GreenRef& ref) {
+  auto it = c->gcache.map.find(key);
+  if (it == c->gcache.map.end()) return false;
+  GreenCache::Entry& e = *it->second;
+  e.last = ++c->gcache.tick;
+  DevBuf& have = sizeof(T) == 4 ? e.f32 : e.f64;
+  if (!have.p) return false;
+  ref = GreenRef{have.p, e.zr, e.zmh, e.zms};
   return true;
 }
-template bool green_primitives<double>(osc_ctx*, const GreenSpec&, DevBuf&);
-template bool green_primitives<float>(osc_ctx*, const GreenSpec&, DevBuf&);
-
+// gives a built spectrum to the cache, or to keep where it is not admitted
 template <typename T>
-GreenRef green_spectrum(osc_ctx* c, const GreenSpec& s, DevBuf& keepalive, const double* prim) {
-  const SpecDims d = SpecDims::of(s.L);
-  const int64_t N = int64_t(s.L[0]) * s.L[1] * s.L[2];
-  const std::string key = green_key(c, s, sizeof(T) == 4);
+static void store_spectrum(osc_ctx* c, const std::string& key, const GreenRef& ref, DevBuf&& sp,
+                           size_t bytes, DevBuf& keep) {
   GreenCache& gc = c->gcache;
-  GreenCache::Entry* hit = nullptr;
-  // a captured solve builds its spectra on every replay (the spacing is only
-  // known on the device then): no cache
-  const bool use_cache = gc.enable && !c->green_md;
-  if (use_cache) {
-    auto it = gc.map.find(key);
-    if (it != gc.map.end()) {
-      hit = it->second.get();
-      hit->last = ++gc.tick;
-      DevBuf& have = sizeof(T) == 4 ? hit->f32 : hit->f64;
-      if (have.p) {
-        ++gc.hits;
-        return GreenRef{have.p, hit->zr, hit->zmh, hit->zms};
-      }
-    }
-    ++gc.misses;
+  auto it = gc.map.find(key);
+  GreenCache::Entry* ep = it == gc.map.end() ? nullptr : it->second.get();
+  if (!ep && !gc.admit(key)) {
+    keep = std::move(sp);
+    return;
   }
-  DevBuf g(c->pool, prim ? 0 : sizeof(double) * N);
-  double* F = g.as<double>();
-  DevBuf sp(c->pool, sizeof(cpx<T>) * d.size());
-  GreenRef ref{};
-  GreenRef* zr = fft_has_plan(s.L[2]) ? &ref : nullptr;
-  const bool fast = sizeof(T) == 4;  // mirrored quarter-grid primitive (prim_mirrors)
-  if (s.kind == GK_OFFSET && !fft_has_plan(s.L[0])) {
-    // the x pass of a length without a plan differences the primitive on the
-    // whole grid, without far-field cells and mirrored halves
-    if (!prim) {
-      ProfScope ps(c, ST_GREEN_EVAL);
-      build_offset_primitive(c, s, F, fast);
-    }
-    const CornerDiff cd{s.L[1], s.L[2], s.out_shift_z, s.zero_raw};
-    spectrum_forward_full<T>(c, prim ? prim : F, sp.as<cpx<T>>(), d, &cd, nullptr, zr);
-  } else if (s.kind == GK_OFFSET) {
-    // the x pass takes the 8-corner difference of the primitive as it loads
-    // its rows, so the difference array is never stored
-    CornerDiff cd{s.L[1], s.L[2], s.out_shift_z, s.zero_raw};
-    int zlo, zhi;
-    far_field_setup(c, s, fast, cd, zlo, zhi);
-    if (!prim && zlo <= zhi) {
-      ProfScope ps(c, ST_GREEN_EVAL);
-      build_offset_primitive(c, s, F, fast, true, zlo, zhi);
-    }
-    // the corner difference of a primitive that is even along an axis is odd
-    // about L/2 - 1 there, and even where the primitive is odd
-    int mev, mod;
-    prim_mirrors(s, fast, mev, mod);
-    int sym[3] = {0, 0, 0};
-    if (mev >= 0) sym[mev] = -1;
-    if (mod >= 0) sym[mod] = 1;
-    spectrum_forward_full<T>(c, prim ? prim : F, sp.as<cpx<T>>(), d, &cd, sym, zr);
-  } else {
-    if (!prim) build_green_real(c, s, F, fast);
-    spectrum_forward_full<T>(c, prim ? prim : F, sp.as<cpx<T>>(), d, nullptr, nullptr, zr);
-  }
-  g.reset();
-  ref.g = sp.p;
-  if (!use_cache || (!hit && !gc.admit(key))) {
-    keepalive = std::move(sp);
-    return ref;
-  }
-  GreenCache::Entry* ep = hit;
   if (!ep) {
     auto e = std::make_unique<GreenCache::Entry>();
     ep = e.get();
@@ -931,7 +928,6 @@ GreenRef green_spectrum(osc_ctx* c, const GreenSpec& s, DevBuf& keepalive, const
   ep->zr = ref.zr;
   ep->zmh = ref.zmh;
   ep->zms = ref.zms;
-  const size_t bytes = sizeof(cpx<T>) * d.size();
   (sizeof(T) == 4 ? ep->f32 : ep->f64) = std::move(sp);
   ep->bytes += bytes;
   ep->last = ++gc.tick;
@@ -942,10 +938,130 @@ GreenRef green_spectrum(osc_ctx* c, const GreenSpec& s, DevBuf& keepalive, const
     gc.evict_to(gc.max_bytes);
     ep->last = gc.tick;
   }
-  return ref;
 }
-template GreenRef green_spectrum<double>(osc_ctx*, const GreenSpec&, DevBuf&, const double*);
-template GreenRef green_spectrum<float>(osc_ctx*, const GreenSpec&, DevBuf&, const double*);
+
+// Grids up to which the components' transforms run as one pass per axis.  One
+// component's passes leave a small grid with fewer workgroups than CUs: with one
+// pass for the three a step on 32^3 takes 137 us instead of 147, on 48^3 in FP32
+// (with one primitive launch as well) 173 instead of 200.  On a large one the y
+// pass then finds its input in memory, where each component's own x pass had
+// left it in the 256 MB cache: 128^3 1999 us instead of 1975, 128x128x256 at the
+// cathode 4607 instead of 4513.
+constexpr int64_t kBatchGrid = int64_t(1) << 22;
+
+// The spectra of n components icomp[] of s that are in no cache: one kernel for
+// their real arrays where the kind has one; transforms together (kBatchGrid).
+template <typename T>
+static void build_spectra(osc_ctx* c, const GreenSpec& s, int n, const int icomp[], DevBuf sp[],
+                          GreenRef* const ref[]) {
+  const SpecDims d = SpecDims::of(s.L);
+  const int64_t N = int64_t(s.L[0]) * s.L[1] * s.L[2];
+  DevBuf real(c->pool, sizeof(double) * N * n);
+  double* g[3];
+  cpx<T>* spec[3];
+  for (int q = 0; q < n; ++q) {
+    g[q] = real.as<double>() + q * N;
+    sp[q] = DevBuf(c->pool, sizeof(cpx<T>) * d.size());
+    spec[q] = sp[q].as<cpx<T>>();
+    ref[q]->g = spec[q];
+  }
+  GreenRef* const* zr = fft_has_plan(s.L[2]) ? ref : nullptr;
+  const bool fast = sizeof(T) == 4;  // mirrored quarter-grid primitive (prim_mirrors)
+  auto forward = [&](const CornerDiff* cd, const int (*sym)[3]) {
+    const int step = N <= kBatchGrid ? n : 1;
+    for (int q = 0; q < n; q += step)
+      spectra_forward<T>(c, step, g + q, spec + q, d, cd ? cd + q : nullptr, sym ? sym + q : nullptr,
+                         zr ? zr + q : nullptr);
+  };
+  if (s.kind != GK_OFFSET) {
+    if (s.igf != 0 && icomp[0] >= 1 && s.kind != GK_PIPE) {
+      double* G[3] = {nullptr, nullptr, nullptr};
+      for (int q = 0; q < n; ++q) G[icomp[q] - 1] = g[q];
+      ProfScope ps(c, ST_GREEN_EVAL);
+      launch_legacy(c, s, false, G);
+    } else {
+      for (int q = 0; q < n; ++q) {
+        GreenSpec t = s;
+        t.icomp = icomp[q];
+        build_green_real(c, t, g[q], fast);
+      }
+    }
+    forward(nullptr, nullptr);
+    return;
+  }
+  // the x pass takes the 8-corner difference of the primitive as it loads its
+  // rows, so the difference array is never stored; the one of a length without
+  // a plan differences it on the whole grid, without far-field cells and
+  // mirrored halves
+  const bool plan = fft_has_plan(s.L[0]);
+  CornerDiff cd[3];
+  int sym[3][3] = {};
+  int zlo = 0, zhi = s.L[2] - 1;
+  for (int q = 0; q < n; ++q) {
+    GreenSpec t = s;
+    t.icomp = icomp[q];
+    cd[q] = CornerDiff{s.L[1], s.L[2], s.out_shift_z, s.zero_raw};
+    if (!plan) continue;
+    far_field_setup(c, t, fast, cd[q], zlo, zhi);
+    // the corner difference of a primitive that is even along an axis is odd
+    // about L/2 - 1 there, and even where the primitive is odd
+    int mev, mod;
+    prim_mirrors(t, fast, mev, mod);
+    if (mev >= 0) sym[q][mev] = -1;
+    if (mod >= 0) sym[q][mod] = 1;
+  }
+  if (zlo <= zhi) {
+    ProfScope ps(c, ST_GREEN_EVAL);
+    build_offset_primitives(c, s, n, icomp, g, fast, plan, zlo, zhi);
+  }
+  forward(cd, plan ? sym : nullptr);
+}
+
+template <typename T>
+void green_spectra(osc_ctx* c, const GreenSpec& s, int n, const int icomp[], DevBuf* const keep[],
+                   GreenRef out[]) {
+  OSC_REQUIRE(n >= 1 && n <= 3, OSC_ERR_ARG, "bad batch");
+  const int64_t N = int64_t(s.L[0]) * s.L[1] * s.L[2];
+  // a captured solve builds its spectra on every replay (the spacing is only
+  // known on the device then): no cache
+  const bool use_cache = c->gcache.enable && !c->green_md;
+  std::string key[3];
+  int want[3], m = 0;
+  for (int q = 0; q < n; ++q) {
+    GreenSpec t = s;
+    t.icomp = icomp[q];
+    key[q] = green_key(c, t, sizeof(T) == 4);
+    if (use_cache && cached_spectrum<T>(c, key[q], out[q])) {
+      ++c->gcache.hits;
+      continue;
+    }
+    if (use_cache) ++c->gcache.misses;
+    want[m++] = q;
+  }
+  // together: kernels that form the components together anyway, and small grids
+  // (build_spectra; on large ones FP32 builds need a third of the real arrays
+  // one at a time)
+  const bool shared = icomp[0] >= 1 && (s.kind == GK_OFFSET ? sizeof(T) == 8 : s.igf != 0);
+  const int step = shared || N <= kBatchGrid ? 3 : 1;
+  for (int f = 0; f < m; f += step) {
+    const int nb = std::min(step, m - f);
+    int ic[3];
+    DevBuf sp[3];
+    GreenRef* ref[3];
+    for (int q = 0; q < nb; ++q) {
+      ic[q] = icomp[want[f + q]];
+      ref[q] = &out[want[f + q]];
+    }
+    build_spectra<T>(c, s, nb, ic, sp, ref);
+    const size_t bytes = sizeof(cpx<T>) * SpecDims::of(s.L).size();
+    for (int q = 0; q < nb; ++q) {
+      if (use_cache) store_spectrum<T>(c, key[want[f + q]], *ref[q], std::move(sp[q]), bytes, *keep[want[f + q]]);
+      else *keep[want[f + q]] = std::move(sp[q]);
+    }
+  }
+}
+template void green_spectra<double>(osc_ctx*, const GreenSpec&, int, const int[], DevBuf* const[], GreenRef[]);
+template void green_spectra<float>(osc_ctx*, const GreenSpec&, int, const int[], DevBuf* const[], GreenRef[]);
 
 // full upstream array F_s[g](k) = F_-[g](sigma_s k), sigma flipping axes with s=+1
 void half_to_upstream(osc_ctx* c, const cpx<double>* spec_dev, const SpecDims& d, const int s[3],

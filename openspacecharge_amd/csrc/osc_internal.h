@@ -255,7 +255,7 @@ struct osc_ctx {
   bool kept_ok = false;
   std::unique_ptr<osc::HostRing> ring;  // pageable host transfers (created on first use)
   void* counters = nullptr;  // small device scratch for counters (persistent)
-  void* fast_tab = nullptr;  // the FastMathTab of fast_math.h, behind the counters
+  const void* fast_tab = nullptr;  // fast_table(device)
   osc::MeshDev* mesh_host = nullptr;  // pinned copy of the device mesh
   hipEvent_t mesh_ev = nullptr;        // recorded after the copy is queued
   // pinned copies of the deposit's and the query's content hashes (in the
@@ -410,26 +410,20 @@ class HostRing {
 bool is_pageable(const void* p);
 
 // ---- green.hip --------------------------------------------------------------
+// the device's copy of the FastMathTab of fast_math.h (a constant, written once
+// per device, when its first context is created); null: a HIP error
+const void* fast_table(int device);
 void build_green_real(osc_ctx* c, const GreenSpec& s, double* g, bool fast = false);  // (L0,L1,L2) real
 // the half spectrum of one pipe Green term from its separable form
 void pipe_spectrum(osc_ctx* c, const GreenSpec& s, const SpecDims& d, cpx<double>* spec);
-// spectrum of a Green function in precision T (z-real when the z length has a
-// compile-time plan); cached by spec
+// spectra of the n <= 3 components icomp[] of s's Green functions in precision T
+// (z-real when the z length has a compile-time plan); cached by spec, or left
+// in *keep[q]
 template <typename T>
-GreenRef green_spectrum(osc_ctx* c, const GreenSpec& s, DevBuf& keepalive,
-                        const double* prim = nullptr);
-// the primitives of s's three E components for green_spectrum's prim (one
-// array of the grid each), where that pays; false: none
-template <typename T>
-bool green_primitives(osc_ctx* c, const GreenSpec& s, DevBuf& F);
-// forward R2C of a real (L0,L1,L2) FP64 array into a half spectrum of precision T
-// (with cd: g is a primitive and the x pass takes its corner difference;
-// sym: per-axis mirror symmetry of that difference, 0 / +1 even / -1 odd;
-// with zr: the z pass is left out and *zr describes the stored z lines)
-template <typename T>
-void spectrum_forward_full(osc_ctx* c, const double* g, cpx<T>* spec, const SpecDims& d,
-                           const CornerDiff* cd = nullptr, const int* sym = nullptr,
-                           GreenRef* zr = nullptr);
+void green_spectra(osc_ctx* c, const GreenSpec& s, int n, const int icomp[], DevBuf* const keep[],
+                   GreenRef out[]);
+// forward R2C of a real (L0,L1,L2) array into a half spectrum
+void spectrum_forward_full(osc_ctx* c, const double* g, cpx<double>* spec, const SpecDims& d);
 void convert_spectrum(osc_ctx* c, const cpx<double>* in, cpx<float>* out, int64_t n);
 // download a half spectrum and expand it to the upstream full-array
 // convention F_s[g] (sign s[d] on axis d)

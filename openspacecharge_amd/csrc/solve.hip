@@ -121,7 +121,11 @@ void conv_solve(osc_ctx* c, const double* rho, const int n[3], const SpecDims& d
   DevBuf S(c->pool, sizeof(cpx<T>) * d.size());
   cpx<T>* sp = S.as<cpx<T>>();
   // forward: x (rows y<ny, z<nz), y (planes z<nz), z (all rows)
-  R2CIO r{};
+  R2CBatch<T> rb{};
+  rb.n = 1;
+  rb.in[0] = rho;
+  rb.out[0] = sp;
+  R2CIO& r = rb.a[0];
   r.in_sy = nx;
   r.in_sz = int64_t(nx) * ny;
   r.out_sy = KXP;
@@ -131,7 +135,7 @@ void conv_solve(osc_ctx* c, const double* rho, const int n[3], const SpecDims& d
   r.n_in = nx;
   {
     ProfScope ps(c, ST_FWD_X);
-    launch_xr2c<T>(L0, rho, sp, r, twiddles<T>(c, L0), s);
+    launch_xr2c<T>(L0, rb, false, twiddles<T>(c, L0), s);
   }
   AxisIO ay{};
   ay.s_b = ay.d_b = 1;

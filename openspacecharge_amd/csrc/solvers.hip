@@ -85,26 +85,26 @@ struct Specs {
   Specs(const Specs&) = delete;
   Specs& operator=(const Specs&) = delete;
   GreenRef get(osc_ctx* c, const GreenSpec& s, size_t slot) {
-    if (!pinned) {
-      pinned = c;
-      c->gcache.pin();
-    }
-    return green_spectrum<T>(c, s, keep[slot]);
+    pin(c);
+    DevBuf* k[1] = {&keep[slot]};
+    GreenRef r;
+    green_spectra<T>(c, s, 1, &s.icomp, k, &r);
+    return r;
   }
   // the three E components of the offset- or legacy-kind specification s, in slots
   // slot .. slot + 2
-  void get3(osc_ctx* c, GreenSpec s, size_t slot, GreenRef out[3]) {
-    if (!pinned) {
-      pinned = c;
-      c->gcache.pin();
-    }
-    DevBuf F;
-    const int64_t N = int64_t(s.L[0]) * s.L[1] * s.L[2];
-    const double* p = green_primitives<T>(c, s, F) ? F.as<const double>() : nullptr;
-    for (int a = 0; a < 3; ++a) {
-      s.icomp = a + 1;
-      out[a] = green_spectrum<T>(c, s, keep[slot + a], p ? p + a * N : nullptr);
-    }
+  void get3(osc_ctx* c, const GreenSpec& s, size_t slot, GreenRef out[3]) {
+    pin(c);
+    const int ic[3] = {1, 2, 3};
+    DevBuf* k[3] = {&keep[slot], &keep[slot + 1], &keep[slot + 2]};
+    green_spectra<T>(c, s, 3, ic, k, out);
+  }
+
+ private:
+  void pin(osc_ctx* c) {
+    if (pinned) return;
+    pinned = c;
+    c->gcache.pin();
   }
 };
 
