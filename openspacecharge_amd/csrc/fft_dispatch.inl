@@ -71,10 +71,13 @@ void xr2c_t(const R2CBatch<T>& b, bool diff, const cpx<T>* tw, hipStream_t s) {
 template <int L>
 void xc2r_t(const cpx<T>* in, const C2RIO<T>& a, int nout, const cpx<T>* tw, hipStream_t s) {
   constexpr int BX = XGeo<T, L>::BX, NT = XGeo<T, L>::NT;
-  if (a.npair > 0)
-    launch((k_xc2r<T, L, true>), grid3(cdiv(a.nrows, BX), a.npair, 1), dim3(NT), 0, s, in, a, tw);
-  else
-    launch((k_xc2r<T, L, false>), grid3(cdiv(cdiv(a.nrows, 2), BX), nout, 1), dim3(NT), 0, s, in, a, tw);
+  if constexpr (sizeof(T) == 8) {  // pairs of parts: FP64 image solves
+    if (a.npair > 0) {
+      launch((k_xc2r<T, L, true>), grid3(cdiv(a.nrows, BX), a.npair, 1), dim3(NT), 0, s, in, a, tw);
+      return;
+    }
+  }
+  launch((k_xc2r<T, L, false>), grid3(cdiv(cdiv(a.nrows, 2), BX), nout, 1), dim3(NT), 0, s, in, a, tw);
 }
 // k_zconv's per-thread byte offsets (line b < BX, position t < TPL of a
 // column block) must fit in 32 bits

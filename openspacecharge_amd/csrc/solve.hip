@@ -153,7 +153,10 @@ void conv_solve(osc_ctx* c, const double* rho, const int n[3], const SpecDims& d
   // rho_hat's z pass inside the multiply (once per column for all outputs)
   ZinvIO<T> zs{};
   zs.sz = zs.o_sz = KXP * L1;
-  bool zconv = fft_has_plan(L2) && zconv_fits<T>(L2, zs), two = zconv;
+  // An FP32 solve adds its terms over full spectra (k_zinv): results leave as
+  // doubles that callers compare between runs, and the two phases' order of
+  // sums moves them by the convolution's rounding, 5e-7 of the largest value
+  bool zconv = fft_has_plan(L2) && zconv_fits<T>(L2, zs), two = zconv && sizeof(T) == 8;
   for (const OutSpec& os : outs) {
     zconv = zconv && os.nt == 1 && os.t[0].mir == 0 && os.t[0].g.zr;
     // ... as do sums of such a term and an image term mirrored in z (two phases)
