@@ -533,7 +533,8 @@ OSC_API int osc_space_charge_step(osc_ctx* c, int64_t n, const double* xa, const
         ia.mn[d] = m->min[d];
         ia.delta[d] = m->delta[d];
       }
-      interpolate_sorted(c, ia, e, b, sp, Eo, Bo, nullptr, nullptr, x, y, z);
+      interpolate_sorted(c, ia, e, b, sp, Eo, Bo, nullptr, nullptr, x, y, z,
+                         sc3d_bform(m->gamma, at_cathode));
     }
     if (n_dropped) *n_dropped = read_counter(c, 0);
     if (n_clamped) *n_clamped = read_counter(c, 2);

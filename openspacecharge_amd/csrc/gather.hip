@@ -30,6 +30,21 @@ __device__ __forceinline__ int clamp_idx(double x, double mn, double hinv, int n
   return ip;
 }
 
+// component c (E, then B) at node g of the planar fields, nt nodes each
+template <typename A>
+__device__ __forceinline__ A field_at(const double* __restrict__ ef, const double* __restrict__ bf,
+                                      const BForm& f, int c, int64_t nt, int64_t g) {
+  if (c >= 3 && f.kind == B_FROM_E) return A(c == 3 ? -f.bc * ef[nt + g] : f.bc * ef[g]);
+  return A((c < 3 ? ef : bf)[(c % 3) * nt + g]);
+}
+
+// the gathered value of a component that is 0 at every node: 0, NaN where a
+// weight is not finite
+template <typename A>
+__device__ __forceinline__ A zero_sum(A ab, A de, A gh) {
+  return A(0) * ab + A(0) * de + A(0) * gh + A(0);
+}
+
 __device__ __forceinline__ double interp8(const double* __restrict__ F, int64_t sy, int64_t sz,
                                           int64_t b, double ab, double de, double gh) {
   // E = sum of 8 terms in the upstream order (:369-376)
@@ -626,25 +641,29 @@ __global__ void __launch_bounds__(kThreads)
 // ---------------------------------------------------------------------------
 // tile gather: the particles of the tiled deposit, in bin order
 // ---------------------------------------------------------------------------
-// Geometry of the tile gather.  Tiles of 8^3 cells (729 nodes) take 40 KB of
-// LDS (FP32: 20 KB), so that three (seven) workgroups of 256 share a CU and
-// one's node loads overlap another's sums, in items down to 512 particles;
-// larger tiles need most of the LDS for one workgroup of 1024.
-template <bool F32, bool SMALL>
+// Geometry of the tile gather, NS values of LDS per node.  Tiles of 8^3 cells
+// (729 nodes) take up to 40 KB of LDS (FP32: 20 KB), so that three (seven)
+// workgroups of 256 or more share a CU and one's node loads overlap another's
+// sums, in items down to 512 particles; larger tiles go by workgroups of 1024,
+// one per CU with five or more FP64 values a node, two with three or in FP32.
+template <bool F32, bool SMALL, int NS>
 struct TileGatherGeo {
-  static constexpr int T = SMALL ? 256 : 1024;
-  static constexpr int PER = SMALL ? 2 : 4;  // particles in flight per thread
+  // LDS for two workgroups of a larger tile
+  static constexpr bool TWO = !SMALL && (F32 || NS < 5);
+  static constexpr int T = SMALL ? 256 : (TWO && !F32 ? 512 : 1024);
+  static constexpr int PER = SMALL || TWO ? 2 : 4;             // particles in flight per thread
+  static constexpr int WAVES = F32 ? (SMALL ? 6 : 8) : 4;      // per SIMD
   static constexpr int kNodes = 729;         // most nodes of a SMALL tile
-  static constexpr int kBytes = SMALL ? (kNodes * 7 * (F32 ? 4 : 8) + 7) / 8 * 8
-                                      : (F32 ? kTileGatherBytes32 : kTileGatherBytes64);
+  static constexpr int kBytes = SMALL ? (kNodes * NS * (F32 ? 4 : 8) + 7) / 8 * 8
+                                      : (F32 ? kTileGatherBytes32 : kTileGatherBytes64) / 7 * NS / 8 * 8 + 8;
   static_assert(512 % (T * PER) == 0 || kTileGatherChunk % (T * PER) == 0, "whole rounds");
 };
 constexpr int kTileGatherStage = 512;
 
-// One workgroup per gather item (gchunk particles of one tile's bin): the E
-// and B values of the tile's nodes are staged in LDS as node records of 7
-// values (FP64; F32: the values of the FP32 node records; the odd stride in
-// 4-byte words spreads random nodes over the LDS banks), then each particle
+// One workgroup per gather item (gchunk particles of one tile's bin): NF values
+// of each of the tile's nodes are staged in LDS as node records (FP64; F32: the
+// values of the FP32 node records; the odd stride NS spreads random nodes over
+// the LDS banks), then each particle
 // sums its 8 nodes from there in the upstream order and leaves its values (E
 // and B, or the one asked for) at its slot of out, in bin order: contiguous
 // stores, which k_tile_return takes to particle order.  (Storing each result
@@ -655,16 +674,29 @@ constexpr int kTileGatherStage = 512;
 // k_interp_cells32.  Tiles holding fewer than kTileGatherStage particles, and
 // particles whose cell lies outside the tile (a gather mesh other than the
 // deposit's), read the planar fields.
-template <bool F32, bool SMALL, int NV>
-__global__ void __launch_bounds__((TileGatherGeo<F32, SMALL>::T))
-    k_tile_gather(const double* __restrict__ ef, const double* __restrict__ bf, TileParams tg,
+//
+// NV = 6: E and B; 3: one of the two; 5: E, Bx and By of a B field known to
+// have no z part (BForm), where NF = 3 is the FP64 gather of a B field formed
+// from E: each node's products are those that stored B, so the sums are the
+// same, from half the LDS.
+//
+// Bound by LDS reads at random nodes and by the waves there are to hide them.
+// With 64 registers (FP32: the loads of a component at a time, the planar
+// branch rolled) or half the LDS (FP64, three values) two workgroups share a
+// CU, one staging while the other sums: 128^3, 10^7 particles, E and B: FP64
+// 329 -> 212 us, FP32 266 -> 187 us.  FP64 in 64 registers spills: 560 us.
+constexpr int tile_gather_stride(int nf) { return nf + 1 - nf % 2; }
+template <bool F32, bool SMALL, int NV, int NF>
+__global__ void __launch_bounds__((TileGatherGeo<F32, SMALL, tile_gather_stride(NF)>::T),
+                                  (TileGatherGeo<F32, SMALL, tile_gather_stride(NF)>::WAVES))
+    k_tile_gather(const double* __restrict__ ef, const double* __restrict__ bf, BForm bform, TileParams tg,
                   int gchunk, const TilePlan* __restrict__ tp, const uint32_t* __restrict__ total,
                   const double4* __restrict__ srec, const uint32_t* __restrict__ sk, IP p,
                   typename std::conditional<F32, float, double>::type* __restrict__ out,
                   uint32_t* __restrict__ nclamp) {
   using A = typename std::conditional<F32, float, double>::type;
-  using G = TileGatherGeo<F32, SMALL>;
-  constexpr int NS = 7;  // LDS values per node record
+  constexpr int NS = tile_gather_stride(NF);
+  using G = TileGatherGeo<F32, SMALL, NS>;
   constexpr int T = G::T, PER = G::PER;
   __shared__ double lds_raw[G::kBytes / 8];
   __shared__ int s_t;
@@ -700,11 +732,11 @@ __global__ void __launch_bounds__((TileGatherGeo<F32, SMALL>::T))
       const int gi = ox + li, gj = oy + lj, gk = oz + lk;
       const bool in = gi < p.nn[0] && gj < p.nn[1] && gk < p.nn[2];
       const int64_t g = in ? gi + sy * gj + sz * gk : 0;
-      A v[NV];
+      A v[NF];
 #pragma unroll
-      for (int c = 0; c < NV; ++c) v[c] = A(in ? (c < 3 ? ef : bf)[(c % 3) * nt + g] : 0.0);
+      for (int c = 0; c < NF; ++c) v[c] = in ? field_at<A>(ef, bf, bform, c, nt, g) : A(0);
 #pragma unroll
-      for (int c = 0; c < NV; ++c) L[NS * node + c] = v[c];
+      for (int c = 0; c < NF; ++c) L[NS * node + c] = v[c];
     }
     __syncthreads();
   }
@@ -764,30 +796,35 @@ __global__ void __launch_bounds__((TileGatherGeo<F32, SMALL>::T))
       }
       mine += fl ? 1u : 0u;
       const int li = i0 - ox, lj = j0 - oy, lk = k0 - oz;
-      A v[NV];
       if (staged && li >= 0 && li < wx && lj >= 0 && lj < wy && lk >= 0 && lk < wz) {
         const int q0 = li + tn0 * lj + tn01 * lk;
 #pragma unroll
         for (int c = 0; c < NV; ++c)
-          v[c] = wsum8_any<A>(
+          out[NV * s + c] = wsum8_any<A>(
               [&](int r2, int d) {
-                return L[NS * (q0 + d + ((r2 & 1) ? tn0 : 0) + ((r2 & 2) ? tn01 : 0)) + c];
+                const A* q = L + NS * (q0 + d + ((r2 & 1) ? tn0 : 0) + ((r2 & 2) ? tn01 : 0));
+                if (c < NF) return q[c];
+                return c == 3 ? A(-bform.bc) * q[1] : A(bform.bc) * q[0];
               },
               ab, de, gh);
       } else {
         const int64_t b = i0 + sy * j0 + sz * k0;
-#pragma unroll
-        for (int c = 0; c < NV; ++c) {
-          const double* F = (c < 3 ? ef : bf) + (c % 3) * nt;
-          v[c] = wsum8_any<A>(
+        auto planar = [&](int c) {
+          out[NV * s + c] = wsum8_any<A>(
               [&](int r2, int d) {
-                return A(F[b + d + ((r2 & 1) ? sy : 0) + ((r2 & 2) ? sz : 0)]);
+                return field_at<A>(ef, bf, bform, c, nt,
+                                   b + d + ((r2 & 1) ? sy : 0) + ((r2 & 2) ? sz : 0));
               },
               ab, de, gh);
+        };
+        if constexpr (SMALL) {  // many tiles of small meshes: the loads overlap
+#pragma unroll
+          for (int c = 0; c < NV; ++c) planar(c);
+        } else {  // rare: few registers
+#pragma clang loop unroll(disable)
+          for (int c = 0; c < NV; ++c) planar(c);
         }
       }
-#pragma unroll
-      for (int c = 0; c < NV; ++c) out[NV * s + c] = v[c];
     }
   }
   if (mine) atomicAdd(&cnt, mine);
@@ -798,25 +835,29 @@ __global__ void __launch_bounds__((TileGatherGeo<F32, SMALL>::T))
 // The results of k_tile_gather (val, NV values per slot) in particle order:
 // each wave reads the records of 64 consecutive particles (their slots from
 // pos; a scatter block's particles of one bin lie side by side, so the lines
-// are shared by the waves around) into LDS and stores them as contiguous runs
+// are shared by the waves around; NV lanes read a record, so that a load
+// touches a few lines instead of one per lane: FP64 237 -> 220 us at 10^7
+// particles, FP32 the same 197) into LDS and stores them as contiguous runs
 // of E and B.  A particle of the off-mesh bin (slots from bstart[ntiles] on)
 // has no value there: it takes the interpolate_field clamp rule from its
 // coordinates here, the planar fields read directly (FP32: the weights
 // rounded as in k_interp_cells32).  Flags, where asked for: FP64 by the
 // clamp rule from the coordinates, F32 (the deposit's own mesh) the off-mesh
-// particles'.  E or B null: val holds the other's three values.
+// particles'.  E or B null: val holds the other's three values.  NV = 5: Bz is
+// 0; a particle whose weights are not finite has NaN in all its values, and
+// then in Bz too.
 template <bool F32, int NV>
 __global__ void __launch_bounds__(kThreads)
     k_tile_return(const typename std::conditional<F32, float, double>::type* __restrict__ val,
                   const uint32_t* __restrict__ pos, int64_t n, const double* __restrict__ ef,
-                  const double* __restrict__ bf, int ntiles, const TilePlan* __restrict__ tp,
-                  const double* __restrict__ x, const double* __restrict__ y,
+                  const double* __restrict__ bf, BForm bform, int ntiles,
+                  const TilePlan* __restrict__ tp, const double* __restrict__ x, const double* __restrict__ y,
                   const double* __restrict__ z, IP p, double* __restrict__ E,
                   double* __restrict__ B, int8_t* __restrict__ clamped,
                   uint32_t* __restrict__ nclamp) {
   using A = typename std::conditional<F32, float, double>::type;
   // an odd stride in 4-byte (FP64: 8-byte) words against bank conflicts
-  constexpr int NP = NV + 1 - NV % 2;
+  constexpr int NW = NV == 5 ? 6 : NV, NP = NW + 1 - NW % 2;
   __shared__ A stage[kThreads / 64][64 * NP];
   const int lane = threadIdx.x & 63;
   A* w = stage[threadIdx.x >> 6];
@@ -826,24 +867,45 @@ __global__ void __launch_bounds__(kThreads)
        i0 += int64_t(gridDim.x) * blockDim.x) {  // uniform per wave
     const int nrec = n - i0 < 64 ? int(n - i0) : 64;
     const int64_t i = i0 + lane;
-    bool fl = false, outside = false;
-    if (lane < nrec) {
-      const uint32_t s = pos[i];
-      outside = s >= off;
-      A v[NV];
-      if (!outside) {
+    bool fl = false;
+    // the slots' records, NV lanes to each
+    const uint32_t mine = lane < nrec ? pos[i] : off;
+    A got[NV];
 #pragma unroll
-        for (int c = 0; c < NV; ++c) v[c] = val[int64_t(NV) * s + c];
+    for (int k = 0; k < NV; ++k) {
+      const int e = lane + 64 * k, r = e / NV;
+      const uint32_t s = __shfl(mine, r);
+      got[k] = val[s < off ? int64_t(NV) * s + (e - r * NV) : 0];
+    }
+#pragma unroll
+    for (int k = 0; k < NV; ++k) {
+      const int e = lane + 64 * k, r = e / NV;
+      w[NP * r + e - r * NV] = got[k];
+    }
+    wave_lds_sync();
+    const bool outside = lane < nrec && mine >= off;
+    if (lane < nrec) {
+      A* v = w + NP * lane;
+      bool none = NV == 5;  // every value NaN
+      if (!outside) {
+        if constexpr (NV == 5) {
+#pragma unroll
+          for (int c = 0; c < NV; ++c) none = none && v[c] != v[c];
+          v[5] = A(0);
+        }
         if (!F32 && clamped) {
           (void)clamp_idx(x[i], p.mn[0], p.hinv[0], p.nhi[0], fl);
           (void)clamp_idx(y[i], p.mn[1], p.hinv[1], p.nhi[1], fl);
           (void)clamp_idx(z[i], p.mn[2], p.hinv[2], p.nhi[2], fl);
         }
-      } else {
+      }
+      if (outside || none) {
         const double xi = x[i], yi = y[i], zi = z[i];
-        const int ip = clamp_idx(xi, p.mn[0], p.hinv[0], p.nhi[0], fl);
-        const int jp = clamp_idx(yi, p.mn[1], p.hinv[1], p.nhi[1], fl);
-        const int kp = clamp_idx(zi, p.mn[2], p.hinv[2], p.nhi[2], fl);
+        bool f2 = false;
+        const int ip = clamp_idx(xi, p.mn[0], p.hinv[0], p.nhi[0], f2);
+        const int jp = clamp_idx(yi, p.mn[1], p.hinv[1], p.nhi[1], f2);
+        const int kp = clamp_idx(zi, p.mn[2], p.hinv[2], p.nhi[2], f2);
+        fl = fl || (outside && f2);
         const A ab = A(((p.mn[0] - xi) + ip * p.delta[0]) * p.hinv[0]);
         const A de = A(((p.mn[1] - yi) + jp * p.delta[1]) * p.hinv[1]);
         const A gh = A(((p.mn[2] - zi) + kp * p.delta[2]) * p.hinv[2]);
@@ -852,18 +914,17 @@ __global__ void __launch_bounds__(kThreads)
         jj = jj < 0 ? 0 : (jj > p.nn[1] - 2 ? p.nn[1] - 2 : jj);
         kk = kk < 0 ? 0 : (kk > p.nn[2] - 2 ? p.nn[2] - 2 : kk);
         const int64_t b = ii + sy * jj + sz * kk;
-#pragma unroll
-        for (int c = 0; c < NV; ++c) {
-          const double* F = (c < 3 ? ef : bf) + (c % 3) * nt;
-          v[c] = wsum8_any<A>(
-              [&](int rr, int d) {
-                return A(F[b + d + ((rr & 1) ? sy : 0) + ((rr & 2) ? sz : 0)]);
-              },
-              ab, de, gh);
-        }
+        if (outside)
+#pragma clang loop unroll(disable)
+          for (int c = 0; c < NV; ++c)
+            v[c] = wsum8_any<A>(
+                [&](int rr, int d) {
+                  return field_at<A>(ef, bf, bform, c, nt,
+                                     b + d + ((rr & 1) ? sy : 0) + ((rr & 2) ? sz : 0));
+                },
+                ab, de, gh);
+        if constexpr (NV == 5) v[5] = zero_sum<A>(ab, de, gh);
       }
-#pragma unroll
-      for (int c = 0; c < NV; ++c) w[NP * lane + c] = v[c];
       if (clamped) clamped[i] = fl ? 1 : 0;
     }
     // the clamped off-mesh particles (k_tile_gather counts its own)
@@ -876,7 +937,7 @@ __global__ void __launch_bounds__(kThreads)
       const int e = lane + 64 * k;  // value of the chunk: record e / 3, component e % 3
       if (e / 3 < nrec) first[3 * i0 + e] = double(w[(e / 3) * NP + e % 3]);
     }
-    if constexpr (NV == 6)
+    if constexpr (NW == 6)
 #pragma unroll
       for (int k = 0; k < 3; ++k) {
         const int e = lane + 64 * k;
@@ -887,9 +948,9 @@ __global__ void __launch_bounds__(kThreads)
 }
 
 // gather of a tiled deposit's particles: k_tile_gather, k_tile_return
-template <bool F32, int NV>
+template <bool F32, int NV, int NF>
 void tile_gather(osc_ctx* c, const SortedParticles& sp, const double* ef, const double* bf,
-                 const IP& p, const double* x, const double* y, const double* z, double* E,
+                 const BForm& bform, const IP& p, const double* x, const double* y, const double* z, double* E,
                  double* B, int8_t* clamped, uint32_t* cnt) {
   using A = typename std::conditional<F32, float, double>::type;
   const int64_t n = sp.n;
@@ -901,11 +962,14 @@ void tile_gather(osc_ctx* c, const SortedParticles& sp, const double* ef, const 
     ProfScope ps(c, ST_GATHER);
     // at most one partial chunk per tile beyond the full ones
     const int64_t items = (n + sp.gchunk - 1) / sp.gchunk + sp.tile.ntiles;
-    const bool small = sp.tile.nodes <= TileGatherGeo<F32, true>::kNodes;
-    hipLaunchKernelGGL((small ? k_tile_gather<F32, true, NV> : k_tile_gather<F32, false, NV>),
+    constexpr int NS = tile_gather_stride(NF);
+    const bool small = sp.tile.nodes <= TileGatherGeo<F32, true, NS>::kNodes;
+    OSC_REQUIRE(small || size_t(sp.tile.nodes) * NS * sizeof(A) <= size_t(TileGatherGeo<F32, false, NS>::kBytes),
+                OSC_ERR_ARG, "tile gather: tile too large");
+    hipLaunchKernelGGL((small ? k_tile_gather<F32, true, NV, NF> : k_tile_gather<F32, false, NV, NF>),
                        dim3(unsigned(items)),
-                       dim3(small ? TileGatherGeo<F32, true>::T : TileGatherGeo<F32, false>::T), 0,
-                       c->stream, f0, bf, sp.tile, sp.gchunk, tpl, sp.total.as<const uint32_t>(),
+                       dim3(small ? TileGatherGeo<F32, true, NS>::T : TileGatherGeo<F32, false, NS>::T), 0,
+                       c->stream, f0, bf, bform, sp.tile, sp.gchunk, tpl, sp.total.as<const uint32_t>(),
                        sp.srec.as<const double4>(), sp.sk.as<const uint32_t>(), p, val.as<A>(),
                        cnt);
     OSC_HIP(hipGetLastError());
@@ -913,7 +977,7 @@ void tile_gather(osc_ctx* c, const SortedParticles& sp, const double* ef, const 
   ProfScope po(c, ST_GATHER_OUT);
   const int64_t nb = std::min<int64_t>((n + kThreads - 1) / kThreads, 65536 * 8);
   hipLaunchKernelGGL((k_tile_return<F32, NV>), dim3(unsigned(nb)), dim3(kThreads), 0, c->stream,
-                     val.as<const A>(), sp.sv.as<const uint32_t>(), n, f0, bf, sp.tile.ntiles, tpl,
+                     val.as<const A>(), sp.sv.as<const uint32_t>(), n, f0, bf, bform, sp.tile.ntiles, tpl,
                      x, y, z, p, E, B, clamped, cnt);
   OSC_HIP(hipGetLastError());
 }
@@ -932,7 +996,7 @@ void pack_nodes(osc_ctx* c, const InterpArgs& a, const double* ef, const double*
 void interpolate_sorted(osc_ctx* c, const InterpArgs& a, const double* ef, const double* bf,
                         const SortedParticles& sp, double* E, double* B, int8_t* clamped,
                         const double* packed, const double* x, const double* y,
-                        const double* z) {
+                        const double* z, BForm bform) {
   IP p{};
   for (int d = 0; d < 3; ++d) {
     p.mn[d] = a.mn[d];
@@ -959,12 +1023,18 @@ void interpolate_sorted(osc_ctx* c, const InterpArgs& a, const double* ef, const
       OSC_HIP(hipGetLastError());
       return;
     }
-    if (Eo && Bo)
-      (sp.f32 ? tile_gather<true, 6> : tile_gather<false, 6>)(c, sp, ef, bf, p, x, y, z, Eo, Bo,
-                                                              clamped, cnt);
+    const BForm any{B_ANY, 0.0};
+    if (!Eo || !Bo)
+      (sp.f32 ? tile_gather<true, 3, 3> : tile_gather<false, 3, 3>)(c, sp, ef, bf, any, p, x, y, z, Eo, Bo,
+                                                                    clamped, cnt);
+    else if (bform.kind == B_ANY)
+      (sp.f32 ? tile_gather<true, 6, 6> : tile_gather<false, 6, 6>)(c, sp, ef, bf, any, p, x, y, z, Eo, Bo,
+                                                                    clamped, cnt);
+    else if (sp.f32 || bform.kind == B_TRANSVERSE)
+      (sp.f32 ? tile_gather<true, 5, 5> : tile_gather<false, 5, 5>)(c, sp, ef, bf, bform, p, x, y, z, Eo, Bo,
+                                                                    clamped, cnt);
     else
-      (sp.f32 ? tile_gather<true, 3> : tile_gather<false, 3>)(c, sp, ef, bf, p, x, y, z, Eo, Bo,
-                                                              clamped, cnt);
+      tile_gather<false, 5, 3>(c, sp, ef, bf, bform, p, x, y, z, Eo, Bo, clamped, cnt);
     return;
   }
   if (!packed && sp.n < 2 * nt) {

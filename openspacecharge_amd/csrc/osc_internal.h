@@ -492,6 +492,16 @@ struct InterpArgs {
   int nlo[3], nhi[3], nn[3];
   double mn[3], delta[3], hi[3];
 };
+// What is known of the B field handed to a gather: nothing; Bz = 0 at every
+// node; or that and Bx = -bc Ey, By = bc Ex, each one product, of the E field
+// handed with it (the fields of space_charge_3d with and without cathode).
+enum BKind { B_ANY = 0, B_TRANSVERSE = 1, B_FROM_E = 2 };
+struct BForm {
+  int kind;
+  double bc;
+};
+// of the fields space_charge_3d leaves
+BForm sc3d_bform(double gamma, int at_cathode);
 int64_t interpolate(osc_ctx* c, const InterpArgs& a, const double* ef, const double* bf,
                     int64_t n, const double* x, const double* y, const double* z, double* E,
                     double* B, int8_t* clamped);
@@ -508,11 +518,12 @@ int noalloc_setup(int device, std::string* err);
 // same, for the particles of the preceding deposit in their cell-sorted order;
 // packed: the node records of (ef, bf) already queued by pack_nodes, or null
 // (sp.f32: the FP32 path, which reads the coordinates x, y, z of dropped
-// particles)
+// particles); bform: what the caller knows of bf
 void interpolate_sorted(osc_ctx* c, const InterpArgs& a, const double* ef, const double* bf,
                         const SortedParticles& sp, double* E, double* B, int8_t* clamped,
                         const double* packed = nullptr, const double* x = nullptr,
-                        const double* y = nullptr, const double* z = nullptr);
+                        const double* y = nullptr, const double* z = nullptr,
+                        BForm bform = BForm{B_ANY, 0.0});
 // queues the 64-byte node records (E, B) of the mesh into rec (8 doubles per node)
 void pack_nodes(osc_ctx* c, const InterpArgs& a, const double* ef, const double* bf, double* rec);
 // stable sort of n points by the mesh cell their gather reads (the clamped

@@ -151,11 +151,7 @@ void sc3d_t(osc_ctx* c, const osc_mesh& m, const double* rho, const double* offs
   const int64_t nt = int64_t(n[0]) * n[1] * n[2];
   double off[3] = {offset ? offset[0] : 0.0, offset ? offset[1] : 0.0, offset ? offset[2] : 0.0};
   const double s1 = kFpeiSolver2 / double(L[0] * L[1] * L[2]);
-  double bc = 0.0;
-  if (calc_b) {
-    const double beta = sqrt(1 - 1 / (m.gamma * m.gamma));  // :457
-    bc = beta / kClightSp;
-  }
+  const double bc = calc_b ? sc3d_bform(m.gamma, at_cathode).bc : 0.0;
   Specs<T> sp(6);
   GreenRef G[3];
   sp.get3(c, offset_spec(L, m.delta, m.gamma, 1, off, 0), 0, G);
@@ -335,6 +331,10 @@ void solver2(osc_ctx* c, const int n[3], const double* rho, double gamma, const 
              double* ef, double* phi, const double* offset) {
   if (c->prec == OSC_PREC_FP32) solver2_t<float>(c, n, rho, gamma, delta, ef, phi, offset);
   else solver2_t<double>(c, n, rho, gamma, delta, ef, phi, offset);
+}
+BForm sc3d_bform(double gamma, int at_cathode) {
+  const double beta = sqrt(1 - 1 / (gamma * gamma));  // :457
+  return BForm{at_cathode ? B_TRANSVERSE : B_FROM_E, beta / kClightSp};
 }
 void space_charge_3d(osc_ctx* c, const osc_mesh& m, const double* rho, const double* offset,
                      int at_cathode, int calc_b, double* ef, double* bf) {

@@ -77,3 +77,26 @@ def test_step_off_mesh(n, prec):
                 w = 16 * 2.0 ** -24 * np.max(np.abs(f[..., c]))
                 far = 1 + np.abs(np.stack([x / m.delta[0], y / m.delta[1], z / m.delta[2]])).max(0) ** 3
                 assert np.all(np.abs(g[:, c] - ref[:, c]) <= w * far)
+
+
+@pytest.mark.parametrize("shape", [(24, 20, 33), (96, 96, 128)])
+@pytest.mark.parametrize("n", [4001, 600011])
+@pytest.mark.parametrize("cathode", [False, True])
+def test_step_known_b(n, shape, cathode):
+    """The fused step's gather, which knows how its B was formed (no z part;
+    from E without a cathode), against interpolate_field of the same fields,
+    which does not: bit for bit, with particles off the mesh and one that has
+    no place."""
+    x, y, z = gaussian_bunch(n, (1e-3, 1e-3, 2e-3), seed=n + 3)
+    z += 8e-3
+    x[n // 2] = np.nan
+    m = osc.Mesh3D(nhi=shape, gamma=3.0)
+    m.min, m.max = np.array([-2e-3, -2.5e-3, 1e-3]), np.array([2.2e-3, 2e-3, 14e-3])
+    m.delta = (m.max - m.min) / (np.array(shape) - 1)
+    ctx = osc.Context(0)
+    E, B = osc.space_charge_step(x, y, z, m, total_charge=1e-9, resize_mesh=False, at_cathode=cathode,
+                                 calc_bfield=True, ctx=ctx)
+    E2, B2 = osc.interpolate_field(x, y, z, m, E=True, B=True, ctx=ctx)
+    ctx.close()
+    assert np.isnan(B[n // 2]).all() and np.count_nonzero(B[:, 2]) == 1
+    assert np.array_equal(E, E2, equal_nan=True) and np.array_equal(B, B2, equal_nan=True)
