@@ -904,9 +904,9 @@ static bool cached_spectrum(osc_ctx* c, const std::string& key, GreenRef& ref) {
   if (it == c->gcache.map.end()) return false;
   GreenCache::Entry& e = *it->second;
   e.last = ++c->gcache.tick;
-  DevBuf& have = sizeof(T) == 4 ? e.f32 : e.f64;
-  if (!have.p) return false;
-  ref = GreenRef{have.p, e.zr, e.zmh, e.zms};
+  const GreenCache::Array& have = sizeof(T) == 4 ? e.f32 : e.f64;
+  if (!have.buf.p) return false;
+  ref = GreenRef{have.buf.p, have.zr, have.zmh, have.zms};
   return true;
 }
 // gives a built spectrum to the cache, or to keep where it is not admitted
@@ -925,10 +925,11 @@ static void store_spectrum(osc_ctx* c, const std::string& key, const GreenRef& r
     ep = e.get();
     gc.map[key] = std::move(e);
   }
-  ep->zr = ref.zr;
-  ep->zmh = ref.zmh;
-  ep->zms = ref.zms;
-  (sizeof(T) == 4 ? ep->f32 : ep->f64) = std::move(sp);
+  GreenCache::Array& a = sizeof(T) == 4 ? ep->f32 : ep->f64;
+  a.buf = std::move(sp);
+  a.zr = ref.zr;
+  a.zmh = ref.zmh;
+  a.zms = ref.zms;
   ep->bytes += bytes;
   ep->last = ++gc.tick;
   gc.bytes += bytes;

@@ -56,9 +56,14 @@ struct GreenRef {
 
 class GreenCache {
  public:
-  struct Entry {
-    DevBuf f64, f32;
+  // the spectrum of one specification, in each precision its array and the
+  // form that is stored in (GreenRef; FP32 builds mirror axes, FP64 ones do not)
+  struct Array {
+    DevBuf buf;
     int zr = 0, zmh = 0, zms = 0;
+  };
+  struct Entry {
+    Array f64, f32;
     size_t bytes = 0;
     uint64_t last = 0;
   };
