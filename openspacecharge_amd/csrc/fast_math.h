@@ -92,14 +92,19 @@ OSC_FM double fm_rcp(double x) {  // 1 / x to about 2^-20 or better
 #ifdef __HIP_DEVICE_COMPILE__
   return __builtin_amdgcn_rcp(x);
 #else
-  return double(1.0f / float(x));  // the CPU test's stand-in: as coarse a start
+  int k;  // the CPU test's stand-in: as coarse a start
+  const double m = frexp(x, &k);
+  return ldexp(double(1.0f / float(m)), -k);
 #endif
 }
 OSC_FM double fm_rsq(double x) {
 #ifdef __HIP_DEVICE_COMPILE__
   return __builtin_amdgcn_rsq(x);
 #else
-  return double(1.0f / sqrtf(float(x)));
+  int k;
+  double m = frexp(x, &k);
+  if (k & 1) m *= 2.0, --k;
+  return ldexp(double(1.0f / sqrtf(float(m))), -k / 2);
 #endif
 }
 OSC_FM double fm_frexp(double x, int& k) {
@@ -186,6 +191,34 @@ OSC_FM double fast_sqrt_near(double s, double r, double h) {
   return fm_fma(fm_fma(-r, r, s), h, r);
 }
 
+// As the functions above, CHECK takes the plain sequence within its range and
+// the library's outside: a solve recorded for replay, whose kernel is the
+// checked one, has the bits of its eager twin.  (fast_sqrt_near and the
+// library's root differ for about one in 2500 of the sums whose root is within
+// 2^-43 of an ulp of the middle of two doubles.)
+OSC_FM bool plain_range(double x, double most) { return fabs(x) > 1.0 / most && fabs(x) < most; }
+
+// The roots r[0..2] of a node's three sums x^2 + y^2 + z^2 in the order of
+// xlafun2(u, v, w), (v, w, u) and (w, u, v): they may differ by an ulp
+template <bool CHECK>
+OSC_FM void prim_roots(double uu, double vv, double ww, double r[3]) {
+  const double s0 = uu + vv + ww, s1 = vv + ww + uu, s2 = ww + uu + vv;
+  if (CHECK && !plain_range(s0, 1e140)) {
+    r[0] = sqrt(s0);
+    r[1] = sqrt(s1);
+    r[2] = sqrt(s2);
+    return;
+  }
+  double h;
+  r[0] = fm_sqrt(s0, h);
+  r[1] = fast_sqrt_near(s1, r[0], h);
+  r[2] = fast_sqrt_near(s2, r[0], h);
+}
+template <bool CHECK>
+OSC_FM double fast_div(double n, double d) {
+  return CHECK && !(plain_range(n, 1e200) && plain_range(d, 1e200)) ? n / d : fm_div(n, d);
+}
+
 // xlafun2 (open_spacecharge_mod.f90:721-726) with the root of its own
 // x^2 + y^2 + z^2:  x atan(yz/(r x)) - z log(r+y) + y log((r-z)/(r+z))/2
 // (the first term is even in x: |x| atan(yz / (r |x|)))
@@ -193,7 +226,7 @@ template <bool CHECK>
 OSC_FM double xlafun2_tab(double x, double y, double z, double r, const FastMathTab& tab) {
   const double p = y * z;
   const double at = copysign(fast_atan_abs<CHECK>(p, r * x, tab), p);
-  const double ratio = CHECK ? (r - z) / (r + z) : fm_div(r - z, r + z);
+  const double ratio = fast_div<CHECK>(r - z, r + z);
   return fabs(x) * at - z * fast_log<CHECK>(r + y, tab) + y * fast_log<CHECK>(ratio, tab) * 0.5;
 }
 

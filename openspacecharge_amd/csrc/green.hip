@@ -129,8 +129,9 @@ struct Prim3 {
   double* F[3];
   double factor[3];
 };
-// CHECK: coordinates the host has not seen, or at which a root, a logarithm or
-// a quotient may leave the range of the plain instruction sequences (plain_grid)
+// CHECK: coordinates the host has not seen (a recorded solve), or at which a
+// root, a logarithm or a quotient may leave the range of the plain instruction
+// sequences (plain_grid); within it both kernels give the same bits
 template <bool CHECK>
 __global__ void __launch_bounds__(256)
     k_prim3(Prim3 o, int L0, int L1, int L2, double dx, double dy, double dz, double umin,
@@ -166,19 +167,11 @@ __global__ void __launch_bounds__(256)
   for (int k = int(blockIdx.z) * kPrimZ; k < k1; ++k) {
     const double w = double(k) * dz + wmin, ww = w * w;
     const int64_t at = i + int64_t(L0) * (j + int64_t(L1) * k);
-    // r of xlafun2(u, v, w), (v, w, u) and (w, u, v)
-    const double s0 = uu + vv + ww;
-    double h = 0.0;
-    const double r0 = CHECK ? sqrt(s0) : fm_sqrt(s0, h);
-    if (o.F[0]) o.F[0][at] = xlafun2_tab<CHECK>(u, v, w, r0, tab) * o.factor[0];
-    if (o.F[1]) {
-      const double s = vv + ww + uu, r = CHECK ? sqrt(s) : fast_sqrt_near(s, r0, h);
-      o.F[1][at] = xlafun2_tab<CHECK>(v, w, u, r, tab) * o.factor[1];
-    }
-    if (o.F[2]) {
-      const double s = ww + uu + vv, r = CHECK ? sqrt(s) : fast_sqrt_near(s, r0, h);
-      o.F[2][at] = xlafun2_tab<CHECK>(w, u, v, r, tab) * o.factor[2];
-    }
+    double r[3];
+    prim_roots<CHECK>(uu, vv, ww, r);
+    if (o.F[0]) o.F[0][at] = xlafun2_tab<CHECK>(u, v, w, r[0], tab) * o.factor[0];
+    if (o.F[1]) o.F[1][at] = xlafun2_tab<CHECK>(v, w, u, r[1], tab) * o.factor[1];
+    if (o.F[2]) o.F[2][at] = xlafun2_tab<CHECK>(w, u, v, r[2], tab) * o.factor[2];
   }
 }
 
