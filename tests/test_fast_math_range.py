@@ -1,7 +1,8 @@
 """The plain roots and quotients of csrc/fast_math.h over the whole range that
 the kernels without checks admit, and the checked sequences against the plain
 ones there: a solve recorded into a graph runs the checked kernel, its eager
-twin the plain one, and both must give the same bits.  (On the CPU: the same
+twin the plain one, and both must give the same bits.  The logarithm against
+80-bit values: as accurate as a library's.  (On the CPU: the same
 code, the reciprocal's start as coarse as the GPU's.)"""
 import os
 import subprocess
@@ -75,6 +76,18 @@ int main() {
     pair += a[0] != b[0] || a[1] != b[1] || a[2] != b[2];
     pair += fast_div<true>(a[0] - w, a[0] + w) != fast_div<false>(a[0] - w, a[0] + w);
   }
+  static FastMathTab tab;
+  fast_math_table(tab);
+  long double worst = 0, near1 = 0;
+  for (int n = 0; n < 4000000; ++n) {
+    double x = (0.5 + 0.5 * U(g)) * exp2(floor(n %% 2 ? 1400.0 * (U(g) - 0.5) : 24.0 * (U(g) - 0.5)));
+    if (n < 256 * 8) x = ldexp(0.5 + (n / 8) / 512.0 + ldexp(1.0, -53) * (n %% 2), n %% 8 - 4);  // the intervals' ends
+    const long double l = logl(x);
+    const double d = fabs(double(l));
+    if (d == 0.0) continue;
+    const long double e = fabsl(fast_log<true>(x, tab) - l) / (nextafter(d, INFINITY) - d);
+    (d >= 0.25 ? worst : near1) = fmaxl(d >= 0.25 ? worst : near1, e);
+  }
   // outside the range: the checked ones are the library's
   int bad = 0;
   const double inf = INFINITY, odd[] = {0.0, 5e-324, 1e-310, 1e-200, 1e200, 1e308, inf, double(NAN)};
@@ -87,7 +100,7 @@ int main() {
       bad += !(q == e || (q != q && e != e));
     }
   }
-  printf("%%ld %%ld %%ld %%ld %%ld %%d %%zu\n", root, quot, pair, plain, near, bad, hard.size());
+  printf("%%ld %%ld %%ld %%ld %%ld %%d %%zu %%.4Lf %%.4Lf\n", root, quot, pair, plain, near, bad, hard.size(), worst, near1);
 }
 '''
 
@@ -103,7 +116,7 @@ def counts(tmp_path_factory):
                     "-ffp-contract=off", "-D__HIP_PLATFORM_AMD__", f"-I{rocm}/include",
                     "-x", "c++", str(src), "-o", exe], check=True)
     out = subprocess.run([exe], check=True, capture_output=True, text=True).stdout.split()
-    return dict(zip(("root", "quot", "pair", "plain", "near", "bad", "hard"), map(int, out)))
+    return dict(zip(("root", "quot", "pair", "plain", "near", "bad", "hard", "log", "log1"), map(float, out)))
 
 
 def test_random_roots_and_quotients(counts):
@@ -119,3 +132,13 @@ def test_checked_sequences_are_the_plain_ones(counts):
 
 def test_checked_sequences_outside_the_range(counts):
     assert counts["bad"] == 0
+
+
+def test_logarithm(counts):
+    # k ln 2 + T is exact, so that the last sum rounds once (0.5); f, the first
+    # and the second sum of the small part (under 2^-7) round at 2^-61 each, and
+    # a last place is 2^-54 or more at |log x| >= 1/4
+    assert counts["log"] < 0.5 + 4 * 2.0 ** -7
+    # next to 1 the small part is up to two thirds of the result: its three
+    # roundings half a place each of a binade no higher
+    assert counts["log1"] < 1.25
