@@ -271,7 +271,8 @@ __device__ __forceinline__ void legacy_corner(double x, double y, double z, cons
 }
 template <bool CHECK, bool PHI>
 __global__ void __launch_bounds__(256)
-    k_green_legacy(Legacy3 o, GreenSpec s, int nk, const FastMathTab* __restrict__ table) {
+    k_green_legacy(Legacy3 o, GreenSpec s, int zbeg, int zend, int nk,
+                   const FastMathTab* __restrict__ table) {
   constexpr int NC = PHI ? 1 : 3;
   __shared__ FastMathTab tab;
   {
@@ -293,14 +294,14 @@ __global__ void __launch_bounds__(256)
     legacy_corner<CHECK, PHI>(x1, y2, z, tab, f[2]);
     legacy_corner<CHECK, PHI>(x2, y2, z, tab, f[3]);
   };
-  const int k0 = int(blockIdx.z) * nk, k1 = min(k0 + nk, s.L[2]);
+  const int k0 = zbeg + int(blockIdx.z) * nk, k1 = min(k0 + nk, zend);
   double zl = 0.0;
   for (int k = k0; k < k1; ++k) {
     const double w = legacy_w(s, k);
     const double z1 = (w - 0.5 * s.delta[2]) * s.gamma, z2 = (w + 0.5 * s.delta[2]) * s.gamma;
     if (k == k0 || z1 != zl) plane(z1, lo);
     plane(z2, up);
-    const int64_t at = i + int64_t(s.L[0]) * (j + int64_t(s.L[1]) * k);
+    const int64_t at = i + int64_t(s.L[0]) * (j + int64_t(s.L[1]) * (k - zbeg));
     const bool self = !PHI && x1 < 0.0 && x2 > 0.0 && y1 < 0.0 && y2 > 0.0 && z1 < 0.0 && z2 > 0.0;
 #pragma unroll
     for (int a = 0; a < NC; ++a) {
@@ -545,9 +546,11 @@ static bool plain_grid(const int n[3], At at) {
   return small <= 1;
 }
 
-// The integrated legacy Green functions of the components with G[ic - 1] set
-// (phi: the potential's into G[0]) of one legacy-kind specification s
-static void launch_legacy(osc_ctx* c, const GreenSpec& s, bool phi, double* const G[3]) {
+// The nz planes from zbeg on of the integrated legacy Green functions of the
+// components with G[ic - 1] set (phi: the potential's into G[0]) of one
+// legacy-kind specification s
+static void launch_legacy(osc_ctx* c, const GreenSpec& s, bool phi, double* const G[3], int zbeg,
+                          int nz) {
   Legacy3 o{};
   const double dx = s.delta[0], dy = s.delta[1], dz = s.delta[2];
   for (int a = 0; a < 3; ++a) {
@@ -565,11 +568,11 @@ static void launch_legacy(osc_ctx* c, const GreenSpec& s, bool phi, double* cons
   // planes per thread: eight where that still gives every CU four workgroups
   const unsigned gx = unsigned((s.L[0] + 63) / 64), gy = unsigned((s.L[1] + 3) / 4);
   int nk = 8;
-  while (nk > 1 && int64_t(gx) * gy * ((s.L[2] + nk - 1) / nk) < 1024) nk /= 2;
+  while (nk > 1 && int64_t(gx) * gy * ((nz + nk - 1) / nk) < 1024) nk /= 2;
   auto kern = phi ? (plain ? k_green_legacy<false, true> : k_green_legacy<true, true>)
                   : (plain ? k_green_legacy<false, false> : k_green_legacy<true, false>);
-  launch(kern, dim3(gx, gy, unsigned((s.L[2] + nk - 1) / nk)), dim3(64, 4), 0, c->stream, o, s, nk,
-         static_cast<const FastMathTab*>(c->fast_tab));
+  launch(kern, dim3(gx, gy, unsigned((nz + nk - 1) / nk)), dim3(64, 4), 0, c->stream, o, s, zbeg,
+         zbeg + nz, nk, static_cast<const FastMathTab*>(c->fast_tab));
   OSC_HIP(hipGetLastError());
 }
 
@@ -746,7 +749,7 @@ void build_green_real(osc_ctx* c, const GreenSpec& s, double* g, bool fast) {
   } else if (s.igf != 0) {
     double* G[3] = {nullptr, nullptr, nullptr};
     G[s.icomp >= 0 && s.icomp <= 2 ? std::max(0, s.icomp - 1) : 2] = g;
-    launch_legacy(c, s, s.icomp == 0, G);
+    launch_legacy(c, s, s.icomp == 0, G, 0, s.L[2]);
   } else {
     launch(k_green_coulomb, dim3(nblk(N)), dim3(kThreads), 0, c->stream, g, s);
     OSC_HIP(hipGetLastError());
@@ -756,7 +759,7 @@ void build_green_real(osc_ctx* c, const GreenSpec& s, double* g, bool fast) {
 // With corner differences and sym (per array and axis: 0, +1 even, -1 odd about
 // L/2 - 1, last plane zero), lines along y and z are computed only for the
 // lower half of a symmetric axis until that axis is transformed, whose pass
-// rebuilds the upper half as it loads (AxisIO::mh).
+// rebuilds the upper half as it loads (AxisIO::mh).  g null: the x pass is done.
 template <typename T>
 static void spectra_forward(osc_ctx* c, int n, const double* const g[], cpx<T>* const spec[],
                             const SpecDims& d, const CornerDiff* cd, const int (*sym)[3],
@@ -779,7 +782,7 @@ static void spectra_forward(osc_ctx* c, int n, const double* const g[], cpx<T>* 
     r.nrows = int64_t(Yh) * Zh;
     r.ny_rows = Yh;
     r.n_in = L0;
-    rb.in[q] = g[q];
+    rb.in[q] = g ? g[q] : nullptr;
     rb.out[q] = spec[q];
     if (cd) rb.cd[q] = cd[q];
     // spectrum q in elements from the first (of one allocation size: aligned alike)
@@ -798,7 +801,7 @@ static void spectra_forward(osc_ctx* c, int n, const double* const g[], cpx<T>* 
     a->mh = a->bmh[0];
     a->ms = a->bms[0];
   }
-  launch_xr2c<T>(L0, rb, cd != nullptr, twiddles<T>(c, L0), c->stream);
+  if (g) launch_xr2c<T>(L0, rb, cd != nullptr, twiddles<T>(c, L0), c->stream);
   ay.s_b = ay.d_b = 1;
   ay.s_p = ay.d_p = d.KXP;
   ay.s_o1 = ay.d_o1 = int64_t(d.KXP) * L1;
@@ -940,39 +943,88 @@ static void store_spectrum(osc_ctx* c, const std::string& key, const GreenRef& r
 // (with one primitive launch as well) 173 instead of 200.  On a large one the y
 // pass then finds its input in memory, where each component's own x pass had
 // left it in the 256 MB cache: 128^3 1999 us instead of 1975, 128x128x256 at the
-// cathode 4607 instead of 4513.
-constexpr int64_t kBatchGrid = int64_t(1) << 22;
+// cathode 4607 instead of 4513 (kBatchGrid, osc_internal.h).
+
+// The real legacy Green functions of n components and their x passes, as many
+// planes of each at a time as one component's array has room for (at least
+// two).  An even number: the rows that share a transform stay the same.
+static int legacy_turn(const GreenSpec& s, int n) { return std::max(2, s.L[2] / n / 2 * 2); }
+template <typename T>
+static void legacy_x_passes(osc_ctx* c, const GreenSpec& s, int n, const int icomp[], double* real,
+                            cpx<T>* const spec[], const SpecDims& d) {
+  const int turn = legacy_turn(s, n);
+  const int64_t plane = int64_t(s.L[0]) * s.L[1];
+  for (int z = 0; z < s.L[2]; z += turn) {
+    const int nz = std::min(turn, s.L[2] - z);
+    double* G[3] = {nullptr, nullptr, nullptr};
+    R2CBatch<T> rb{};
+    rb.n = n;
+    for (int q = 0; q < n; ++q) {
+      G[icomp[q] - 1] = real + q * turn * plane;
+      R2CIO& r = rb.a[q];
+      r.in_sy = s.L[0];
+      r.in_sz = plane;
+      r.out_sy = d.KXP;
+      r.out_sz = int64_t(d.KXP) * s.L[1];
+      r.nrows = int64_t(s.L[1]) * nz;
+      r.ny_rows = s.L[1];
+      r.n_in = s.L[0];
+      rb.in[q] = G[icomp[q] - 1];
+      rb.out[q] = spec[q] + z * r.out_sz;
+    }
+    {
+      ProfScope ps(c, ST_GREEN_EVAL);
+      launch_legacy(c, s, false, G, z, nz);
+    }
+    ProfScope ps(c, ST_GREEN_FFT);
+    launch_xr2c<T>(s.L[0], rb, false, twiddles<T>(c, s.L[0]), c->stream);
+  }
+}
 
 // The spectra of n components icomp[] of s that are in no cache: one kernel for
 // their real arrays where the kind has one; transforms together (kBatchGrid).
+// Above kBatchGrid the components' real arrays take no more memory than one's
+// beside the spectra, which a mesh that fills the device needs: in FP64 a
+// spectrum's place holds the next component's real array until that has been
+// transformed; in FP32, where it is half as large, the legacy components go by
+// planes (legacy_x_passes; the offset kind's are built one at a time).
 template <typename T>
 static void build_spectra(osc_ctx* c, const GreenSpec& s, int n, const int icomp[], DevBuf sp[],
                           GreenRef* const ref[]) {
   const SpecDims d = SpecDims::of(s.L);
   const int64_t N = int64_t(s.L[0]) * s.L[1] * s.L[2];
-  DevBuf real(c->pool, sizeof(double) * N * n);
+  const bool shared = s.kind != GK_OFFSET && s.kind != GK_PIPE && s.igf != 0 && icomp[0] >= 1;
+  const bool large = N > kBatchGrid && n > 1, planes = large && shared && sizeof(T) == 4;
+  const int64_t room = planes ? int64_t(n) * legacy_turn(s, n) * s.L[0] * s.L[1] : (large ? N : N * n);
+  OSC_REQUIRE(!large || planes || sizeof(T) == 8, OSC_ERR_ARG, "large FP32 builds are one at a time");
+  // (before the spectra: they would take the larger buffer that the last one left)
+  DevBuf real(c->pool, sizeof(double) * room);
   double* g[3];
   cpx<T>* spec[3];
   for (int q = 0; q < n; ++q) {
-    g[q] = real.as<double>() + q * N;
     sp[q] = DevBuf(c->pool, sizeof(cpx<T>) * d.size());
     spec[q] = sp[q].as<cpx<T>>();
     ref[q]->g = spec[q];
   }
+  for (int q = 0; q < n; ++q)
+    g[q] = large && q + 1 < n ? reinterpret_cast<double*>(spec[q + 1])
+                              : real.as<double>() + (large ? 0 : q * N);
   GreenRef* const* zr = fft_has_plan(s.L[2]) ? ref : nullptr;
   const bool fast = sizeof(T) == 4;  // mirrored quarter-grid primitive (prim_mirrors)
   auto forward = [&](const CornerDiff* cd, const int (*sym)[3]) {
     const int step = N <= kBatchGrid ? n : 1;
     for (int q = 0; q < n; q += step)
-      spectra_forward<T>(c, step, g + q, spec + q, d, cd ? cd + q : nullptr, sym ? sym + q : nullptr,
-                         zr ? zr + q : nullptr);
+      spectra_forward<T>(c, step, planes ? nullptr : g + q, spec + q, d, cd ? cd + q : nullptr,
+                         sym ? sym + q : nullptr, zr ? zr + q : nullptr);
   };
   if (s.kind != GK_OFFSET) {
-    if (s.igf != 0 && icomp[0] >= 1 && s.kind != GK_PIPE) {
+    if (planes) {
+      legacy_x_passes<T>(c, s, n, icomp, real.as<double>(), spec, d);
+    } else if (shared) {
       double* G[3] = {nullptr, nullptr, nullptr};
       for (int q = 0; q < n; ++q) G[icomp[q] - 1] = g[q];
       ProfScope ps(c, ST_GREEN_EVAL);
-      launch_legacy(c, s, false, G);
+      launch_legacy(c, s, false, G, 0, s.L[2]);
     } else {
       for (int q = 0; q < n; ++q) {
         GreenSpec t = s;

@@ -415,6 +415,9 @@ class HostRing {
 bool is_pageable(const void* p);
 
 // ---- green.hip --------------------------------------------------------------
+// grids up to which the Green functions of a solve's components are built
+// together, their real arrays side by side (green_spectra)
+constexpr int64_t kBatchGrid = int64_t(1) << 22;
 // the device's copy of the FastMathTab of fast_math.h (a constant, written once
 // per device, when its first context is created); null: a HIP error
 const void* fast_table(int device);
