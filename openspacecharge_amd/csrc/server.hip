@@ -77,12 +77,13 @@ uint64_t route_key(const osc_request& r) {
 }
 
 // device bytes of one request: mesh arrays, doubled-grid half spectra (rho,
-// up to four Green terms, the inverse work buffer), the real Green builds of
-// three components, node records, and the particle sort
+// up to four Green terms, the inverse work buffer), the real Green build (of
+// three components up to kBatchGrid), node records, and the particle sort
 int64_t estimate_bytes(const osc_request& r) {
   const int64_t n = int64_t(r.nhi[0]) * r.nhi[1] * r.nhi[2];
   const int64_t half = (int64_t(r.nhi[0]) + 1) * 4 * int64_t(r.nhi[1]) * r.nhi[2] * 16;
-  return 64 * n + 10 * half + 3 * 64 * n + 64 * n + 96 * r.n + (int64_t(64) << 20);
+  const int64_t green = (8 * n <= osc::kBatchGrid ? 3 : 1) * 64 * n;
+  return 64 * n + 10 * half + green + 64 * n + 96 * r.n + (int64_t(64) << 20);
 }
 
 }  // namespace
