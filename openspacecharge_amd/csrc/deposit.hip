@@ -1387,11 +1387,27 @@ __global__ void __launch_bounds__(TA_T)
 // tile face (i a multiple of the tile width), a - 1, per axis.  Bound by the
 // latency of the chunk blocks' loads where a node has many of them (a corner
 // of eight central tiles): LPN lanes share a node, lane q of them taking the
-// chunks q, q + LPN, ... of each tile (integer sums: any order).  Eight lanes
-// on meshes of at most kNodesSplit nodes, where one lane per node leaves CUs
-// idle; above it the loads of one lane per node, contiguous over a wave, fill
-// the chip.
-constexpr uint32_t kNodesSplit = 1u << 19;
+// chunks q, q + LPN, ... of each tile (integer sums: any order).
+//
+// Lanes cost every node its index arithmetic LPN times and an exchange, and
+// save loads only where tiles have several chunks, which a mesh of few nodes
+// has (few tiles) and few chunks in all rule out: as many lanes as keep
+// LPN nodes under 2^20, and under 2^13 for each chunk.  FP64 Gaussian bunch of
+// 4 sigma, 1 / 2 / 4 / 8 lanes in us (FP32 the same less a fifth):
+//   nodes        2 10^6 particles           3 10^4 particles (29 chunks)
+//   32^3         50.9 33.2 25.1 22.5        14.3 11.9 11.6 11.6
+//   64x32x64     33.7 25.8 24.1 21.5        11.8 12.4 13.8 16.5
+//   64^3         28.8 27.1 23.1 27.2        13.0 13.5 16.4 24.3
+//   64x64x128    24.4 24.2 28.9 45.7        14.1 17.1 24.5 40.5
+//   96x96x128    27.8 28.4 39.9 69.2        17.2 24.0 36.4 64.1
+// (a bunch a quarter as wide: at 64x64x128 59.1 43.3 39.5 37.1; a flat one:
+// 15.3 18.8 27.0 44.9.)
+inline int node_lanes(int64_t nodes, int64_t chunks) {
+  const int64_t most = std::min(int64_t(1) << 20, chunks << 13);
+  int lanes = 8;
+  while (lanes > 1 && lanes * nodes > most) lanes /= 2;
+  return lanes;
+}
 template <bool F32, int LPN>
 __global__ void k_tile_nodes(const unsigned long long* __restrict__ part,
                              const TilePlan* __restrict__ tp, TileParams p,
@@ -1777,10 +1793,15 @@ static void deposit_tiled(osc_ctx* c, const DepositArgs& a, double* rho, SortedP
   }
   {
     ProfScope ps(c, ST_DEP_NODES);
-    const bool split = ntot <= int64_t(kNodesSplit);
-    auto* k = f32 ? (split ? k_tile_nodes<true, 8> : k_tile_nodes<true, 1>)
-                  : (split ? k_tile_nodes<false, 8> : k_tile_nodes<false, 1>);
-    hipLaunchKernelGGL(k, dim3(nblk(split ? 8 * ntot : ntot)), dim3(kThreads), 0, c->stream,
+    const int lanes = node_lanes(ntot, (n + chunk - 1) / chunk);
+    auto sums = [&](auto l) {
+      return f32 ? k_tile_nodes<true, decltype(l)::value> : k_tile_nodes<false, decltype(l)::value>;
+    };
+    auto* k = lanes == 8   ? sums(std::integral_constant<int, 8>{})
+              : lanes == 4 ? sums(std::integral_constant<int, 4>{})
+              : lanes == 2 ? sums(std::integral_constant<int, 2>{})
+                           : sums(std::integral_constant<int, 1>{});
+    hipLaunchKernelGGL(k, dim3(nblk(lanes * ntot)), dim3(kThreads), 0, c->stream,
                        part.as<const unsigned long long>(), pl, tp, rho);
     OSC_HIP(hipGetLastError());
   }
