@@ -23,12 +23,14 @@ void axis_tv(int dir, const cpx<T>* in, cpx<T>* out, const AxisIO& a, int g1, in
              const cpx<T>* tw, hipStream_t s) {
   constexpr int BX = AxisTiles<T, L>::bx(V), NT = BX * Geo<T, L>::TPL;
   dim3 g = grid3(cdiv(a.nb, BX), g1, g2);
-  if (mirrored(a))
-    launch((k_axis<T, L, -1, true, BX>), g, dim3(NT), 0, s, in, out, a, tw);
+  if (a.batch)
+    launch((k_axis<T, L, -1, AX_BATCH, BX>), g, dim3(NT), 0, s, in, out, a, tw);
+  else if (a.mh > 0)
+    launch((k_axis<T, L, -1, AX_MIRROR, BX>), g, dim3(NT), 0, s, in, out, a, tw);
   else if (dir < 0)
-    launch((k_axis<T, L, -1, false, BX>), g, dim3(NT), 0, s, in, out, a, tw);
+    launch((k_axis<T, L, -1, AX_LINES, BX>), g, dim3(NT), 0, s, in, out, a, tw);
   else
-    launch((k_axis<T, L, 1, false, BX>), g, dim3(NT), 0, s, in, out, a, tw);
+    launch((k_axis<T, L, 1, AX_LINES, BX>), g, dim3(NT), 0, s, in, out, a, tw);
 }
 // the tile width the tuner picked for this pass (fft_tune_*)
 template <int L>
@@ -97,13 +99,21 @@ void zinv_t(const cpx<T>* rho, cpx<T>* out, const ZinvIO<T>& a, int Ly, int nout
   if (a.zreal && a.zin > 0) {
     OSC_REQUIRE(zconv_fits_t<L>(a), OSC_ERR_ARG, "fused z convolution: offsets exceed 32 bits");
     const int nxb = int(cdiv(a.nb, ZGeo<T, L>::BX));
-    ZinvIO<T> b = a;
-    // phases that add into one output follow each other
-    const int launches = a.nphase == 2 && a.acc ? 2 : 1;
-    b.nphase = a.nphase / launches;
-    const dim3 g1 = grid3(int64_t(nxb) * Ly * b.nphase, 1, 1);
-    for (b.phase0 = 0; b.phase0 < launches; ++b.phase0)
-      launch((k_zconv<T, L>), g1, dim3(ZGeo<T, L>::NT), 0, s, rho, out, b, tw, nxb);
+    if constexpr (sizeof(T) == 8) {
+      if (a.nphase == 2) {
+        ZinvIO<T> b = a;
+        // phases that add into one output follow each other
+        const int launches = a.acc ? 2 : 1;
+        b.nphase = a.nphase / launches;
+        const dim3 g1 = grid3(int64_t(nxb) * Ly * b.nphase, 1, 1);
+        for (b.phase0 = 0; b.phase0 < launches; ++b.phase0)
+          launch((k_zconv<T, L, true>), g1, dim3(ZGeo<T, L>::NT), 0, s, rho, out, b, tw, nxb);
+        return;
+      }
+    }
+    OSC_REQUIRE(a.nphase <= 1, OSC_ERR_ARG, "fused z convolution: phases in FP64 only");
+    launch((k_zconv<T, L, false>), grid3(int64_t(nxb) * Ly, 1, 1), dim3(ZGeo<T, L>::NT), 0, s, rho,
+           out, a, tw, nxb);
   } else if (a.zreal) {
     const int nxb = int(cdiv(a.nb, ZGeo<T, L>::BX));
     const int64_t units = int64_t(nxb) * Ly;
@@ -117,10 +127,10 @@ void zinv_t(const cpx<T>* rho, cpx<T>* out, const ZinvIO<T>& a, int Ly, int nout
 template <>
 void launch_axis<T>(int L, int dir, const cpx<T>* in, cpx<T>* out, const AxisIO& a, int g1, int g2,
                     const cpx<T>* tw, hipStream_t s) {
-  OSC_REQUIRE(a.batch == 0 || (a.batch == g2 && g2 <= 3), OSC_ERR_ARG, "bad batch");
+  OSC_REQUIRE(a.batch == 0 || (a.batch == g2 && g2 <= 3 && dir < 0), OSC_ERR_ARG, "bad batch");
   for (int o = 0; o < (a.batch ? a.batch : 1); ++o) {
     const int mh = a.batch ? a.bmh[o] : a.mh;
-    OSC_REQUIRE(mh == 0 || (dir < 0 && 2 * mh == L), OSC_ERR_ARG,
+    OSC_REQUIRE(mh == 0 || (dir < 0 && 2 * mh == L && !(a.batch && sizeof(T) == 8)), OSC_ERR_ARG,
                 "half-stored input lines are for forward passes over even lengths");
   }
   switch (L) {

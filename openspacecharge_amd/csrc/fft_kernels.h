@@ -25,9 +25,10 @@ struct AxisIO {
   // ms * element L-2-p and element L-1 is zero
   int mh, ms;
   // batch > 0: the blocks o2 are arrays of their own, at[o2] elements from the
-  // first (input and output), with o1 < n1[o2] and their own mh and ms.  (Not
-  // by these arrays always: arguments at a place that depends on the workgroup
-  // cost it a round trip to memory before its first load, 1 to 2 % of a pass.)
+  // first (input and output), with o1 < n1[o2] and their own mh and ms.  (In
+  // kernels of their own: arguments at a place that depends on the workgroup, or
+  // the question whether they are, cost it a round trip to memory before its
+  // first load, 3 to 7 % of a pass: y pass of 96^3 in FP64 14.3 us against 13.6.)
   int batch;
   int n1[3], bmh[3], bms[3];
   int64_t at[3];
@@ -174,8 +175,10 @@ __device__ __forceinline__ cpx<T> ldc(const cpx<T>* p) {
 // ---------------------------------------------------------------------------
 // strided line FFT (y or z axis, or x with s_p = 1)
 // ---------------------------------------------------------------------------
-// MIR: input lines may be stored as halves (AxisIO::mh)
-template <typename T, int L, int DIR, bool MIR, int BX = Geo<T, L>::BX>
+// AX_MIRROR: input lines are stored as halves (AxisIO::mh); AX_BATCH: arrays of
+// their own (AxisIO::batch), in FP32 stored as halves or not, in FP64 whole
+enum AxisMode { AX_LINES = 0, AX_MIRROR = 1, AX_BATCH = 2 };
+template <typename T, int L, int DIR, int MODE, int BX = Geo<T, L>::BX>
 __global__ void __launch_bounds__((BX * Geo<T, L>::TPL))
     k_axis(const cpx<T>* __restrict__ in, cpx<T>* out, AxisIO a, const cpx<T>* __restrict__ tw) {
   using F = FftTile<T, L, DIR, BX, false>;
@@ -187,7 +190,7 @@ __global__ void __launch_bounds__((BX * Geo<T, L>::TPL))
   const int bx = int(lw % gx), by = int((lw / gx) % gy), bz = int(lw / (gx * gy));
   int64_t src = bz * a.s_o2, dst = bz * a.d_o2;
   int mh = a.mh, ms = a.ms;
-  if (a.batch) {
+  if constexpr (MODE == AX_BATCH) {
     if (by >= a.n1[bz]) return;
     src = dst = a.at[bz];
     mh = a.bmh[bz];
@@ -196,7 +199,7 @@ __global__ void __launch_bounds__((BX * Geo<T, L>::TPL))
   const int bg = bx * BX + f.b;
   const bool ok = bg < a.nb;
   const cpx<T>* ib = in + (ok ? bg * a.s_b + by * a.s_o1 + src : 0);
-  if constexpr (MIR)
+  if constexpr (MODE == AX_MIRROR || (MODE == AX_BATCH && sizeof(T) == 4))
     f.load([&](int, int p) { return ok ? axis_in(ib, a, mh, ms, L, p) : mk<T>(0, 0); });
   else
     f.load([&](int, int p) { return (ok && p < a.n_in) ? ib[p * a.s_p] : mk<T>(0, 0); });
@@ -695,7 +698,9 @@ __device__ __forceinline__ const cpx<T>& at_off(const char* base, uint32_t vo) {
 // next Green line during the inverse transform, needs about 150 VGPRs
 // (3 waves per SIMD instead of 4) and is 5-10 % slower.
 //
-template <typename T, int L>
+// TWO: with phases (FP64 image solves).  Asking every workgroup cost solves
+// without them 1 to 1.5 % of this kernel (96^3 in FP64 176 us against 173).
+template <typename T, int L, bool TWO>
 __global__ void __launch_bounds__((ZGeo<T, L>::NT))
     k_zconv(const cpx<T>* __restrict__ rho, cpx<T>* __restrict__ out, ZinvIO<T> a,
             const cpx<T>* __restrict__ tw, int nxb) {
@@ -708,7 +713,7 @@ __global__ void __launch_bounds__((ZGeo<T, L>::NT))
   __shared__ cpx<T> lds[FF::LDS];
   // the phases of a column are consecutive logical workgroups (one L2)
   const int lw = int(xcd_block(blockIdx.x, gridDim.x));
-  const int ph = a.phase0 + lw % a.nphase, unit = lw / a.nphase;
+  const int ph = TWO ? a.phase0 + lw % a.nphase : 0, unit = TWO ? lw / a.nphase : lw;
   const int xb = unit % nxb, ky = unit / nxb;
   FF fr;
   const int b = fr.b, t = fr.t;
