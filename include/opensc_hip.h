@@ -113,7 +113,7 @@ const char* osc_stage_name(int stage);
 /* 1 if this transform length is supported (prime factors <= 23 and fits LDS) */
 int osc_fft_length_supported(int n);
 /* 1 if this length has a compile-time radix plan (LDS-tiled multi-line passes);
- * other supported lengths use the runtime-radix engine, one line per workgroup */
+ * other supported lengths use the runtime-length engine (prime radices grouped at run time) */
 int osc_fft_length_planned(int n);
 /* Tile width (lines per workgroup) of the strided FFT passes, chosen per
  * (precision, length, pass kind, line count) by an online tuner: the first

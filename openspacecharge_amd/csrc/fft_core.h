@@ -359,7 +359,7 @@ struct GenericPlan {
   int L;
   int ns;  // stages; -1: a prime factor above 23
   RtStage s[11];
-  // launch geometry, set per pass (rt_geometry): lines per workgroup as a
+  // launch geometry, set per pass (rt_plan): lines per workgroup as a
   // power of two, threads, and whether the stages alternate between two
   // buffers (some stage has more butterflies than threads)
   int bs, nt, pp;

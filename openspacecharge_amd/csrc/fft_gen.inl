@@ -16,8 +16,8 @@ inline dim3 grid3(int64_t x, int64_t y, int64_t z) {
   return dim3((unsigned)x, (unsigned)y, (unsigned)z);
 }
 
-// the same for a length without a compile-time plan (the line blocks
-// XCD-grouped as in k_axis)
+// k_axis for a length without a compile-time plan (the line blocks XCD-grouped
+// alike)
 template <typename T, int DIR, bool BIG>
 __global__ void __launch_bounds__(kRtMaxThreads)
     k_axis_gen(const cpx<T>* __restrict__ in, cpx<T>* out, AxisIO a, const cpx<T>* __restrict__ tw,

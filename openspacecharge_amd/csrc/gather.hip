@@ -6,8 +6,6 @@ namespace osc {
 
 namespace {
 constexpr int kThreads = 256;
-// batches at least this large are sorted by cell before the gather
-
 
 struct IP {
   double mn[3], delta[3], hinv[3];

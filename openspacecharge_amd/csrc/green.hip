@@ -525,8 +525,8 @@ static void prim_mirrors(const GreenSpec& s, bool fast, int& mev, int& mod) {
 // from the limits of doubles, and from the axes, for the kernels without checks:
 // magnitudes in 1e+-60 (their products and squares in range) and at most one
 // axis with coordinates under 1e-5 of the largest radius, so that r + y and
-// r - z, about (x^2 + z^2) / (2 r) where they cancel, stay 1e-10 r or more, a
-// million roundings of r (or they are exact: x = z = 0 does not occur).
+// r - z, about (x^2 + z^2) / (2 r) where they cancel, stay 5e-11 r or more, half
+// a million roundings of r (or they are exact: x = z = 0 does not occur).
 template <typename At>
 static bool plain_grid(const int n[3], At at) {
   double near[3], far[3];
@@ -944,13 +944,22 @@ static void store_spectrum(osc_ctx* c, const std::string& key, const GreenRef& r
   }
 }
 
-// Grids up to which the components' transforms run as one pass per axis.  One
-// component's passes leave a small grid with fewer workgroups than CUs: with one
-// pass for the three a step on 32^3 takes 137 us instead of 147, on 48^3 in FP32
-// (with one primitive launch as well) 173 instead of 200.  On a large one the y
-// pass then finds its input in memory, where each component's own x pass had
-// left it in the 256 MB cache: 128^3 1999 us instead of 1975, 128x128x256 at the
-// cathode 4607 instead of 4513 (kBatchGrid, osc_internal.h).
+// Grids up to which the components' transforms run as one pass per axis
+// (kBatchGrid, osc_internal.h).  One component's passes leave a small grid with
+// fewer workgroups than CUs: with one pass for the three a step on 32^3 takes
+// 137 us instead of 147, on 48^3 in FP32 (with one primitive launch as well) 173
+// instead of 200.  On a large one the y pass then finds its input in memory,
+// where each component's own x pass had left it in the 256 MB cache: 128^3 1999
+// us instead of 1975, 128x128x256 at the cathode 4607 instead of 4513.  Between,
+// with 2 10^5 particles, apart / together in us (free, cathode):
+//   mesh          values       FP64                     FP32
+//   64x64x128     2^22         373/369    616/616       249/231   475/434
+//   96x96x64      1.1 2^22     437/427    754/737       260/232   511/453
+//   96^3          1.7 2^22     674/637    1185/1140     319/298   670/609
+//   96x96x128     2.3 2^22     771/743    1346/1293     359/345   797/735
+//   128x128x108   3.4 2^22     1004/1022  1833/1864     460/450   1127/1101
+// The line stays at 2^22, below the crossing: together also takes three real
+// arrays' memory (96 MB there), apart one.
 
 // The real legacy Green functions of n components and their x passes, as many
 // planes of each at a time as one component's array has room for (at least
