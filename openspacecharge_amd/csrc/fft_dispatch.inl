@@ -12,12 +12,20 @@ inline dim3 grid3(int64_t x, int64_t y, int64_t z) {
 }
 inline int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
+inline bool mirrored(const AxisIO& a) {
+  bool m = a.batch == 0 && a.mh > 0;
+  for (int o = 0; o < a.batch; ++o) m = m || a.bmh[o] > 0;
+  return m;
+}
+
 template <int L, int V>
 void axis_tv(int dir, const cpx<T>* in, cpx<T>* out, const AxisIO& a, int g1, int g2,
              const cpx<T>* tw, hipStream_t s) {
   constexpr int BX = AxisTiles<T, L>::bx(V), NT = BX * Geo<T, L>::TPL;
   dim3 g = grid3(cdiv(a.nb, BX), g1, g2);
-  if (a.mh > 0)
+  if (a.batch)
+    launch((k_axis<T, L, -1, AX_BATCH, BX>), g, dim3(NT), 0, s, in, out, a, tw);
+  else if (a.mh > 0)
     launch((k_axis<T, L, -1, AX_MIRROR, BX>), g, dim3(NT), 0, s, in, out, a, tw);
   else if (dir < 0)
     launch((k_axis<T, L, -1, AX_LINES, BX>), g, dim3(NT), 0, s, in, out, a, tw);
@@ -28,16 +36,7 @@ void axis_tv(int dir, const cpx<T>* in, cpx<T>* out, const AxisIO& a, int g1, in
 template <int L>
 void axis_t(int dir, const cpx<T>* in, cpx<T>* out, const AxisIO& a, int g1, int g2,
             const cpx<T>* tw, hipStream_t s) {
-  // small grids: the default width (the others gain nothing there, steps on 32^3
-  // and 48^3 129 and 167 us with either; every kernel costs 60 us of a process's
-  // first use)
-  if (a.batch) {
-    constexpr int BX = AxisTiles<T, L>::bx(1);
-    launch((k_axis<T, L, -1, AX_BATCH, BX>), grid3(cdiv(a.nb, BX), g1, g2), dim3(BX * Geo<T, L>::TPL),
-           0, s, in, out, a, tw);
-    return;
-  }
-  const int kind = dir > 0 ? 2 : (a.mh > 0 ? 1 : 0);
+  const int kind = dir > 0 ? 2 : (mirrored(a) ? 1 : 0);
   const int64_t lines = int64_t(a.nb) * g1 * g2;
   bool distinct[3];
   for (int v = 0; v < 3; ++v) distinct[v] = v == 1 || AxisTiles<T, L>::bx(v) != AxisTiles<T, L>::bx(1);
